@@ -1,16 +1,24 @@
 // Strided / batched / split-K GEMM on CDNA4 matrix cores (gfx950).
 //
-// FP64: v_mfma_f64_16x16x4f64.  Block tile 128x128, K tile 16, 256 threads
-// (2x2 waves, 64x64 per wave = 4x4 MFMA tiles).  Operands are staged
-// global -> registers -> LDS (k-major, padded so a wave's 16x4 fragment reads
-// hit all 64 banks once per half-wave); the next K tile's global loads are
-// issued before the MFMAs of the current tile so their latency is hidden.
+// FP64: v_mfma_f64_16x16x4f64.  Block tile 128x128, 64x64 or 32x32 (K step
+// 16, 32 or 64), 256 threads as 2x2 waves.  Operands are staged global ->
+// registers -> LDS (padded so a wave's 16x4 fragment reads hit all 64 banks
+// once per half-wave); the next K step's global loads are issued before the
+// MFMAs of the current one.  No load is bounds-checked but those of a last,
+// partial K step.  Large products are bound by the matrix cores (68 TFLOP/s of
+// the 77 they sustain alone; 8192^3 in order k-fast x row-fast), small ones by
+// the latency of a K step, so tile and K chunks are planned per shape.  Sum
+// of the 20 products of one vector function, before (one 128 tile, every load
+// checked where K is not a multiple of 16, chunks of 1024 or more) and with
+// this kernel: o=5 v=19 1124 -> 136 us, o=11 v=93 3357 -> 1521, o=13 v=117
+// 5829 -> 3980, o=21 v=170 27900 -> 24440, o=32 v=256 72540 -> 69790.
 //
 // All operands are described by element strides, so the same kernel serves
 // row-major, transposed, batched and two-level-K (k = ko*Kin + ki)
 // contractions.  Which dimension the loader walks fastest (for coalescing)
 // is a template parameter chosen from the strides on the host.
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -20,17 +28,9 @@
 namespace ccgpu {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 
 enum { KFAST = 0, RFAST = 1 };  // loader order: k fastest / row (m or n) fastest
-
-template <bool K2>
-__device__ __forceinline__ long koff(long k, long s_k, long s_ko, long Kin) {
-  if (K2) {
-    long ko = k / Kin;
-    return ko * s_ko + (k - ko * Kin) * s_k;
-  }
-  return k * s_k;
-}
 
 // Logical tile for a linear block id.  Workgroups are dispatched round-robin
 // over the 8 XCDs (block b runs on XCD b % 8), each with its own L2: give each
@@ -49,40 +49,157 @@ __device__ __forceinline__ void tile_of(long b, long tiles_m, long tiles_n, long
   tn = r / gsz;
 }
 
-// LDS staging: an operand loaded k-fastest is stored [row][k] (stride TK+1,
-// conflict-free for both the stores and the 16x4 fragment reads); one loaded
-// row-fastest is stored [k][row] (stride T+16).
+// K steps and LDS staging of a T x T block tile: TK = 2048 / T columns of
+// K per step, so that every thread stages eight elements per operand whatever
+// the tile.  An operand loaded k-fastest is stored [row][k] with row stride
+// TK + 2, one loaded row-fastest [k][row] with stride T + 16 (the 32 tile:
+// stride 32, odd k with row bit 4 flipped, so that two blocks fit a CU); the
+// 8-byte fragment reads of a half wave then fall on all 64 banks once.
+template <int T>
+struct Step {
+  static constexpr int TK = 2048 / T, LDK = TK + 2, LDR = T == 32 ? T : T + 16;
+};
 template <int MODE, int T>
 struct Stage;
 template <int T>
-struct Stage<KFAST, T> {
-  double s[T][17];
-  __device__ __forceinline__ double& at(int r, int k) { return s[r][k]; }
+struct __attribute__((aligned(16))) Stage<KFAST, T> {
+  double s[T * Step<T>::LDK];
+  __device__ __forceinline__ double& at(int r, int k) { return s[r * Step<T>::LDK + k]; }
 };
 template <int T>
-struct Stage<RFAST, T> {
-  double s[16][T + 16];
-  __device__ __forceinline__ double& at(int r, int k) { return s[k][r]; }
+struct __attribute__((aligned(16))) Stage<RFAST, T> {
+  double s[Step<T>::TK * Step<T>::LDR];
+  __device__ __forceinline__ double& at(int r, int k) {
+    return s[k * Step<T>::LDR + (T == 32 ? r ^ ((k & 1) << 4) : r)];
+  }
 };
 
-// Block tile T x T (T = 128 or 64), 2x2 waves of (T/2)x(T/2), each wave
-// (T/32)x(T/32) MFMA 16x16 tiles.
+// Element offset of k: two-level K by a multiply-high with the truncated
+// 2^32 / Kin, at most 2^32 - 1 (the quotient is at most one short for k < 2^32).
+struct KMap {
+  long s_k, s_ko;
+  unsigned Kin, magic;
+};
+template <bool K2>
+__device__ __forceinline__ long koff(const KMap& m, long k) {
+  if (!K2) return k * m.s_k;
+  unsigned q = __umulhi((unsigned)k, m.magic), r = (unsigned)k - q * m.Kin;
+  if (r >= m.Kin) {
+    r -= m.Kin;
+    ++q;
+  }
+  return (long)q * m.s_ko + (long)r * m.s_k;
+}
+
+// This thread's eight elements of one K step of an operand tile whose first
+// row is at base: k-fastest, column tid % TK of rows tid / TK + (256 / TK) i;
+// row-fastest, row tid % T of columns tid / T + (256 / T) i.  One pointer per
+// operand walks K (two-level K recomputes it per step) and the eight
+// elements are uniform steps from it.  An element past the matrix (EDGE;
+// rmax = last row of the tile inside it) re-reads a row inside it, whose
+// results are never stored; only the last, partial step (TAIL) compares k
+// with kend, re-reads a column inside and takes zeros.
+template <int MODE, bool K2, int T, bool EDGE>
+struct Cursor {
+  static constexpr int TK = Step<T>::TK, NR = MODE == KFAST ? 256 / TK : 256 / T;
+  const double* p;
+  long s_r;
+  KMap km;
+  int r0, c0, rmax;
+
+  __device__ __forceinline__ Cursor(const double* base, long sr, const KMap& m, int rm, long kbeg, int tid)
+      : s_r(sr), km(m), rmax(rm) {
+    r0 = MODE == KFAST ? tid / TK : tid % T;
+    c0 = MODE == KFAST ? tid % TK : tid / T;
+    if (EDGE) r0 = min(r0, rmax);
+    p = base + r0 * s_r;
+    if (!K2) p += (kbeg + c0) * km.s_k;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ void load(double (&v)[8], long k0, long kend) {
+    const long k = k0 + c0;
+    if (MODE == KFAST) {
+      const double* q = p;
+      if (K2)
+        q += koff<true>(km, TAIL ? min(k, kend - 1) : k);
+      else if (TAIL && k >= kend)
+        q -= (k - (kend - 1)) * km.s_k;
+      const long st = NR * s_r;
+      int r = r0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[i] = *q;
+        if (EDGE) {
+          r += NR;
+          q += r <= rmax ? st : 0;
+        } else {
+          q += st;
+        }
+      }
+      if (TAIL && k >= kend) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = 0.0;
+      }
+    } else if (K2) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const long ki = k + NR * i;
+        const double x = p[koff<true>(km, TAIL ? min(ki, kend - 1) : ki)];
+        v[i] = (TAIL && ki >= kend) ? 0.0 : x;
+      }
+    } else {
+      const double* q = p;
+      if (TAIL && k >= kend) q -= (k - (kend - 1)) * km.s_k;
+      const long st = NR * km.s_k;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const double x = *q;
+        v[i] = (TAIL && k + NR * i >= kend) ? 0.0 : x;
+        if (TAIL)
+          q += k + NR * (i + 1) < kend ? st : 0;
+        else
+          q += st;
+      }
+    }
+    if (!K2) p += TK * km.s_k;
+  }
+};
+
+template <int MODE, int T>
+__device__ __forceinline__ void stage8(Stage<MODE, T>& S, const double (&v)[8], int tid) {
+  constexpr int TK = Step<T>::TK;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (MODE == KFAST)
+      S.at(tid / TK + (256 / TK) * i, tid % TK) = v[i];
+    else
+      S.at(tid % T, tid / T + (256 / T) * i) = v[i];
+  }
+}
+
+// Block tile T x T (T = 128, 64 or 32), 2x2 waves of (T/2)x(T/2), each wave
+// (T/32)x(T/32) MFMA 16x16 tiles.  The next step's global loads are in
+// flight while the current step's MFMAs run.  The 128 tile, which is bound
+// by the matrix cores, has one LDS stage (two barriers a step); the smaller
+// tiles, bound by the latency of a step, two stages and one barrier.
 template <int AMODE, int BMODE, bool K2, int T>
-__global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, double* ws) {
-  constexpr int TM = T, TN = T, TK = 16;
-  constexpr int NL = T / 16;      // elements per thread per operand and K tile
-  constexpr int RS = 256 / T;     // row-fastest loader: K columns per pass
+__global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, unsigned magic, double* ws) {
+  constexpr int TM = T, TN = T, TK = Step<T>::TK;
   constexpr int IW = T / 32;      // MFMA tiles per wave and dimension
-  __shared__ Stage<AMODE, T> As;
-  __shared__ Stage<BMODE, T> Bs;
+  constexpr int NS = T == 128 ? 1 : 2;
+  // both operands [row][k]: a lane takes two consecutive k of a group of
+  // eight for two MFMAs in turn, in 16-byte reads
+  constexpr bool PAIR = AMODE == KFAST && BMODE == KFAST;
+  __shared__ Stage<AMODE, T> As[NS];
+  __shared__ Stage<BMODE, T> Bs[NS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const long tiles_m = (d.M + TM - 1) / TM, tiles_n = (d.N + TN - 1) / TN;
   long tm, tn;
   tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const long m0 = tm * TM, n0 = tn * TN;
-  const double* A = static_cast<const double*>(d.A);
-  const double* B = static_cast<const double*>(d.B);
+  const double* A = static_cast<const double*>(d.A) + m0 * d.a_m;
+  const double* B = static_cast<const double*>(d.B) + n0 * d.b_n;
   long kbeg = 0, kend = d.K;
   if (kchunk > 0) {
     kbeg = (long)blockIdx.z * kchunk;
@@ -91,113 +208,100 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, doubl
     A += (long)blockIdx.z * d.a_b;
     B += (long)blockIdx.z * d.b_b;
   }
+  const KMap ka{d.a_k, d.a_ko, (unsigned)d.Kin, magic}, kb{d.b_k, d.b_ko, (unsigned)d.Kin, magic};
+  const int ma = (int)min((long)TM - 1, d.M - 1 - m0), nb = (int)min((long)TN - 1, d.N - 1 - n0);
+  const long nfull = (kend - kbeg) / TK;
+  const int rem = (int)((kend - kbeg) - nfull * TK);
 
-  // Interior tiles (inside M x N, whole K steps) load without bounds checks:
-  // the checks would otherwise branch around every load of the K loop.
-  const bool inside = m0 + TM <= d.M && n0 + TN <= d.N && (kend - kbeg) % TK == 0;
-  auto run = [&](auto guarded) {
-    constexpr bool G = decltype(guarded)::value;
-    double ra[NL], rb[NL];
-    // k-fastest: thread owns column c = tid % 16 and rows tid/16 + 16 i;
-    // row-fastest: thread owns row tid % T and columns tid/T + RS i.
-    auto load = [&](long k0) {
-      if (AMODE == KFAST) {
-        const long k = k0 + (tid % TK);
-        const bool kok = k < kend;
-        const long ko = (!G || kok) ? koff<K2>(k, d.a_k, d.a_ko, d.Kin) : 0;
-        const long mb = m0 + tid / TK;
-  #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-          const long m = mb + 16 * i;
-          ra[i] = (!G || (kok && m < d.M)) ? A[m * d.a_m + ko] : 0.0;
-        }
-      } else {
-        const long m = m0 + (tid % TM);
-        const bool mok = m < d.M;
-        const double* Ar = A + (mok ? m : 0) * d.a_m;
-        const long kb = k0 + tid / TM;
-  #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-          const long k = kb + RS * i;
-          ra[i] = (!G || (mok && k < kend)) ? Ar[koff<K2>(k, d.a_k, d.a_ko, d.Kin)] : 0.0;
-        }
-      }
-      if (BMODE == KFAST) {
-        const long k = k0 + (tid % TK);
-        const bool kok = k < kend;
-        const long ko = (!G || kok) ? koff<K2>(k, d.b_k, d.b_ko, d.Kin) : 0;
-        const long nb = n0 + tid / TK;
-  #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-          const long n = nb + 16 * i;
-          rb[i] = (!G || (kok && n < d.N)) ? B[n * d.b_n + ko] : 0.0;
-        }
-      } else {
-        const long n = n0 + (tid % TN);
-        const bool nok = n < d.N;
-        const double* Br = B + (nok ? n : 0) * d.b_n;
-        const long kb = k0 + tid / TN;
-  #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-          const long k = kb + RS * i;
-          rb[i] = (!G || (nok && k < kend)) ? Br[koff<K2>(k, d.b_k, d.b_ko, d.Kin)] : 0.0;
-        }
-      }
-    };
-    auto store = [&]() {
-  #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int e = tid + i * 256;
-        int r, c;
-        if (AMODE == KFAST) { r = e / TK; c = e % TK; } else { r = e % TM; c = e / TM; }
-        As.at(r, c) = ra[i];
-      }
-  #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const int e = tid + i * 256;
-        int r, c;
-        if (BMODE == KFAST) { r = e / TK; c = e % TK; } else { r = e % TN; c = e / TN; }
-        Bs.at(r, c) = rb[i];
-      }
-    };
+  const int lr = lane & 15, lk = lane >> 4;
 
+  auto run = [&](auto edge) {
+    constexpr bool E = decltype(edge)::value;
     d4 acc[IW][IW];
-  #pragma unroll
+#pragma unroll
     for (int i = 0; i < IW; ++i)
-  #pragma unroll
+#pragma unroll
       for (int j = 0; j < IW; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-
-    const int lr = lane & 15, lk = lane >> 4;
-    load(kbeg);
-    for (long k0 = kbeg; k0 < kend; k0 += TK) {
-      __syncthreads();
-      store();
-      __syncthreads();
-      if (k0 + TK < kend) load(k0 + TK);
-  #pragma unroll
-      for (int kk = 0; kk < TK / 4; ++kk) {
+    double ra[8], rb[8];
+    Cursor<AMODE, K2, T, E> ca(A, d.a_m, ka, ma, kbeg, tid);
+    Cursor<BMODE, K2, T, E> cb(B, d.b_n, kb, nb, kbeg, tid);
+    auto load = [&](long k0, auto tail) {
+      constexpr bool TL = decltype(tail)::value;
+      ca.template load<TL>(ra, k0, kend);
+      cb.template load<TL>(rb, k0, kend);
+    };
+    auto mfma8 = [&](int st, int k) {  // k .. k + 7 of the staged step
+      d2 pa[IW], pb[IW];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
         double a[IW], b[IW];
-  #pragma unroll
-        for (int t = 0; t < IW; ++t) a[t] = As.at(wm * (T / 2) + t * 16 + lr, kk * 4 + lk);
-  #pragma unroll
-        for (int t = 0; t < IW; ++t) b[t] = Bs.at(wn * (T / 2) + t * 16 + lr, kk * 4 + lk);
-  #pragma unroll
+#pragma unroll
+        for (int t = 0; t < IW; ++t) {
+          const int ra0 = wm * (T / 2) + t * 16 + lr, rb0 = wn * (T / 2) + t * 16 + lr;
+          if constexpr (PAIR) {
+            if (h == 0) {
+              pa[t] = *reinterpret_cast<const d2*>(&As[st].at(ra0, k + 2 * lk));
+              pb[t] = *reinterpret_cast<const d2*>(&Bs[st].at(rb0, k + 2 * lk));
+            }
+            a[t] = pa[t][h];
+            b[t] = pb[t][h];
+          } else {
+            a[t] = As[st].at(ra0, k + 4 * h + lk);
+            b[t] = Bs[st].at(rb0, k + 4 * h + lk);
+          }
+        }
+#pragma unroll
         for (int i = 0; i < IW; ++i)
-  #pragma unroll
+#pragma unroll
           for (int j = 0; j < IW; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
       }
+    };
+    const long nstep = nfull + (rem ? 1 : 0);
+    if (nfull > 0)
+      load(kbeg, std::false_type{});
+    else if (rem > 0)
+      load(kbeg, std::true_type{});
+    if constexpr (NS == 2) {
+      if (nstep > 0) {
+        stage8(As[0], ra, tid);
+        stage8(Bs[0], rb, tid);
+      }
+      __syncthreads();
     }
+    for (long s = 0; s < nstep; ++s) {
+      const int st = NS == 2 ? (int)(s & 1) : 0;
+      if constexpr (NS == 1) {
+        __syncthreads();
+        stage8(As[0], ra, tid);
+        stage8(Bs[0], rb, tid);
+        __syncthreads();
+      }
+      if (s + 1 < nfull)
+        load(kbeg + (s + 1) * TK, std::false_type{});
+      else if (s + 1 < nstep)
+        load(kbeg + (s + 1) * TK, std::true_type{});
+#pragma unroll
+      for (int k = 0; k < TK; k += 8) mfma8(st, k);
+      if constexpr (NS == 2) {
+        if (s + 1 < nstep) {
+          stage8(As[st ^ 1], ra, tid);
+          stage8(Bs[st ^ 1], rb, tid);
+        }
+        __syncthreads();
+      }
+    }
+
 
     // D[i][j] of a 16x16 f64 MFMA tile: lane = j + 16*(i%4), element i/4.
     if (kchunk > 0) {
       // split-K partial: ws[z][m][n] (dense M x N)
       double* W = ws + (long)blockIdx.z * d.M * d.N;
-  #pragma unroll
+#pragma unroll
       for (int i = 0; i < IW; ++i)
-  #pragma unroll
+#pragma unroll
         for (int j = 0; j < IW; ++j)
-  #pragma unroll
+#pragma unroll
           for (int r = 0; r < 4; ++r) {
             const long m = m0 + wm * (T / 2) + i * 16 + r * 4 + lk;
             const long n = n0 + wn * (T / 2) + j * 16 + lr;
@@ -208,22 +312,22 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, doubl
     // per 16-row block: C read (beta != 0) before any of the block's stores,
     // so the loads overlap instead of each waiting behind a store
     double* C = static_cast<double*>(d.C) + (long)blockIdx.z * d.c_b;
-  #pragma unroll
+#pragma unroll
     for (int i = 0; i < IW; ++i) {
       double cv[IW][4] = {};
       if (d.beta != 0.0) {  // uniform; indices clamped into C: no per-element branch
-  #pragma unroll
+#pragma unroll
         for (int j = 0; j < IW; ++j)
-  #pragma unroll
+#pragma unroll
           for (int r = 0; r < 4; ++r) {
             const long m = min(m0 + wm * (T / 2) + i * 16 + r * 4 + lk, d.M - 1);
             const long n = min(n0 + wn * (T / 2) + j * 16 + lr, d.N - 1);
             cv[j][r] = C[m * d.c_m + n * d.c_n];
           }
       }
-  #pragma unroll
+#pragma unroll
       for (int j = 0; j < IW; ++j)
-  #pragma unroll
+#pragma unroll
         for (int r = 0; r < 4; ++r) {
           const long m = m0 + wm * (T / 2) + i * 16 + r * 4 + lk;
           const long n = n0 + wn * (T / 2) + j * 16 + lr;
@@ -235,50 +339,119 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, doubl
         }
     }
   };
-  if (inside)
+  if (ma == TM - 1 && nb == TN - 1)
     run(std::false_type{});
   else
     run(std::true_type{});
 }
 
-// C = alpha * sum_z ws[z] + beta * C  (fixed summation order: deterministic)
-__global__ void k_splitk_reduce_f64(GemmDesc d, int nz, const double* ws) {
+// C = alpha * sum_z ws[z] + beta * C (fixed summation order: deterministic).
+// G groups of 256 / G threads share the z of 256 / G elements: with many
+// chunks of a small C one thread per element would walk them one load
+// latency after another.
+template <int G>
+__global__ __launch_bounds__(256) void k_splitk_reduce_f64(GemmDesc d, int nz, const double* ws) {
+  constexpr int E = 256 / G;
+  __shared__ double part[G][E];
   const long mn = d.M * d.N;
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < mn; e += (long)gridDim.x * blockDim.x) {
+  const int x = threadIdx.x % E, g = threadIdx.x / E;
+  for (long e0 = (long)blockIdx.x * E; e0 < mn; e0 += (long)gridDim.x * E) {
+    const long e = e0 + x;
     double s = 0.0;
-    for (int z = 0; z < nz; ++z) s += ws[(long)z * mn + e];
-    const long m = e / d.N, n = e - m * d.N;
-    double* p = static_cast<double*>(d.C) + m * d.c_m + n * d.c_n;
-    double v = d.alpha * s;
-    if (d.beta != 0.0) v += d.beta * *p;
-    *p = v;
+    if (e < mn) {
+#pragma unroll 4
+      for (int z = g; z < nz; z += G) s += ws[(long)z * mn + e];
+    }
+    if constexpr (G > 1) {
+      __syncthreads();  // the previous element's sums are read
+      part[g][x] = s;
+      __syncthreads();
+    }
+    if (g == 0 && e < mn) {
+      if constexpr (G > 1) {
+        for (int q = 1; q < G; ++q) s += part[q][x];
+      }
+      const long m = e / d.N, n = e - m * d.N;
+      double* p = static_cast<double*>(d.C) + m * d.c_m + n * d.c_n;
+      double v = d.alpha * s;
+      if (d.beta != 0.0) v += d.beta * *p;
+      *p = v;
+    }
   }
 }
 
 namespace {
-const char* const kDgemmName[2][2][2][2] = {
-    {{{"k_dgemm<0,0,false,128>", "k_dgemm<0,0,false,64>"}, {"k_dgemm<0,0,true,128>", "k_dgemm<0,0,true,64>"}},
-     {{"k_dgemm<0,1,false,128>", "k_dgemm<0,1,false,64>"}, {"k_dgemm<0,1,true,128>", "k_dgemm<0,1,true,64>"}}},
-    {{{"k_dgemm<1,0,false,128>", "k_dgemm<1,0,false,64>"}, {"k_dgemm<1,0,true,128>", "k_dgemm<1,0,true,64>"}},
-     {{"k_dgemm<1,1,false,128>", "k_dgemm<1,1,false,64>"}, {"k_dgemm<1,1,true,128>", "k_dgemm<1,1,true,64>"}}}};
+const char* const kDgemmName[2][2][2][3] = {
+    {{{"k_dgemm<0,0,false,128>", "k_dgemm<0,0,false,64>", "k_dgemm<0,0,false,32>"},
+      {"k_dgemm<0,0,true,128>", "k_dgemm<0,0,true,64>", "k_dgemm<0,0,true,32>"}},
+     {{"k_dgemm<0,1,false,128>", "k_dgemm<0,1,false,64>", "k_dgemm<0,1,false,32>"},
+      {"k_dgemm<0,1,true,128>", "k_dgemm<0,1,true,64>", "k_dgemm<0,1,true,32>"}}},
+    {{{"k_dgemm<1,0,false,128>", "k_dgemm<1,0,false,64>", "k_dgemm<1,0,false,32>"},
+      {"k_dgemm<1,0,true,128>", "k_dgemm<1,0,true,64>", "k_dgemm<1,0,true,32>"}},
+     {{"k_dgemm<1,1,false,128>", "k_dgemm<1,1,false,64>", "k_dgemm<1,1,false,32>"},
+      {"k_dgemm<1,1,true,128>", "k_dgemm<1,1,true,64>", "k_dgemm<1,1,true,32>"}}}};
+
+bool two_level(const GemmDesc& d) { return d.Kin > 0 && d.Kin < d.K; }
 
 template <int AM, int BM, int T>
 void launch_f64(const GemmDesc& d, dim3 grid, long kchunk, double* ws, hipStream_t s) {
-  const bool k2 = d.Kin > 0 && d.Kin < d.K;
-  const int id =
-      prof_begin(kDgemmName[AM][BM][k2 ? 1 : 0][T == 64 ? 1 : 0], 2.0 * d.M * d.N * d.K * d.batch, s);
+  const bool k2 = two_level(d);
+  const unsigned magic =
+      k2 ? (unsigned)std::min<unsigned long long>(0xFFFFFFFFull, (1ull << 32) / (unsigned long long)d.Kin) : 0u;
+  const int id = prof_begin(kDgemmName[AM][BM][k2 ? 1 : 0][T == 128 ? 0 : (T == 64 ? 1 : 2)],
+                            2.0 * d.M * d.N * d.K * d.batch, s);
   if (k2)
-    CCGPU_LAUNCH((k_dgemm<AM, BM, true, T>), grid, dim3(256), 0, s, d, kchunk, ws);
+    CCGPU_LAUNCH((k_dgemm<AM, BM, true, T>), grid, dim3(256), 0, s, d, kchunk, magic, ws);
   else
-    CCGPU_LAUNCH((k_dgemm<AM, BM, false, T>), grid, dim3(256), 0, s, d, kchunk, ws);
+    CCGPU_LAUNCH((k_dgemm<AM, BM, false, T>), grid, dim3(256), 0, s, d, kchunk, magic, ws);
   prof_end(id, s);
 }
 
-// Launch configuration of one FP64 GEMM: block tile and split-K on/off.
+// Launch configuration of one FP64 GEMM: block tile and K chunks (1: no split).
 struct F64Cfg {
   int tile = 128;
-  bool splitk = true;
+  int nz = 1;
 };
+
+// Estimated time (microseconds) of block tile T with K in nz chunks.  Two
+// blocks of any tile are resident per CU (256 CUs): a K step takes kOne
+// cycles while one block has a CU to itself and kTwo when two share it, the
+// blocks beyond whole rounds of 512 take a shared round again; a split adds a
+// launch and the pass over the partials, and C bounds the time from below.
+// The step times are measured (o = 5..32, v = 19..256 products of a vector
+// function): the 128 tile runs at 68 TFLOP/s in full rounds, the 64 tile at
+// 52 and the 32 tile at 37, but 64 x 64 and 32 x 32 tiles fill the chip, or
+// leave it sooner, where 128 x 128 ones are few or mostly padding.
+double cost_f64(const GemmDesc& d, int T, long nz) {
+  const int q = T == 128 ? 0 : (T == 64 ? 1 : 2);
+  constexpr double kOne[3] = {5900.0, 4200.0, 2700.0}, kTwo[3] = {9300.0, 5800.0, 3900.0}, kMhz = 2300.0;
+  const double tiles = (double)cdiv(d.M, T) * cdiv(d.N, T) * d.batch;
+  const double blocks = tiles * nz, steps = (double)cdiv(cdiv(d.K, nz), 2048 / T);
+  const long full = (long)(blocks / 512.0);
+  const double left = blocks - 512.0 * full;
+  const double last = left <= 0.0 ? 0.0 : (full == 0 && left <= 256.0 ? kOne[q] : kTwo[q]);
+  const double us = 3.5 + steps / kMhz * (full * kTwo[q] + last) * (two_level(d) ? 1.15 : 1.0);
+  const double cbytes = 8.0 * d.batch * (double)d.M * d.N * (d.beta != 0.0 ? 2.0 : 1.0);
+  return std::max(us, cbytes / 4.0e6) + (nz > 1 ? 2.5 + 0.02 * nz + (double)nz * d.M * d.N * 16.0 / 3.0e6 : 0.0);
+}
+
+// The configuration of least estimated time.
+F64Cfg plan_f64(const GemmDesc& d) {
+  F64Cfg best;
+  double bt = 1e300;
+  for (int T : {128, 64, 32}) {
+    // chunks of at least two K steps
+    const long kmax = d.batch == 1 ? std::max<long>(1, d.K / (2 * (2048 / T))) : 1;
+    for (long nz = 1; nz <= std::min<long>(kmax, 256); nz = nz < 4 ? nz + 1 : nz + nz / 3) {
+      const double t = cost_f64(d, T, nz);
+      if (t < bt) {
+        bt = t;
+        best = F64Cfg{T, (int)nz};
+      }
+    }
+  }
+  return best;
+}
 
 // ---- autotuner: per GEMM shape class, the fastest configuration measured
 struct ShapeKey {
@@ -338,49 +511,27 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
   long kchunk = 0;
   int nz = d.batch;
   double* ws = nullptr;
-  // Resident blocks when the chip is full: 2 per CU for 128-tiles, 4 for 64.
-  const long slots = T == 128 ? 512 : 1024;
-  if (cfg.splitk && d.batch == 1 && d.K >= 2048) {
-    // Split K over blockIdx.z so the launch fills whole waves of resident
-    // blocks: under one wave, enough chunks for two waves; otherwise the
-    // factor (<= 8, K chunks >= 1024) with the best fraction
-    // tiles*nz / (slots * waves) of occupied slots, the smallest on ties.
-    long want = 1;
-    if (tiles < slots) {
-      // under one wave: aim at two waves of blocks
-      want = std::min<long>((2 * slots + tiles - 1) / tiles, d.K / 1024);
-    } else {
-      double best = (double)tiles / (double)(((tiles + slots - 1) / slots) * slots);
-      for (long f = 2; f <= 8 && d.K / f >= 1024; ++f) {
-        const long tf = tiles * f;
-        const double e = (double)tf / (double)(((tf + slots - 1) / slots) * slots);
-        if (e > best + 0.02) {
-          best = e;
-          want = f;
-        }
-      }
-    }
-    if (want >= 2) {
-      long chunk = (d.K + want - 1) / want;
-      chunk = (chunk + 15) / 16 * 16;  // K tiles never straddle two chunks
-      nz = static_cast<int>((d.K + chunk - 1) / chunk);
-      if (nz >= 2) {
-        kchunk = chunk;
-        ws = grow_scratch(scratch_for(s).splitk, static_cast<size_t>(nz) * d.M * d.N, s);
-      } else {
-        nz = 1;
-      }
+  if (cfg.nz > 1 && d.batch == 1) {
+    const long tk = 2048 / T;  // chunks are whole K steps
+    const long chunk = cdiv(cdiv(d.K, cfg.nz), tk) * tk;
+    nz = (int)cdiv(d.K, chunk);
+    if (nz >= 2) {
+      kchunk = chunk;
+      ws = grow_scratch(scratch_for(s).splitk, static_cast<size_t>(nz) * d.M * d.N, s);
     }
   }
   CCGPU_REQUIRE(nz <= 65535, "gemm: too many batches");
   CCGPU_REQUIRE(tiles < (1L << 24), "gemm: too many tiles");
+  CCGPU_REQUIRE(!two_level(d) || d.K < (1L << 32), "gemm: two-level K too long");
   dim3 grid((unsigned)tiles, 1, nz);
 #define CCGPU_F64_LAUNCH(TT)                                                   \
   if (am == KFAST && bm == KFAST) launch_f64<KFAST, KFAST, TT>(d, grid, kchunk, ws, s); \
   else if (am == KFAST) launch_f64<KFAST, RFAST, TT>(d, grid, kchunk, ws, s);          \
   else if (bm == KFAST) launch_f64<RFAST, KFAST, TT>(d, grid, kchunk, ws, s);          \
   else launch_f64<RFAST, RFAST, TT>(d, grid, kchunk, ws, s);
-  if (T == 64) {
+  if (T == 32) {
+    CCGPU_F64_LAUNCH(32)
+  } else if (T == 64) {
     CCGPU_F64_LAUNCH(64)
   } else {
     CCGPU_F64_LAUNCH(128)
@@ -390,7 +541,11 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
   if (kchunk > 0) {
     const long mn = d.M * d.N;
     unsigned nb = static_cast<unsigned>(std::min<long>((mn + 255) / 256, 4096));
-    CCGPU_LAUNCH(k_splitk_reduce_f64, dim3(nb), dim3(256), 0, s, d, nz, ws);
+    if (nz > 4)
+      CCGPU_LAUNCH(k_splitk_reduce_f64<8>, dim3((unsigned)std::min<long>((mn + 31) / 32, 8192)), dim3(256), 0, s, d, nz,
+                   ws);
+    else
+      CCGPU_LAUNCH(k_splitk_reduce_f64<1>, dim3(nb), dim3(256), 0, s, d, nz, ws);
     CCGPU_HIPX(hipGetLastError());
   }
 }
@@ -398,15 +553,13 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
 // Times every candidate configuration of this shape (the GEMM runs for real,
 // so tuning passes produce throwaway results) and returns the fastest.
 F64Cfg tune_f64(const GemmDesc& d, int am, int bm, hipStream_t s) {
-  const F64Cfg cands[4] = {{128, true}, {128, false}, {64, true}, {64, false}};
-  const bool can_split = d.batch == 1 && d.K >= 2048;
+  const F64Cfg p = plan_f64(d), cands[4] = {p, {128, 1}, {64, 1}, {32, 1}};
   hipEvent_t e0, e1;
   CCGPU_HIP(hipEventCreate(&e0));
   CCGPU_HIP(hipEventCreate(&e1));
   F64Cfg best;
   float best_ms = 1e30f;
   for (const F64Cfg& c : cands) {
-    if (!c.splitk && !can_split) continue;  // identical to the split variant
     run_f64(d, c, am, bm, s);                // warm-up (also sizes scratch)
     CCGPU_HIP(hipEventRecord(e0, s));
     for (int r = 0; r < 2; ++r) run_f64(d, c, am, bm, s);
@@ -425,12 +578,36 @@ F64Cfg tune_f64(const GemmDesc& d, int am, int bm, hipStream_t s) {
 }
 }  // namespace
 
+namespace {
+// plan_f64 through a small direct-mapped table per thread (the plan depends
+// on the key and beta alone, and takes about as long as a launch).
+F64Cfg planned(const GemmDesc& d, const ShapeKey& key) {
+  struct Entry {
+    ShapeKey key{};
+    bool acc = false, set = false;
+    F64Cfg cfg;
+  };
+  static thread_local Entry table[256];
+  const bool acc = d.beta != 0.0;
+  unsigned long h = 1469598103934665603ul;
+  for (long x : {key.M, key.N, key.K, key.Kin, (long)key.batch, acc ? 1L : 0L}) h = (h ^ (unsigned long)x) * 1099511628211ul;
+  Entry& e = table[(h ^ (h >> 32)) & 255];
+  if (!e.set || e.acc != acc || e.key < key || key < e.key) {
+    e.key = key;
+    e.acc = acc;
+    e.cfg = plan_f64(d);
+    e.set = true;
+  }
+  return e.cfg;
+}
+}  // namespace
+
 void gemm_f64(const GemmDesc& d, hipStream_t s) {
   if (d.M <= 0 || d.N <= 0 || d.batch <= 0) return;
   check_gemm(d, sizeof(double));
   const int am = (d.a_m == 1 && d.a_k != 1) ? RFAST : KFAST;
   const int bm = (d.b_n == 1 && d.b_k != 1) ? RFAST : KFAST;
-  F64Cfg cfg;  // default: 128 x 128 tiles, split K when the launch is small
+  F64Cfg cfg;
   Tuner& tu = tuner();
   const ShapeKey key{d.M, d.N, d.K, (d.Kin > 0 && d.Kin < d.K) ? d.Kin : 0, d.batch, am, bm};
   bool found = false;
@@ -447,9 +624,11 @@ void gemm_f64(const GemmDesc& d, hipStream_t s) {
   const long tiles128 = (long)cdiv(d.M, 128) * cdiv(d.N, 128) * d.batch;
   if (!found && tu.on && tiles128 < 1024 && !dryrun() && !capturing(s)) {
     cfg = tune_f64(d, am, bm, s);
+    found = true;
     std::lock_guard<std::mutex> lk(tu.mu);
     tu.best[key] = cfg;
   }
+  if (!found) cfg = planned(d, key);
   run_f64(d, cfg, am, bm, s);
 }
 
