@@ -166,17 +166,20 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
   // of its stores, so their loads overlap instead of each waiting behind the
   // previous element's store.
   CCGPU_GLOBAL OutT* C = gptr(static_cast<OutT*>(p.C) + z * p.c_b);
+  // the descriptor's fields are read once (a store through C could alias them)
+  const long M = p.M, N = p.N, c_m = p.c_m, c_n = p.c_n;
+  const double alpha = p.alpha, beta = p.beta;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     OutT cv[4][4] = {};
-    if (p.beta != 0.0) {  // uniform; indices clamped into C, so the loads need no per-element branch
+    if (beta != 0.0) {  // uniform; indices clamped into C, so the loads need no per-element branch
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const long m = min(m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r, p.M - 1);
-          const long n = min(n0 + wn * 64 + j * 16 + lr, p.N - 1);
-          cv[j][r] = C[m * p.c_m + n * p.c_n];
+          const long m = min(m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r, M - 1);
+          const long n = min(n0 + wn * 64 + j * 16 + lr, N - 1);
+          cv[j][r] = C[m * c_m + n * c_n];
         }
     }
 #pragma unroll
@@ -185,10 +188,10 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
       for (int r = 0; r < 4; ++r) {
         const long m = m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r;
         const long n = n0 + wn * 64 + j * 16 + lr;
-        if (m < p.M && n < p.N) {
-          double v = p.alpha * (double)acc[i][j][r];
-          if (p.beta != 0.0) v += p.beta * (double)cv[j][r];
-          C[m * p.c_m + n * p.c_n] = static_cast<OutT>(v);
+        if (m < M && n < N) {
+          double v = alpha * (double)acc[i][j][r];
+          if (beta != 0.0) v += beta * (double)cv[j][r];
+          C[m * c_m + n * c_n] = static_cast<OutT>(v);
         }
       }
   }

@@ -158,15 +158,15 @@ class CCSD {
   void ladder_mixed(double* Om);
   void mark(const char* name);
   void ensure_work();
-  // (T) drivers: per-triple launches of the pre-packed three-pass W build and
-  // blocked energy (default); the same as one persistent kernel; the first
-  // per-triple driver (twelve GEMMs, per-triple packing, transposed W copies)
+  // (T) drivers: launches per group of triples of the pre-packed three-pass W
+  // build and blocked energy (default); the same as one persistent kernel
   enum class PtPath { Launch = 0, Persistent = 1 };
   void pt_prepare(GemmPrec mode, PtPath path);
   void pt_energy_persistent(long first, long n, long stride, double* e4, double* e5);
   void pt_energy_launches(long first, long n, long stride, double* e4, double* e5);
   void pt_descs(int i, int j, int k, int slot, unsigned char* out);
   size_t pt_desc_bytes() const;
+  long pt_group(bool mixed) const;
   void side_stream();
   void ensure_diis();
   void reset_cycle();
@@ -213,10 +213,11 @@ class CCSD {
   // (T), mixed path: (yd|zk) packed as bf16 hi/lo [k][(y,z)][d] in both (y,z)
   // orders, per-triple packed slices, FP32 W
   DBuf<unsigned short> GTh_, GTl_, GpTh_, GpTl_;
-  DBuf<float> W32_;  // four W slots (FP32)
+  DBuf<float> W32_;  // W slots (FP32)
   // (T), persistent kernel: bf16 hi/lo of every T(p,q) [x][d] and Q_rq [z][l]
   // slice and of -Tvvo_p in both (x,y) orders (mixed), Tvvo with (x,y)
-  // swapped (FP64); four W slots (in W32_ / Wt_); launch tables
+  // swapped (FP64); W slots (in W32_ / Wt_): four for the persistent kernel,
+  // pt_group() for the launches; launch tables
   PtPath pt_path_ = PtPath::Launch;
   DBuf<unsigned short> ppH_[4], ppL_[4];
   DBuf<double> TvvoS_;

@@ -24,13 +24,9 @@
 #include <type_traits>
 
 #include "common.h"
+#include "dgemm_tile.h"
 
 namespace ccgpu {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef double d2 __attribute__((ext_vector_type(2)));
-
-enum { KFAST = 0, RFAST = 1 };  // loader order: k fastest / row (m or n) fastest
 
 // Logical tile for a linear block id.  Workgroups are dispatched round-robin
 // over the 8 XCDs (block b runs on XCD b % 8), each with its own L2: give each
@@ -47,134 +43,6 @@ __device__ __forceinline__ void tile_of(long b, long tiles_m, long tiles_n, long
   const long r = lg - grp * GM * tiles_n;
   tm = fm + r % gsz;
   tn = r / gsz;
-}
-
-// K steps and LDS staging of a T x T block tile: TK = 2048 / T columns of
-// K per step, so that every thread stages eight elements per operand whatever
-// the tile.  An operand loaded k-fastest is stored [row][k] with row stride
-// TK + 2, one loaded row-fastest [k][row] with stride T + 16 (the 32 tile:
-// stride 32, odd k with row bit 4 flipped, so that two blocks fit a CU); the
-// 8-byte fragment reads of a half wave then fall on all 64 banks once.
-template <int T>
-struct Step {
-  static constexpr int TK = 2048 / T, LDK = TK + 2, LDR = T == 32 ? T : T + 16;
-};
-template <int MODE, int T>
-struct Stage;
-template <int T>
-struct __attribute__((aligned(16))) Stage<KFAST, T> {
-  double s[T * Step<T>::LDK];
-  __device__ __forceinline__ double& at(int r, int k) { return s[r * Step<T>::LDK + k]; }
-};
-template <int T>
-struct __attribute__((aligned(16))) Stage<RFAST, T> {
-  double s[Step<T>::TK * Step<T>::LDR];
-  __device__ __forceinline__ double& at(int r, int k) {
-    return s[k * Step<T>::LDR + (T == 32 ? r ^ ((k & 1) << 4) : r)];
-  }
-};
-
-// Element offset of k: two-level K by a multiply-high with the truncated
-// 2^32 / Kin, at most 2^32 - 1 (the quotient is at most one short for k < 2^32).
-struct KMap {
-  long s_k, s_ko;
-  unsigned Kin, magic;
-};
-template <bool K2>
-__device__ __forceinline__ long koff(const KMap& m, long k) {
-  if (!K2) return k * m.s_k;
-  unsigned q = __umulhi((unsigned)k, m.magic), r = (unsigned)k - q * m.Kin;
-  if (r >= m.Kin) {
-    r -= m.Kin;
-    ++q;
-  }
-  return (long)q * m.s_ko + (long)r * m.s_k;
-}
-
-// This thread's eight elements of one K step of an operand tile whose first
-// row is at base: k-fastest, column tid % TK of rows tid / TK + (256 / TK) i;
-// row-fastest, row tid % T of columns tid / T + (256 / T) i.  One pointer per
-// operand walks K (two-level K recomputes it per step) and the eight
-// elements are uniform steps from it.  An element past the matrix (EDGE;
-// rmax = last row of the tile inside it) re-reads a row inside it, whose
-// results are never stored; only the last, partial step (TAIL) compares k
-// with kend, re-reads a column inside and takes zeros.
-template <int MODE, bool K2, int T, bool EDGE>
-struct Cursor {
-  static constexpr int TK = Step<T>::TK, NR = MODE == KFAST ? 256 / TK : 256 / T;
-  const double* p;
-  long s_r;
-  KMap km;
-  int r0, c0, rmax;
-
-  __device__ __forceinline__ Cursor(const double* base, long sr, const KMap& m, int rm, long kbeg, int tid)
-      : s_r(sr), km(m), rmax(rm) {
-    r0 = MODE == KFAST ? tid / TK : tid % T;
-    c0 = MODE == KFAST ? tid % TK : tid / T;
-    if (EDGE) r0 = min(r0, rmax);
-    p = base + r0 * s_r;
-    if (!K2) p += (kbeg + c0) * km.s_k;
-  }
-  template <bool TAIL>
-  __device__ __forceinline__ void load(double (&v)[8], long k0, long kend) {
-    const long k = k0 + c0;
-    if (MODE == KFAST) {
-      const double* q = p;
-      if (K2)
-        q += koff<true>(km, TAIL ? min(k, kend - 1) : k);
-      else if (TAIL && k >= kend)
-        q -= (k - (kend - 1)) * km.s_k;
-      const long st = NR * s_r;
-      int r = r0;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        v[i] = *q;
-        if (EDGE) {
-          r += NR;
-          q += r <= rmax ? st : 0;
-        } else {
-          q += st;
-        }
-      }
-      if (TAIL && k >= kend) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = 0.0;
-      }
-    } else if (K2) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const long ki = k + NR * i;
-        const double x = p[koff<true>(km, TAIL ? min(ki, kend - 1) : ki)];
-        v[i] = (TAIL && ki >= kend) ? 0.0 : x;
-      }
-    } else {
-      const double* q = p;
-      if (TAIL && k >= kend) q -= (k - (kend - 1)) * km.s_k;
-      const long st = NR * km.s_k;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const double x = *q;
-        v[i] = (TAIL && k + NR * i >= kend) ? 0.0 : x;
-        if (TAIL)
-          q += k + NR * (i + 1) < kend ? st : 0;
-        else
-          q += st;
-      }
-    }
-    if (!K2) p += TK * km.s_k;
-  }
-};
-
-template <int MODE, int T>
-__device__ __forceinline__ void stage8(Stage<MODE, T>& S, const double (&v)[8], int tid) {
-  constexpr int TK = Step<T>::TK;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (MODE == KFAST)
-      S.at(tid / TK + (256 / TK) * i, tid % TK) = v[i];
-    else
-      S.at(tid % T, tid / T + (256 / T) * i) = v[i];
-  }
 }
 
 // Block tile T x T (T = 128, 64 or 32), 2x2 waves of (T/2)x(T/2), each wave

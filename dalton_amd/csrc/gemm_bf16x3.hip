@@ -210,17 +210,6 @@ struct NoTune {
   ~NoTune() { --t_no_tune; }
 };
 
-// Without a measurement: the 256x256 tile computes Mp x Np (padded to 256),
-// the 128x128 one ceil(M/128) x ceil(N/128) tiles, at 361 against 307
-// TFLOP/s measured on square products; the 256 tile also needs a wave of
-// tiles over the CUs to be worth its larger grain.
-int model_choice(const BMulti& p, int batch) {
-  const double a256 = (double)p.Mp * (double)p.Np;
-  const double a128 = (double)cdiv(p.M, TM) * TM * (double)cdiv(p.N, TN) * TN;
-  const long t256 = (p.Mp / DT) * (p.Np / DT) * (long)batch;
-  return (a256 * 307.0 <= a128 * 361.0 && t256 >= 256) ? kT256 : kT128;
-}
-
 // Times both tiles on the product itself: an overwriting product (beta = 0)
 // runs as given, since the real launch that follows rewrites the same
 // values; an accumulating one runs with alpha = 0 and beta = 1, which leaves
@@ -274,7 +263,7 @@ void launch_multi(BMulti p, int batch, hipStream_t s) {
         tu.best[key] = kern;
         ++tu.timed;
       } else {
-        kern = model_choice(p, batch);
+        kern = bf16x3_large_tile(p.M, p.N, batch) ? kT256 : kT128;
       }
     }
   }
@@ -287,6 +276,18 @@ long bf16x3_kpad(long K) { return std::max<long>(TK, (K + TK - 1) / TK * TK); }
 long bf16x3_rpad(long R) {
   const long t = variant() != 0 ? DT : TM;  // rows padded to the block tile in use
   return (R + t - 1) / t * t;
+}
+
+// Without a measurement: the 256x256 tile computes M x N padded to 256,
+// the 128x128 one ceil(M/128) x ceil(N/128) tiles, at 361 against 307
+// TFLOP/s measured on square products; the 256 tile also needs a wave of
+// tiles over the CUs to be worth its larger grain.
+bool bf16x3_large_tile(long M, long N, long batch) {
+  if (variant() != 1) return false;  // operands padded to 128 rows only
+  const double a256 = (double)bf16x3_rpad(M) * (double)bf16x3_rpad(N);
+  const double a128 = (double)cdiv(M, TM) * TM * (double)cdiv(N, TN) * TN;
+  const long t256 = (bf16x3_rpad(M) / DT) * (bf16x3_rpad(N) / DT) * batch;
+  return a256 * 307.0 <= a128 * 361.0 && t256 >= 256;
 }
 
 void bf16x3_pack(const double* src, long rows, long K, long s_r, long s_k, long s_b, int batch, long Rp, long Kp,

@@ -55,8 +55,7 @@ void CCSD::pt_release() {
 
 // Integral and amplitude layouts for the triple loop (built once per call
 // sequence; the iteration workspace is released first to make room): every
-// per-triple operand pre-packed, and four W slots (the persistent kernel's
-// pipeline; the per-triple launches use the first).
+// per-triple operand pre-packed, and the W slots.
 void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
   if (pt_ready_ && pt_mode_ == mode && pt_path_ == path) return;
   pt_release();
@@ -66,7 +65,10 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
   const bool mixed = mode == GemmPrec::BF16X3;
   Tvvo_.alloc((size_t)o * vv * o);
   Q_.alloc((size_t)o * o * o * v);
-  ptpart_.alloc(std::max<size_t>((size_t)(vv + v) + 2, 8 * 2048));
+  // W slots and energy partials (at most 2048 pairs a triple): the persistent
+  // kernel's four, or one per triple of a group of launches
+  const size_t slots = path == PtPath::Persistent ? 4 : (size_t)pt_group(mixed);
+  ptpart_.alloc(2 * 2048 * slots);
   {
     // undressed virtual-virtual and occupied-occupied blocks of B
     DBuf<double> Bvv0((size_t)naux * vv), Boo0((size_t)naux * o * o), R((size_t)nov * o * o);
@@ -75,7 +77,7 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
     if (!mixed) {
       G_.alloc((size_t)o * vvv);
       Gp_.alloc((size_t)o * vvv);
-      Wt_.alloc(4 * (size_t)vvv);
+      Wt_.alloc(slots * (size_t)vvv);
       TvvoS_.alloc((size_t)o * vv * o);
       // G[k][d][y][z] = (yd|zk) = sum_P B[P][d][y] B[P][k][z], batched over k
       g(vv, v, naux, 1.0, Bvv0.p, 1, vv, Bov_.p, nov, 1, 0.0, G_.p, v, 1, st_, o, 0, v, vvv);
@@ -90,7 +92,7 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
       GTl_.alloc(ng);
       GpTh_.alloc(ng);
       GpTl_.alloc(ng);
-      W32_.alloc(4 * (size_t)vvv);
+      W32_.alloc(slots * (size_t)vvv);
       DBuf<double> Gk(vvv), Gpk(vvv);
       for (int k = 0; k < o; ++k) {
         g(vv, v, naux, 1.0, Bvv0.p, 1, vv, Bov_.p + (long)k * v, nov, 1, 0.0, Gk.p, v, 1, st_);
@@ -168,8 +170,8 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
   pt_ready_ = true;
 }
 
-// (T) driver from CCGPU_PT_PATH: "launch" (default: per-triple launches of
-// the pass kernels) or "persistent" (one cooperative kernel per chunk of
+// (T) driver from CCGPU_PT_PATH: "launch" (default: launches of the pass
+// kernels per group of triples) or "persistent" (one cooperative kernel per chunk of
 // triples).
 static int pt_path_from_env() {
   const char* e = std::getenv("CCGPU_PT_PATH");

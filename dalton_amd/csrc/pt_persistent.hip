@@ -35,15 +35,13 @@
 
 #include "bf16x3_tile.h"
 #include "ccsd.h"
+#include "dgemm_tile.h"
 #include "kernels.h"
 #include "ops.h"
 
 namespace ccgpu {
 
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef double d2 __attribute__((ext_vector_type(2)));
 
 // ------------------------------------------------------------ FP64 tiles
 // One term of a multi-term FP64 product: A(m,k) of batch z at
@@ -70,104 +68,52 @@ struct DMulti {
 namespace dt {
 // Tile 128 x 128, K step 16, 256 threads as 2 x 2 waves of 64 x 64
 // (4 x 4 v_mfma_f64_16x16x4f64 tiles each); operands staged
-// global -> registers -> LDS, the next step's loads issued before the MFMAs.
-// Each step derives its eight load addresses from one pointer (an empty asm
-// keeps the compiler from hoisting eight 64-bit row offsets out of the K
-// loop, which would not fit beside the accumulators).
-// An operand read along k is staged [row][k] (row stride TK + 1), one read
-// along its rows [k][row] (stride T + 16): both conflict-free.
-constexpr int T = 128, TK = 16, NL = 8, IW = 4, LDR = T + 16;
+// global -> registers -> LDS as in the FP64 GEMM (one pointer per operand
+// walks K, rows past the matrix re-read a row inside it, only a last partial
+// K step compares k with K), the next step's loads issued before the MFMAs.
+constexpr int T = 128, TK = Step<T>::TK, IW = 4;
 struct __attribute__((aligned(16))) Smem {
-  double A[TK * LDR];
-  double B[TK * LDR];
+  double A[TK * Step<T>::LDR];
+  double B[TK * Step<T>::LDR];
 };
-template <bool KF>
-__device__ __forceinline__ double& at(double* s, int r, int k) {
-  return KF ? s[r * (TK + 1) + k] : s[k * LDR + r];
-}
+static_assert(sizeof(Stage<KFAST, T>) <= sizeof(double) * TK * Step<T>::LDR &&
+                  sizeof(Stage<RFAST, T>) <= sizeof(double) * TK * Step<T>::LDR,
+              "pt: operand stages");
 
-// G = false: the tile lies inside M x N and K is a multiple of 16, so the
-// loads need no bounds checks.
-template <bool AKF, bool G = true>
-__device__ __forceinline__ void term(const DTerm& t, long M, long N, long m0, long n0, long z, d4 (&acc)[IW][IW],
+// E: the tile reaches past M or N.
+template <bool AKF, bool E>
+__device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, long n0, long z, d4 (&acc)[IW][IW],
                                      Smem& S) {
-  constexpr bool BKF = !AKF;
+  constexpr int AM = AKF ? KFAST : RFAST, BM = AKF ? RFAST : KFAST;
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // thread-index arithmetic stays inside the item (not hoisted into the claim loop)
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const CCGPU_GLOBAL double* A = gptr(t.A + z * t.a_b);
-  const CCGPU_GLOBAL double* B = gptr(t.B + z * t.b_b);
-  const long K = t.K, a_m = t.a_m, a_k = t.a_k, b_n = t.b_n, b_k = t.b_k;
+  const long K = t.K;
   const double al = t.alpha;
-  double ra[NL], rb[NL];
+  using GP = const CCGPU_GLOBAL double*;
+  Cursor<AM, false, T, E, GP> ca(gptr(t.A + z * t.a_b + m0 * t.a_m), t.a_m, KMap{t.a_k, 0, 0u, 0u}, ma, 0, tid);
+  Cursor<BM, false, T, E, GP> cb(gptr(t.B + z * t.b_b + n0 * t.b_n), t.b_n, KMap{t.b_k, 0, 0u, 0u}, nb, 0, tid);
+  Stage<AM, T>& SA = *reinterpret_cast<Stage<AM, T>*>(S.A);
+  Stage<BM, T>& SB = *reinterpret_cast<Stage<BM, T>*>(S.B);
+  double ra[8], rb[8];
   auto load = [&](long k0) {
-    if (AKF) {  // column k0 + tid % 16, rows tid / 16 + 16 i
-      const long k = k0 + (tid & 15);
-      const bool kok = k < K;
-      const long mb = m0 + (tid >> 4);
-      const CCGPU_GLOBAL double* pa = A + (mb * a_m + k * a_k);
-      asm volatile("" : "+v"(pa));
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        ra[i] = (!G || (kok && mb + 16 * i < M)) ? al * *pa : 0.0;
-        pa += 16 * a_m;
-      }
-    } else {  // row tid % 128, columns tid / 128 + 2 i
-      const long m = m0 + (tid & (T - 1));
-      const bool mok = m < M;
-      const long kb = k0 + (tid >> 7);
-      const CCGPU_GLOBAL double* pa = A + ((mok ? m : 0) * a_m + kb * a_k);
-      asm volatile("" : "+v"(pa));
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        ra[i] = (!G || (mok && kb + 2 * i < K)) ? al * *pa : 0.0;
-        pa += 2 * a_k;
-      }
-    }
-    if (BKF) {
-      const long k = k0 + (tid & 15);
-      const bool kok = k < K;
-      const long nb = n0 + (tid >> 4);
-      const CCGPU_GLOBAL double* pb = B + (nb * b_n + k * b_k);
-      asm volatile("" : "+v"(pb));
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        rb[i] = (!G || (kok && nb + 16 * i < N)) ? *pb : 0.0;
-        pb += 16 * b_n;
-      }
+    if (k0 + TK <= K) {
+      ca.template load<false>(ra, k0, K);
+      cb.template load<false>(rb, k0, K);
     } else {
-      const long n = n0 + (tid & (T - 1));
-      const bool nok = n < N;
-      const long kb = k0 + (tid >> 7);
-      const CCGPU_GLOBAL double* pb = B + ((nok ? n : 0) * b_n + kb * b_k);
-      asm volatile("" : "+v"(pb));
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        rb[i] = (!G || (nok && kb + 2 * i < K)) ? *pb : 0.0;
-        pb += 2 * b_k;
-      }
-    }
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int e = tid + 256 * i;
-      if (AKF)
-        at<true>(S.A, e >> 4, e & 15) = ra[i];
-      else
-        at<false>(S.A, e & (T - 1), e >> 7) = ra[i];
-      if (BKF)
-        at<true>(S.B, e >> 4, e & 15) = rb[i];
-      else
-        at<false>(S.B, e & (T - 1), e >> 7) = rb[i];
+      ca.template load<true>(ra, k0, K);
+      cb.template load<true>(rb, k0, K);
     }
   };
   const int lr = lane & 15, lk = lane >> 4;
   load(0);
   for (long k0 = 0; k0 < K; k0 += TK) {
     __syncthreads();
-    store();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ra[i] *= al;
+    stage8<AM, T>(SA, ra, tid);
+    stage8<BM, T>(SB, rb, tid);
     __syncthreads();
     if (k0 + TK < K) load(k0 + TK);
 #pragma unroll
@@ -175,8 +121,8 @@ __device__ __forceinline__ void term(const DTerm& t, long M, long N, long m0, lo
       double a[IW], b[IW];
 #pragma unroll
       for (int u = 0; u < IW; ++u) {
-        a[u] = at<AKF>(S.A, wm * 64 + u * 16 + lr, kk * 4 + lk);
-        b[u] = at<BKF>(S.B, wn * 64 + u * 16 + lr, kk * 4 + lk);
+        a[u] = SA.at(wm * 64 + u * 16 + lr, kk * 4 + lk);
+        b[u] = SB.at(wn * 64 + u * 16 + lr, kk * 4 + lk);
       }
 #pragma unroll
       for (int i = 0; i < IW; ++i)
@@ -189,35 +135,39 @@ __device__ __forceinline__ void term(const DTerm& t, long M, long N, long m0, lo
 // Four terms, the first two read with A along k (X) or along m (!X), the
 // other two the other way; the sequence is static so the accumulators stay
 // in registers from term to term.
-template <bool X, bool G = true>
+template <bool X, bool E>
 __device__ __forceinline__ void tile4(const DMulti& p, long m0, long n0, long z, Smem& S) {
   d4 acc[IW][IW];
 #pragma unroll
   for (int i = 0; i < IW; ++i)
 #pragma unroll
     for (int j = 0; j < IW; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-  term<X, G>(p.t[0], p.M, p.N, m0, n0, z, acc, S);
-  term<X, G>(p.t[1], p.M, p.N, m0, n0, z, acc, S);
-  term<!X, G>(p.t[2], p.M, p.N, m0, n0, z, acc, S);
-  term<!X, G>(p.t[3], p.M, p.N, m0, n0, z, acc, S);
+  const int ma = (int)min((long)T - 1, p.M - 1 - m0), nb = (int)min((long)T - 1, p.N - 1 - n0);
+  term<X, E>(p.t[0], ma, nb, m0, n0, z, acc, S);
+  term<X, E>(p.t[1], ma, nb, m0, n0, z, acc, S);
+  term<!X, E>(p.t[2], ma, nb, m0, n0, z, acc, S);
+  term<!X, E>(p.t[3], ma, nb, m0, n0, z, acc, S);
   __syncthreads();  // the next item reuses the LDS
   // D[i][j] of a 16x16 f64 MFMA tile: lane = j + 16*(i%4), element i/4.
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lk = lane >> 4;
   // per 16-row block: C read (beta != 0) before any of the block's stores,
   // so the loads overlap instead of each waiting behind a store
+  // the descriptor's fields are read once (a store through C could alias them)
   CCGPU_GLOBAL double* C = gptr(p.C + z * p.c_b);
+  const long M = p.M, N = p.N, c_m = p.c_m, c_n = p.c_n;
+  const double beta = p.beta;
 #pragma unroll
   for (int i = 0; i < IW; ++i) {
     double cv[IW][4] = {};
-    if (p.beta != 0.0) {  // uniform; indices clamped into C: no per-element branch
+    if (beta != 0.0) {  // uniform; indices clamped into C: no per-element branch
 #pragma unroll
       for (int j = 0; j < IW; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const long m = min(m0 + wm * 64 + i * 16 + r * 4 + lk, p.M - 1);
-          const long n = min(n0 + wn * 64 + j * 16 + lr, p.N - 1);
-          cv[j][r] = C[m * p.c_m + n * p.c_n];
+          const long m = min(m0 + wm * 64 + i * 16 + r * 4 + lk, M - 1);
+          const long n = min(n0 + wn * 64 + j * 16 + lr, N - 1);
+          cv[j][r] = C[m * c_m + n * c_n];
         }
     }
 #pragma unroll
@@ -226,10 +176,10 @@ __device__ __forceinline__ void tile4(const DMulti& p, long m0, long n0, long z,
       for (int r = 0; r < 4; ++r) {
         const long m = m0 + wm * 64 + i * 16 + r * 4 + lk;
         const long n = n0 + wn * 64 + j * 16 + lr;
-        if (m < p.M && n < p.N) {
+        if (m < M && n < N) {
           double v = acc[i][j][r];
-          if (p.beta != 0.0) v += p.beta * cv[j][r];
-          C[m * p.c_m + n * p.c_n] = v;
+          if (beta != 0.0) v += beta * cv[j][r];
+          C[m * c_m + n * c_n] = v;
         }
       }
   }
@@ -554,8 +504,7 @@ __device__ __forceinline__ void pass_tile(const PtRun& r, long q, int ph, long t
     const DMulti& d = static_cast<const DMulti*>(r.desc)[q * 3 + ph];
     dt::Smem& GS = *reinterpret_cast<dt::Smem*>(lds);
     const long m0 = tmi * 128, n0 = tni * 128;
-    bool inside = m0 + 128 <= d.M && n0 + 128 <= d.N;  // interior tile: no bounds checks
-    for (int k = 0; k < 4; ++k) inside = inside && d.t[k].K % dt::TK == 0;
+    const bool inside = m0 + 128 <= d.M && n0 + 128 <= d.N;
     if (ph < 2) {
       if (inside)
         dt::tile4<true, false>(d, m0, n0, z, GS);
@@ -685,35 +634,57 @@ __device__ __forceinline__ void tile_xcd(long b, long tiles_m, long tiles_n, lon
   tile_grouped((b < full) ? (b % 8) * per + b / 8 : b, tiles_m, tiles_n, tm, tn);
 }
 
+// One W pass of several triples: blockIdx.y takes the triple (its descriptor
+// in list), blockIdx.z the batch, blockIdx.x the tile.  Bound by the matrix
+// cores once the chip is full, which a single triple's pass does not do below
+// v = 256 (80 to 101 blocks at v = 101, 50 us a launch).  The full list at
+// o=12 v=101, FP64: 87.9 ms in 1760 launches one triple at a time, 18.6 ms in
+// 70 with 26 triples each.
 template <bool X>
-__global__ __launch_bounds__(256, 2) void k_dtile4(DMulti p, long tiles_m, long tiles_n) {
+__global__ __launch_bounds__(256, 2) void k_dtile4(const DMulti* list, long tiles_m, long tiles_n) {
   __shared__ dt::Smem S;
+  const DMulti& p = list[blockIdx.y];
   long tm, tn;
   tile_xcd(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const long m0 = tm * 128, n0 = tn * 128;
-  bool inside = m0 + 128 <= p.M && n0 + 128 <= p.N;
-  for (int t = 0; t < 4; ++t) inside = inside && p.t[t].K % dt::TK == 0;
-  if (inside)
+  if (m0 + 128 <= p.M && n0 + 128 <= p.N)
     dt::tile4<X, false>(p, m0, n0, blockIdx.z, S);
   else
     dt::tile4<X, true>(p, m0, n0, blockIdx.z, S);
 }
 
+// The mixed passes: the 256x256 tile (W8) or the 128x128 one.
+template <bool W8>
+__global__ __launch_bounds__(W8 ? 512 : 256, W8 ? 1 : 2) void k_btile4(const BMulti* list, long tiles_m, long tiles_n) {
+  const BMulti& p = list[blockIdx.y];
+  long tm, tn;
+  tile_xcd(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  if constexpr (W8) {
+    __shared__ bf3w8::Smem S;
+    bf3w8::tile<float, true>(p, tm * bf3w8::DT, tn * bf3w8::DT, blockIdx.z, S);
+  } else {
+    __shared__ bf3::Smem<2> S;
+    bf3::tile<float, 2>(p, tm * 128, tn * 128, blockIdx.z, S);
+  }
+}
+
 // Item of block b: each XCD (block b runs on XCD b % 8) gets a contiguous
 // range of items, whose canonical blocks are neighbours along C and share W
 // cache lines in that XCD's L2 (the item's blocks, and so its partial, do not
-// depend on the mapping).
+// depend on the mapping).  Triple blockIdx.y of the group: its W slot and its
+// nE partials.
 template <typename WT>
-__global__ __launch_bounds__(256) void k_pt_energy_blocked(EArgs a, const WT* W, int i, int j, int k,
+__global__ __launch_bounds__(256) void k_pt_energy_blocked(EArgs a, const WT* W, long wslot, const int* tri,
                                                            double* part) {
   __shared__ ESmem<WT, 1, 256> S;
-  const long b = blockIdx.x, per = (long)gridDim.x / 8, full = per * 8;
-  energy_item<WT, 1, 256>(a, W, i, j, k, (b < full) ? (b % 8) * per + b / 8 : b, part, S);
+  const long b = blockIdx.x, per = (long)gridDim.x / 8, full = per * 8, t = blockIdx.y;
+  energy_item<WT, 1, 256>(a, W + t * wslot, tri[3 * t], tri[3 * t + 1], tri[3 * t + 2],
+                          (b < full) ? (b % 8) * per + b / 8 : b, part + 2 * a.nE * t, S);
 }
 
 __global__ __launch_bounds__(256) void k_reduce_pairs(const double* part, long n, double* out) {
   __shared__ double red[2][4];
-  reduce_partials<256>(part, n, out, red);
+  reduce_partials<256>(part + 2 * n * blockIdx.x, n, out + 2 * blockIdx.x, red);
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n) {
@@ -772,7 +743,7 @@ long env_long(const char* name, long dflt) {
 
 // Tiles of the three W passes: G1 v x v^2, G2 v batches of v x v, G3 v^2 x v.
 struct PassShape {
-  long tm[3], tn[3], batch[3], ng[3];
+  long M[3], N[3], tm[3], tn[3], batch[3], ng[3];
 };
 PassShape pass_shape(bool mixed, int v) {
   PassShape ps{};
@@ -782,6 +753,8 @@ PassShape pass_shape(bool mixed, int v) {
     // mixed: 256 x 256 tiles over operands padded to 256 rows; FP64: 128 x 128
     ps.tm[g] = mixed ? cdiv(bf16x3_rpad(Ms[g]), bf3w8::DT) : cdiv(Ms[g], 128);
     ps.tn[g] = mixed ? cdiv(bf16x3_rpad(Ns[g]), bf3w8::DT) : cdiv(Ns[g], 128);
+    ps.M[g] = Ms[g];
+    ps.N[g] = Ns[g];
     ps.batch[g] = Bs[g];
     ps.ng[g] = ps.tm[g] * ps.tn[g] * Bs[g];
   }
@@ -863,52 +836,104 @@ EArgs energy_args(const int* ctab, const double* J, const double* t1, const doub
 }
 }  // namespace
 
-// (T) as launches per triple: three W passes, the blocked energy, the sum.
+// Triples per launch of the W passes: enough for four waves of blocks over the
+// CUs (two 128 x 128 blocks or one 256 x 256 block per CU), at most 64, with
+// their W slots inside 256 MB, about what the last-level cache holds (G2, G3
+// and the energy re-read W).  One at v = 512.
+long CCSD::pt_group(bool mixed) const {
+  const PassShape ps = pass_shape(mixed, dm_.v);
+  const long fewest = std::min(std::min(ps.ng[0], ps.ng[1]), ps.ng[2]), vvv = (long)dm_.v * dm_.v * dm_.v;
+  const long fill = ((mixed ? 1024 : 2048) + fewest - 1) / fewest;
+  const long room = (256L << 20) / (vvv * (long)(mixed ? sizeof(float) : sizeof(double)));
+  return std::max<long>(1, std::min<long>({fill, room, 64, pt_ntriples()}));
+}
+
+// (T) as launches per group of triples: three W passes, the blocked energy,
+// the sums; the descriptors and indices of a range of triples are copied over
+// before its launches.
 void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, double* e5) {
   const bool mixed = pt_mode_ == GemmPrec::BF16X3;
   const int o = dm_.o, v = dm_.v;
   const long vv = (long)v * v, vvv = vv * v;
   const EArgs ea = energy_args(ptctab_.p, J_.p, t1_.p, eps_.p, o, v);
   const PassShape ps = pass_shape(mixed, v);
-  check_span(ptpart_.p, 0, 2 * ea.nE - 1, sizeof(double), "pt partials");
+  const long ng = pt_group(mixed);
+  const void* W = mixed ? (const void*)W32_.p : (const void*)Wt_.p;
+  check_span(ptpart_.p, 0, 2 * ea.nE * ng - 1, sizeof(double), "pt partials");
   check_span(ea.ctab, 0, ea.nct - 1, sizeof(int), "pt block table");
   check_span(ea.J, 0, dm_.nov2 - 1, sizeof(double), "pt J");
-  check_span(mixed ? (const void*)W32_.p : (const void*)Wt_.p, 0, vvv - 1, mixed ? sizeof(float) : sizeof(double),
-             "pt W");
+  check_span(W, 0, ng * vvv - 1, mixed ? sizeof(float) : sizeof(double), "pt W");
   etrip_.ensure(2 * (size_t)std::max<long>(n, 1));
-  // flops of the passes: two K = v and two K = o terms each
+  // flops of a pass of one triple: two K = v and two K = o terms
   const double fg = 2.0 * (2.0 * (double)vv * vv + 2.0 * (double)vv * v * o);
-  std::vector<unsigned char> hd(3 * pt_desc_bytes());
-  long idx = 0;
-  for (long t = first; idx < n; t += stride, ++idx) {
-    const int i = tri_i_[t], j = tri_j_[t], k = tri_k_[t];
-    pt_descs(i, j, k, 0, hd.data());
-    for (int g = 0; g < 3; ++g) {
-      const long ntiles = ps.tm[g] * ps.tn[g];
-      CCGPU_REQUIRE(ntiles < (1L << 24) && ps.batch[g] < 65536, "pt: grid too large");
-      if (mixed) {
-        bf16x3_run(reinterpret_cast<const BMulti*>(hd.data())[g], (int)ps.batch[g], true, fg, st_);
-      } else {
-        const DMulti& d = reinterpret_cast<const DMulti*>(hd.data())[g];
-        const dim3 grid((unsigned)ntiles, 1, (unsigned)ps.batch[g]);
-        const int id = prof_begin(g < 2 ? "k_dtile4<true>" : "k_dtile4<false>", fg, st_);
-        if (g < 2)
-          CCGPU_LAUNCH(k_dtile4<true>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
-        else
-          CCGPU_LAUNCH(k_dtile4<false>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
-        prof_end(id, st_);
-      }
+  constexpr long kRange = 4096;  // triples whose descriptors are held at once
+  const long nr = std::min(n, kRange);
+  const size_t dsz = pt_desc_bytes();
+  if (n > 0) {
+    ptdesc_.ensure(3 * nr * dsz);
+    pttri_.ensure(3 * (size_t)nr);
+    check_span(pttri_.p, 0, 3 * nr - 1, sizeof(int), "pt triples");
+  }
+  std::vector<unsigned char> hd(3 * nr * dsz), one(3 * dsz);
+  std::vector<int> ht(3 * nr);
+  for (long r0 = 0; r0 < n; r0 += kRange) {
+    const long nq = std::min(kRange, n - r0);
+    for (long q = 0; q < nq; ++q) {
+      const long t = first + (r0 + q) * stride;
+      const int i = tri_i_[t], j = tri_j_[t], k = tri_k_[t];
+      ht[3 * q] = i;
+      ht[3 * q + 1] = j;
+      ht[3 * q + 2] = k;
+      pt_descs(i, j, k, (int)(q % ng), one.data());
+      for (int g = 0; g < 3; ++g) std::memcpy(hd.data() + (g * nr + q) * dsz, one.data() + g * dsz, dsz);
     }
-    const int id = prof_begin(mixed ? "k_pt_energy_blocked<float>" : "k_pt_energy_blocked<double>", 0.0, st_);
-    if (mixed)
-      CCGPU_LAUNCH(k_pt_energy_blocked<float>, dim3((unsigned)ea.nE), dim3(256), 0, st_, ea, W32_.p, i, j, k,
-                   ptpart_.p);
-    else
-      CCGPU_LAUNCH(k_pt_energy_blocked<double>, dim3((unsigned)ea.nE), dim3(256), 0, st_, ea, Wt_.p, i, j, k,
-                   ptpart_.p);
-    prof_end(id, st_);
-    CCGPU_LAUNCH(k_reduce_pairs, dim3(1), dim3(256), 0, st_, ptpart_.p, ea.nE, etrip_.p + 2 * idx);
-    CCGPU_HIPX(hipGetLastError());
+    // the previous range's launches precede the copies on the stream, and the
+    // host arrays are refilled only after the copies have left them
+    CCGPU_HIPX(hipMemcpyAsync(ptdesc_.p, hd.data(), hd.size(), hipMemcpyHostToDevice, st_));
+    CCGPU_HIPX(hipMemcpyAsync(pttri_.p, ht.data(), 3 * nq * sizeof(int), hipMemcpyHostToDevice, st_));
+    CCGPU_HIPX(hipStreamSynchronize(st_));
+    for (long q0 = 0; q0 < nq; q0 += ng) {
+      const unsigned gn = (unsigned)std::min(ng, nq - q0);
+      for (int g = 0; g < 3; ++g) {
+        const unsigned char* list = ptdesc_.p + (g * nr + q0) * dsz;
+        const unsigned nb = (unsigned)ps.batch[g];
+        CCGPU_REQUIRE(ps.tm[g] * ps.tn[g] < (1L << 23) && ps.batch[g] < 65536, "pt: grid too large");
+        if (mixed) {
+          const BMulti* d = reinterpret_cast<const BMulti*>(list);
+          // the 256 tile where padding to 256 rows does not cost more than its higher rate gives
+          // (cost model of the BF16x3 GEMM) and the group fills the CUs with it
+          const long tm1 = cdiv(ps.M[g], 128), tn1 = cdiv(ps.N[g], 128);
+          const bool w8 = bf16x3_large_tile(ps.M[g], ps.N[g], (long)gn * nb);
+          const int id = prof_begin("k_gemm_bf16x3", fg * gn, st_);
+          if (w8)
+            CCGPU_LAUNCH(k_btile4<true>, dim3((unsigned)(ps.tm[g] * ps.tn[g]), gn, nb), dim3(512), 0, st_, d,
+                         ps.tm[g], ps.tn[g]);
+          else
+            CCGPU_LAUNCH(k_btile4<false>, dim3((unsigned)(tm1 * tn1), gn, nb), dim3(256), 0, st_, d, tm1, tn1);
+          prof_end(id, st_);
+        } else {
+          const DMulti* d = reinterpret_cast<const DMulti*>(list);
+          const dim3 grid((unsigned)(ps.tm[g] * ps.tn[g]), gn, nb);
+          const int id = prof_begin(g < 2 ? "k_dtile4<true>" : "k_dtile4<false>", fg * gn, st_);
+          if (g < 2)
+            CCGPU_LAUNCH(k_dtile4<true>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
+          else
+            CCGPU_LAUNCH(k_dtile4<false>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
+          prof_end(id, st_);
+        }
+      }
+      const int id = prof_begin(mixed ? "k_pt_energy_blocked<float>" : "k_pt_energy_blocked<double>", 0.0, st_);
+      const dim3 egrid((unsigned)ea.nE, gn);
+      if (mixed)
+        CCGPU_LAUNCH(k_pt_energy_blocked<float>, egrid, dim3(256), 0, st_, ea, W32_.p, vvv, pttri_.p + 3 * q0,
+                     ptpart_.p);
+      else
+        CCGPU_LAUNCH(k_pt_energy_blocked<double>, egrid, dim3(256), 0, st_, ea, Wt_.p, vvv, pttri_.p + 3 * q0,
+                     ptpart_.p);
+      prof_end(id, st_);
+      CCGPU_LAUNCH(k_reduce_pairs, dim3(gn), dim3(256), 0, st_, ptpart_.p, ea.nE, etrip_.p + 2 * (r0 + q0));
+      CCGPU_HIPX(hipGetLastError());
+    }
   }
   double s4 = 0.0, s5 = 0.0;
   if (n > 0) {
