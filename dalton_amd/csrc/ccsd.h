@@ -156,6 +156,8 @@ class CCSD {
   void dress(const double* t1);
   void ladder(const double* T, double* Om);
   void ladder_mixed(double* Om);
+  std::vector<int> ladder_strips(int a0, int a1, long rows, long tiles) const;
+  void ladder_y(int a0, int a1);
   void mark(const char* name);
   void ensure_work();
   // (T) drivers: launches per group of triples of the pre-packed three-pass W

@@ -260,6 +260,21 @@ void CCSD::dress(const double* t1) {
   (void)nov;
 }
 
+// a-strips of one ladder a-batch [a0, a1) for its integral product
+// Y[(a,c),(b,d)] = (ac|bd): V+/- reads the blocks b >= a only, so the strip
+// [s0, s1) is formed for b >= s0 and nearly half of the square is left out.
+// At most 16 strips, each with `tiles` 128 x 128 tiles over a product of
+// `rows` rows on average: two waves over the chip for Y (1024), so that the
+// last waves of the strips cost less than they save.
+// o=21 v=170 FP64: Y 17.9 -> 9.7 ms; o=32 v=256 mixed: 15.6 -> 8.9 ms.
+std::vector<int> CCSD::ladder_strips(int a0, int a1, long rows, long tiles) const {
+  const double v = dm_.v, have = rows * (a1 - a0) * v / (128.0 * 128.0);
+  const int n = (int)std::max(1.0, std::min({16.0, have / tiles, (double)(a1 - a0)}));
+  std::vector<int> s;
+  for (int q = 0; q <= n; ++q) s.push_back(a0 + (int)((long)(a1 - a0) * q / n));
+  return s;
+}
+
 // Particle-particle ladder sum_cd t_ij^cd (ac~|bd~) in the symmetric /
 // antisymmetric scheme (CC_BF/CC_BF1/CCRHS_IPM, cc/ccsd_rhs.F:9129,9319,7571):
 // V+/-_{ab,cd} = (ac|bd) +/- (ad|bc) for a<=b, c<=d, formed per a-batch from
@@ -277,12 +292,25 @@ void CCSD::ladder(const double* T, double* Om) {
     const int a0 = lad_batches_[bi], a1 = lad_batches_[bi + 1];
     long rows = 0;
     for (int a = a0; a < a1; ++a) rows += v - a;
-    const long M = (long)(a1 - a0) * v, Nn = (long)(v - a0) * v;
-    bulk(M, Nn, naux, 1.0, Bvv_.p + (long)a0 * v, 1, vv, Bvv_.p + (long)a0 * v, vv, 1, 0.0, Y_.p, Nn, 1);
+    const long Nn = (long)(v - a0) * v;
+    ladder_y(a0, a1);
     ladder_vpm(Vp_.p, Vm_.p, Y_.p, Nn, a0, a1, v, st_);
     bulk(rows, dm_.npo, dm_.npv, 1.0, Vp_.p, dm_.npv, 1, taup_.p, 1, dm_.npv, 0.0, Sp_.p, dm_.npo, 1);
     bulk(rows, dm_.npo, dm_.npv, 1.0, Vm_.p, dm_.npv, 1, taum_.p, 1, dm_.npv, 0.0, Sm_.p, dm_.npo, 1);
     ladder_scatter(Om, Sp_.p, Sm_.p, a0, a1, o, v, st_);
+  }
+}
+
+// Y of the a-batch [a0, a1) (rows (a,c) from a0, columns (b,d) from a0) in
+// strips; blocks b < a before a strip's first a are not written.
+void CCSD::ladder_y(int a0, int a1) {
+  const long v = dm_.v, vv = v * v, Nn = (v - a0) * v;
+  const Gemm bulk{bulk_, st_};
+  const std::vector<int> st = ladder_strips(a0, a1, Nn, 1024);
+  for (size_t q = 0; q + 1 < st.size(); ++q) {
+    const long s0 = st[q], s1 = st[q + 1];
+    const double* B = Bvv_.p + s0 * v;
+    bulk((s1 - s0) * v, (v - s0) * v, dm_.naux, 1.0, B, 1, vv, B, vv, 1, 0.0, Y_.p + (s0 - a0) * v * (Nn + 1), Nn, 1);
   }
 }
 
@@ -322,9 +350,14 @@ void CCSD::ladder_mixed(double* Om) {
     for (int a = a0; a < a1; ++a) rows += v - a;
     const long M = (long)(a1 - a0) * v, Nn = (long)(v - a0) * v;
     CCGPU_REQUIRE((size_t)(M * Nn) <= 2 * Y_.n, "ladder_mixed: Y block exceeds its buffer");
-    const BTerm ty{lpBh_.p + a0 * v * KpB, lpBl_.p + a0 * v * KpB, lpBh_.p + a0 * v * KpB,
-                   lpBl_.p + a0 * v * KpB, KpB, 0, 0};
-    bf16x3_multi(&ty, 1, M, Nn, 1, Y32, true, Nn, 1, 0, 1.0, 0.0, 2.0 * M * Nn * naux, st_);
+    const std::vector<int> strips = ladder_strips(a0, a1, Nn, 1024);
+    for (size_t q = 0; q + 1 < strips.size(); ++q) {
+      const long s0 = strips[q], Ms = (strips[q + 1] - s0) * v, Ns = (v - s0) * v;
+      const unsigned short *bh = lpBh_.p + s0 * v * KpB, *bl = lpBl_.p + s0 * v * KpB;
+      const BTerm ty{bh, bl, bh, bl, KpB, 0, 0};
+      bf16x3_multi(&ty, 1, Ms, Ns, 1, Y32 + (s0 - a0) * v * (Nn + 1), true, Nn, 1, 0, 1.0, 0.0, 2.0 * Ms * Ns * naux,
+                   st_);
+    }
     const long Rp = bf16x3_rpad(rows);
     ladder_vpm_pack(lpVh_.p, lpVl_.p, Y32, Nn, a0, a1, v, Rp, KpT, st_);
     const BTerm ts{lpVh_.p, lpVl_.p, lpTh_.p, lpTl_.p, KpT, Rp * KpT, RpT * KpT};

@@ -91,7 +91,7 @@ void CCSD::lhtr_ladder(const double* Xb) {
     for (int a = a0; a < a1; ++a) rows += v - a;
     const long M = (long)(a1 - a0) * v, Nn = (long)(v - a0) * v;
     const double* Bb = Bvv_.p + (long)a0 * v;
-    bulk(M, Nn, naux, 1.0, Bb, 1, vv, Bb, vv, 1, 0.0, Y_.p, Nn, 1);
+    ladder_y(a0, a1);
     ladder_vpm(Vp_.p, Vm_.p, Y_.p, Nn, a0, a1, v, st_);
     ladder_gather(Sp_.p, Sm_.p, Xb, a0, a1, o, v, st_);
     bulk(npo, npv, rows, 0.5, Sp_.p, 1, npo, Vp_.p, npv, 1, 1.0, taupb_.p, npv, 1);
@@ -100,9 +100,22 @@ void CCSD::lhtr_ladder(const double* Xb) {
     bulk(rows, npv, npo, 0.5, Sm_.p, npo, 1, taum_.p, npv, 1, 0.0, Vm_.p, npv, 1);
     fill(Y_.p, 0.0, M * Nn, st_);  // entries with b < a stay zero
     ladder_vpm_adj(Y_.p, Nn, Vp_.p, Vm_.p, a0, a1, v, st_);
+    // Y_bar is zero for b < a: the strip [s0, s1) of a sums over b >= s0, that
+    // of b over a < s1.  Both sums start and end at multiples of 64, the K
+    // padding of the packed operands, so they add the same terms in the same
+    // groups as the whole sums do.  K is the long side here and is not split in
+    // BF16x3: there a strip keeps one wave of output tiles (512).
     double* Bbb = Bvvb_.p + (long)a0 * v;
-    bulk(naux, M, Nn, 1.0, Bb, vv, 1, Y_.p, 1, Nn, 1.0, Bbb, vv, 1);
-    bulk(naux, Nn, M, 1.0, Bb, vv, 1, Y_.p, Nn, 1, 1.0, Bbb, vv, 1);
+    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::BF16X3 ? 512 : 64);
+    for (size_t q = 0; q + 1 < sa.size(); ++q) {
+      const long r0 = (long)(sa[q] - a0) * v, nr = (long)(sa[q + 1] - sa[q]) * v, k0 = r0 / 64 * 64;
+      bulk(naux, nr, Nn - k0, 1.0, Bb + k0, vv, 1, Y_.p + r0 * Nn + k0, 1, Nn, 1.0, Bbb + r0, vv, 1);
+    }
+    for (size_t q = 0; q + 1 < sa.size(); ++q) {
+      const long c0 = (long)(sa[q] - a0) * v, c1 = (long)(sa[q + 1] - a0) * v, k1 = std::min(M, (c1 + 63) / 64 * 64);
+      bulk(naux, c1 - c0, k1, 1.0, Bb, vv, 1, Y_.p + c0, Nn, 1, 1.0, Bbb + c0, vv, 1);
+    }
+    if (Nn > M) bulk(naux, Nn - M, M, 1.0, Bb, vv, 1, Y_.p + M, Nn, 1, 1.0, Bbb + M, vv, 1);
   }
 }
 
