@@ -190,15 +190,15 @@ class CCSD {
   hipStream_t st_ = nullptr;
 
   // inputs / constants
-  DBuf<double> eps_, B_, h_, Bov_, J_, K_, L_, Joovv_;
+  DBuf<double> eps_, B_, Bov_, J_, K_, L_, Joovv_;
   // dressing
-  DBuf<double> Bt_, Bvv_, Boo_, BvoT_, F_, ht_, Jd_, G1_, Gam_, Z_, W_, E1_, E2_, hx_;
+  DBuf<double> Bt_, Bvv_, Boo_, BvoT_, F_, Jd_, G1_, Gam_, Z_, W_, E1_, E2_, hx_;
   // amplitudes / residual
   DBuf<double> t1_, T_, om1_, Om_;
   DBuf<double> rt1_, rT_;  // amplitudes handed to residual_host (ccgpu_rhs)
   DBuf<double> bufR_, bufX2_, bufTx_, bufU_, bufC_, bufD_;
   // ladder
-  DBuf<double> taup_, taum_, Y_, Vp_, Vm_, Sp_, Sm_;
+  DBuf<double> tau_, Y_, V_, S_;  // tau, V and S: the + array, then the - array
   std::vector<int> lad_batches_;
   // mixed-precision ladder: bf16 hi/lo of Bvv [(a,c)][P], tau+/- [s][ij][cd],
   // V+/- [s][r][cd]; S+/- [s][r][ij]
@@ -231,7 +231,7 @@ class CCSD {
   bool lhtr_ready_ = false;
   GemmPrec lhtr_prec_ = GemmPrec::F64;
   DBuf<double> Tb_, Ub_, Txb_, Db_, Btb_, Bvvb_, Boob_, BvoTb_, Zb_, Wb_, Fb_, E1b_, E2b_, Jdb_, Gamb_, G1b_,
-      taupb_, taumb_, vecb_;
+      taub_, vecb_;
   // trial-vector staging (two in, two out slots) and the copy stream
   DBuf<double> lst_;
   hipStream_t cst_ = nullptr;

@@ -51,22 +51,23 @@ CCSD::CCSD(int o, int v, int naux, const double* eps_host, const double* B_host,
   const long N = dm_.N, nov = dm_.nov, nov2 = dm_.nov2;
 
   eps_.alloc(N);
-  B_.alloc((size_t)naux * N * N);
+  B_.alloc((size_t)(naux + 1) * N * N);  // the factor, then h: both are T1-dressed alike
   CCGPU_HIPX(hipMemcpyAsync(eps_.p, eps_host, N * sizeof(double), hipMemcpyHostToDevice, st_));
-  CCGPU_HIPX(hipMemcpyAsync(B_.p, B_host, B_.bytes(), hipMemcpyHostToDevice, st_));
+  CCGPU_HIPX(hipMemcpyAsync(B_.p, B_host, (size_t)naux * N * N * sizeof(double), hipMemcpyHostToDevice, st_));
 
   // implicit one-electron operator: h = diag(eps) - sum_k [2(pq|kk) - (pk|kq)]
-  h_.alloc(N * N);
-  Jd_.alloc(naux);
+  double* h = B_.p + (long)naux * N * N;
+  Jd_.alloc(naux + 1);  // the last entry stays 1: the weight of the dressed h in the Fock matrix
+  fill(Jd_.p + naux, 1.0, 1, st_);
   coulomb_diag(Jd_.p, B_.p, naux, (int)N, o, st_);
-  gemv_mc(N * N, naux, -1.0, B_.p, N * N, Jd_.p, 0.0, h_.p, st_);
-  g(N, N, (long)naux * o, 1.0, B_.p, N, 1, B_.p, N, 1, 1.0, h_.p, N, 1, st_, 1, 0, 0, 0, o, N * N, N * N);
+  gemv_mc(N * N, naux, -1.0, B_.p, N * N, Jd_.p, 0.0, h, st_);
+  g(N, N, (long)naux * o, 1.0, B_.p, N, 1, B_.p, N, 1, 1.0, h, N, 1, st_, 1, 0, 0, 0, o, N * N, N * N);
   if (!dryrun()) {
     std::vector<double> hh(N * N);
-    CCGPU_HIPX(hipMemcpyAsync(hh.data(), h_.p, N * N * sizeof(double), hipMemcpyDeviceToHost, st_));
+    CCGPU_HIPX(hipMemcpyAsync(hh.data(), h, N * N * sizeof(double), hipMemcpyDeviceToHost, st_));
     CCGPU_HIPX(hipStreamSynchronize(st_));
     for (long p = 0; p < N; ++p) hh[p * N + p] += eps_host[p];
-    CCGPU_HIP(hipMemcpy(h_.p, hh.data(), N * N * sizeof(double), hipMemcpyHostToDevice));
+    CCGPU_HIP(hipMemcpy(h, hh.data(), N * N * sizeof(double), hipMemcpyHostToDevice));
   }
 
   // ovov constants: J = (kc|ld), K = X(J) = (kd|lc), L = 2J - K, Joovv[(k,l),(c,d)]
@@ -106,12 +107,11 @@ void CCSD::ensure_work() {
   const long N = dm_.N, nov = dm_.nov, nov2 = dm_.nov2;
   (void)N;
   // per-iteration buffers
-  Bt_.alloc((size_t)naux * N * N);
+  Bt_.alloc((size_t)(naux + 1) * N * N);
   Bvv_.alloc((size_t)naux * v * v);
   Boo_.alloc((size_t)naux * o * o);
   BvoT_.alloc((size_t)naux * nov);
   F_.alloc(N * N);
-  ht_.alloc(N * N);
   hx_.alloc(nov);
   G1_.alloc((size_t)o * o * o * o);
   Gam_.alloc((size_t)o * o * o * o);
@@ -125,8 +125,7 @@ void CCSD::ensure_work() {
   bufU_.alloc(nov2);
   bufC_.alloc(nov2);
   bufD_.alloc(nov2);
-  taup_.alloc(dm_.npo * dm_.npv);
-  taum_.alloc(dm_.npo * dm_.npv);
+  tau_.alloc(2 * dm_.npo * dm_.npv);
 
   // particle-ladder batches over a: V+/- rows (a,b>=a) x npv and the
   // Y[(a,c),(b,d)] block must fit a fixed budget; rows < 65536 (grid.y).
@@ -166,10 +165,8 @@ void CCSD::ensure_work() {
   maxr = std::max(maxr, rows);
   maxy = std::max(maxy, (long)(v - a0) * v * (long)(v - a0) * v);
   Y_.alloc(maxy);
-  Vp_.alloc(maxr * dm_.npv);
-  Vm_.alloc(maxr * dm_.npv);
-  Sp_.alloc(maxr * dm_.npo);
-  Sm_.alloc(maxr * dm_.npo);
+  V_.alloc(2 * maxr * dm_.npv);
+  S_.alloc(2 * maxr * dm_.npo);
 
   work_ = true;
 }
@@ -193,10 +190,10 @@ void CCSD::reset_cycle() {
 
 void CCSD::release_work() {
   if (!work_) return;
-  for (DBuf<double>* b : {&Bt_, &Bvv_, &Boo_, &BvoT_, &F_, &ht_, &hx_, &G1_, &Gam_, &Z_, &W_, &E1_, &E2_,
-                          &bufR_, &bufX2_, &bufTx_, &bufU_, &bufC_, &bufD_, &taup_, &taum_, &Y_, &Vp_,
-                          &Vm_, &Sp_, &Sm_, &S2_, &diisS_, &diisE_, &Tb_, &Ub_, &Txb_, &Db_, &Btb_, &Bvvb_, &Boob_,
-                          &BvoTb_, &Zb_, &Wb_, &Fb_, &E1b_, &E2b_, &Jdb_, &Gamb_, &G1b_, &taupb_, &taumb_, &vecb_,
+  for (DBuf<double>* b : {&Bt_, &Bvv_, &Boo_, &BvoT_, &F_, &hx_, &G1_, &Gam_, &Z_, &W_, &E1_, &E2_,
+                          &bufR_, &bufX2_, &bufTx_, &bufU_, &bufC_, &bufD_, &tau_, &Y_, &V_, &S_, &S2_,
+                           &diisS_, &diisE_, &Tb_, &Ub_, &Txb_, &Db_, &Btb_, &Bvvb_, &Boob_,
+                          &BvoTb_, &Zb_, &Wb_, &Fb_, &E1b_, &E2b_, &Jdb_, &Gamb_, &G1b_, &taub_, &vecb_,
                           &lst_, &rt1_, &rT_})
     b->release();
   for (DBuf<unsigned short>* b : {&lpBh_, &lpBl_, &lpTh_, &lpTl_, &lpVh_, &lpVl_}) b->release();
@@ -240,23 +237,17 @@ void CCSD::mark(const char* name) { prof_phase(name, st_); }
 void CCSD::dress(const double* t1) {
   const int o = dm_.o, v = dm_.v, naux = dm_.naux;
   const long N = dm_.N, NN = N * N, nov = dm_.nov;
+  // the factor and h (slice naux) together
   CCGPU_HIPX(hipMemcpyAsync(Bt_.p, B_.p, B_.bytes(), hipMemcpyDeviceToDevice, st_));
   // Bt[P][o+a][q] -= sum_l t(l,a) B[P][l][q]
-  g(v, N, o, -1.0, t1, 1, v, B_.p, N, 1, 1.0, Bt_.p + o * N, N, 1, st_, naux, 0, NN, NN);
+  g(v, N, o, -1.0, t1, 1, v, B_.p, N, 1, 1.0, Bt_.p + o * N, N, 1, st_, naux + 1, 0, NN, NN);
   // Bt[P][p][i] += sum_a Bt[P][p][o+a] t(i,a)
-  g(N, o, v, 1.0, Bt_.p + o, N, 1, t1, 1, v, 1.0, Bt_.p, N, 1, st_, naux, NN, 0, NN);
-  CCGPU_HIPX(hipMemcpyAsync(ht_.p, h_.p, NN * sizeof(double), hipMemcpyDeviceToDevice, st_));
-  g(v, N, o, -1.0, t1, 1, v, h_.p, N, 1, 1.0, ht_.p + o * N, N, 1, st_);
-  g(N, o, v, 1.0, ht_.p + o, N, 1, t1, 1, v, 1.0, ht_.p, N, 1, st_);
+  g(N, o, v, 1.0, Bt_.p + o, N, 1, t1, 1, v, 1.0, Bt_.p, N, 1, st_, naux + 1, NN, 0, NN);
   // F = ht + sum_P Bt[P] * 2 sum_k Bt[P,k,k] - sum_{P,k} Bt[P,p,k] Bt[P,k,q]
   coulomb_diag(Jd_.p, Bt_.p, naux, (int)N, o, st_);
-  CCGPU_HIPX(hipMemcpyAsync(F_.p, ht_.p, NN * sizeof(double), hipMemcpyDeviceToDevice, st_));
-  gemv_mc(NN, naux, 1.0, Bt_.p, NN, Jd_.p, 1.0, F_.p, st_);
+  gemv_mc(NN, naux + 1, 1.0, Bt_.p, NN, Jd_.p, 0.0, F_.p, st_);
   g(N, N, (long)naux * o, -1.0, Bt_.p, N, 1, Bt_.p, N, 1, 1.0, F_.p, N, 1, st_, 1, 0, 0, 0, o, NN, NN);
-  // contiguous blocks
-  perm(Bvv_.p, Bt_.p + o * N + o, 1, naux, v, v, 0, NN, N, 1, 1.0, 0.0, st_);
-  perm(Boo_.p, Bt_.p, 1, naux, o, o, 0, NN, N, 1, 1.0, 0.0, st_);
-  perm(BvoT_.p, Bt_.p + o * N, 1, naux, o, v, 0, NN, 1, N, 1.0, 0.0, st_);
+  split_dressed(Bvv_.p, Boo_.p, BvoT_.p, Bt_.p, o, v, naux, st_);
   (void)nov;
 }
 
@@ -294,10 +285,11 @@ void CCSD::ladder(const double* T, double* Om) {
     for (int a = a0; a < a1; ++a) rows += v - a;
     const long Nn = (long)(v - a0) * v;
     ladder_y(a0, a1);
-    ladder_vpm(Vp_.p, Vm_.p, Y_.p, Nn, a0, a1, v, st_);
-    bulk(rows, dm_.npo, dm_.npv, 1.0, Vp_.p, dm_.npv, 1, taup_.p, 1, dm_.npv, 0.0, Sp_.p, dm_.npo, 1);
-    bulk(rows, dm_.npo, dm_.npv, 1.0, Vm_.p, dm_.npv, 1, taum_.p, 1, dm_.npv, 0.0, Sm_.p, dm_.npo, 1);
-    ladder_scatter(Om, Sp_.p, Sm_.p, a0, a1, o, v, st_);
+    const long nv = rows * dm_.npv, ns = rows * dm_.npo;  // V-, S- follow V+, S+
+    ladder_vpm(V_.p, V_.p + nv, Y_.p, Nn, a0, a1, v, st_);
+    bulk(rows, dm_.npo, dm_.npv, 1.0, V_.p, dm_.npv, 1, tau_.p, 1, dm_.npv, 0.0, S_.p, dm_.npo, 1, 2, nv,
+         dm_.npo * dm_.npv, ns);
+    ladder_scatter(Om, S_.p, S_.p + ns, a0, a1, o, v, st_);
   }
 }
 
@@ -339,8 +331,7 @@ void CCSD::ladder_mixed(double* Om) {
   lpVl_.ensure((size_t)2 * RpV * KpT);
   S2_.ensure((size_t)2 * maxr * npo);
   bf16x3_pack(Bvv_.p, vv, naux, 1, vv, 0, 1, RpB, KpB, 1.0f, lpBh_.p, lpBl_.p, st_);
-  bf16x3_pack(taup_.p, npo, npv, npv, 1, 0, 1, RpT, KpT, 1.0f, lpTh_.p, lpTl_.p, st_);
-  bf16x3_pack(taum_.p, npo, npv, npv, 1, 0, 1, RpT, KpT, 1.0f, lpTh_.p + RpT * KpT, lpTl_.p + RpT * KpT, st_);
+  bf16x3_pack(tau_.p, npo, npv, npv, 1, npo * npv, 2, RpT, KpT, 1.0f, lpTh_.p, lpTl_.p, st_);
   float* Y32 = reinterpret_cast<float*>(Y_.p);
   double* Sp = S2_.p;
   double* Sm = S2_.p + maxr * npo;
@@ -375,6 +366,7 @@ void CCSD::residual(const double* t1, const double* T, double* om1, double* Om) 
   const long N = dm_.N, nov = dm_.nov, nov2 = dm_.nov2, oo = (long)o * o, vv = (long)v * v;
   mark("start");
   dress(t1);
+  fock_blocks(E1_.p, E2_.p, hx_.p, om1, F_.p, o, v, st_);  // E1, E2, F_kc, and om1 = F~_ai
   mark("dress");
 
   // A2 integral part: (ai~|bj~)
@@ -384,7 +376,7 @@ void CCSD::residual(const double* t1, const double* T, double* om1, double* Om) 
   // Too[(i,j),(a,b)] (into bufR), tau+/-, hole-hole ladder (CCRHS_A :2505)
   double* Too = bufR_.p;
   perm(Too, T, o, o, v, v, (long)v * nov, v, nov, 1, 1.0, 0.0, st_);
-  ladder_tau(taup_.p, taum_.p, Too, o, v, st_);
+  ladder_tau(tau_.p, tau_.p + dm_.npo * dm_.npv, Too, o, v, st_);
   g(oo, oo, naux, 1.0, Boo_.p, 1, oo, Boo_.p, oo, 1, 0.0, G1_.p, oo, 1, st_);  // [(k,i),(l,j)]
   perm(Gam_.p, G1_.p, o, o, o, o, oo * o, o, oo, 1, 1.0, 0.0, st_);               // [(k,l),(i,j)]
   bulk(oo, oo, vv, 1.0, Joovv_.p, vv, 1, Too, 1, vv, 1.0, Gam_.p, oo, 1);
@@ -399,15 +391,12 @@ void CCSD::residual(const double* t1, const double* T, double* om1, double* Om) 
   // ring terms (CCRHS_C/CIO :4272,7656; CCRHS_D/DIO :3525,8023)
   double* Tx = bufTx_.p;
   double* U = bufU_.p;
-  perm(Tx, T, o, v, o, v, v, nov, (long)v * nov, 1, 1.0, 0.0, st_);
-  perm(U, T, 1, 1, 1, nov2, 0, 0, 0, 1, 2.0, 0.0, st_);
-  perm(U, Tx, 1, 1, 1, nov2, 0, 0, 0, 1, -1.0, 1.0, st_);
+  exchange_tu(Tx, U, T, o, v, st_);
   double* R = bufR_.p;
   bulk(vv, oo, naux, 1.0, Bvv_.p, 1, vv, Boo_.p, oo, 1, 0.0, R, oo, 1);  // [(a,c),(k,i)] = (ki~|ac~)
   double* C = bufC_.p;
   double* D = bufD_.p;
-  perm(C, R, o, v, o, v, 1, (long)v * oo, o, oo, 1.0, 0.0, st_);   // C[(i,a),(k,c)]
-  perm(D, R, o, v, o, v, 1, (long)v * oo, o, oo, -1.0, 0.0, st_);  // D = -(ac~|ki~)
+  ring_integrals(C, D, R, o, v, st_);  // C[(i,a),(k,c)], D = -(ac~|ki~)
   mark("CD_int");
   bulk(nov, nov, nov, -0.5, Tx, nov, 1, K_.p, nov, 1, 1.0, C, nov, 1);
   bulk(nov, nov, naux, 2.0, BvoT_.p, 1, nov, Bov_.p, nov, 1, 1.0, D, nov, 1);
@@ -416,16 +405,13 @@ void CCSD::residual(const double* t1, const double* T, double* om1, double* Om) 
   double* P = bufR_.p;
   double* X2 = bufX2_.p;
   bulk(nov, nov, nov, 1.0, C, nov, 1, Tx, nov, 1, 0.0, P, nov, 1);
-  perm(X2, P, 1, 1, 1, nov2, 0, 0, 0, 1, -0.5, 0.0, st_);
-  perm(X2, P, o, v, o, v, v, nov, (long)v * nov, 1, -1.0, 1.0, st_);
+  exchange_ring(X2, P, o, v, st_);
   bulk(nov, nov, nov, 0.5, D, nov, 1, U, nov, 1, 1.0, X2, nov, 1);
   mark("CD_contract");
 
   // E terms (CCRHS_EI/EFCK/E :3158,8604,2280)
-  perm(E1_.p, F_.p + o * N + o, 1, 1, v, v, 0, 0, N, 1, 1.0, 0.0, st_);
   g(v, v, (long)o * nov, -1.0, U, nov, 1, J_.p, 1, nov, 1.0, E1_.p, v, 1, st_, 1, 0, 0, 0, nov,
     (long)v * nov, (long)v * nov);
-  perm(E2_.p, F_.p, 1, 1, o, o, 0, 0, N, 1, 1.0, 0.0, st_);
   g(o, o, (long)v * nov, 1.0, J_.p, (long)v * nov, 1, U, 1, (long)v * nov, 1.0, E2_.p, o, 1, st_, 1, 0,
     0, 0, nov, nov, nov);
   g(oo * v, v, v, 1.0, T, v, 1, E1_.p, 1, v, 1.0, X2, v, 1, st_);
@@ -433,19 +419,16 @@ void CCSD::residual(const double* t1, const double* T, double* om1, double* Om) 
   mark("E");
 
   // Om += X2 + X2^T  (P_ij^ab)
-  perm(Om, X2, 1, 1, 1, nov2, 0, 0, 0, 1, 1.0, 1.0, st_);
-  perm(Om, X2, 1, 1, nov, nov, 0, 0, 1, nov, 1.0, 1.0, st_);
+  add_sym(Om, X2, nov, st_);
   mark("sym");
 
   // singles (CCRHS_G/H/I/J :2986,2858,2450,2686)
   bulk(naux, nov, nov, 1.0, Bov_.p, nov, 1, U, nov, 1, 0.0, Z_.p, nov, 1);
-  g(o, v, (long)naux * v, 1.0, Z_.p, v, 1, Bvv_.p, 1, v, 0.0, om1, v, 1, st_, 1, 0, 0, 0, v, nov, vv);
+  g(o, v, (long)naux * v, 1.0, Z_.p, v, 1, Bvv_.p, 1, v, 1.0, om1, v, 1, st_, 1, 0, 0, 0, v, nov, vv);
   g(oo, nov, naux, 1.0, Boo_.p, 1, oo, Bov_.p, nov, 1, 0.0, W_.p, nov, 1, st_);
   g(o, v, (long)o * nov, -1.0, W_.p, nov, 1, U, 1, nov, 1.0, om1, v, 1, st_, 1, 0, 0, 0, nov,
     (long)o * nov, (long)v * nov);
-  perm(hx_.p, F_.p + o, 1, 1, o, v, 0, 0, N, 1, 1.0, 0.0, st_);  // F_kc
   gemv_mc(nov, nov, 1.0, U, nov, hx_.p, 1.0, om1, st_);
-  perm(om1, F_.p + o * N, 1, 1, o, v, 0, 0, 1, N, 1.0, 1.0, st_);  // F~_ai
   mark("singles");
 }
 

@@ -152,8 +152,8 @@ void gemm(const GemmDesc& d, GemmPrec prec, hipStream_t s);
 
 // FP64 GEMM autotuner.  While enabled, the first call of every new shape
 // class (M, N, K, two-level K, batch, operand orders) with fewer than 1024
-// 128 x 128 tiles times each candidate launch configuration (the planned one
-// and block tiles 128, 64 and 32 without a split) on its stream and
+// 128 x 128 tiles times each candidate launch configuration (block tiles 128,
+// 64 and 32, each with its planned split of K) on its stream and
 // caches the fastest; later calls of that shape use it, enabled or not.  Timing runs the GEMM for real, so a tuning pass gives throwaway
 // results.  Never tunes during graph capture or a dry run.
 void autotune_enable(bool on);

@@ -51,7 +51,7 @@ __device__ __forceinline__ void tile_of(long b, long tiles_m, long tiles_n, long
 // by the matrix cores, has one LDS stage (two barriers a step); the smaller
 // tiles, bound by the latency of a step, two stages and one barrier.
 template <int AMODE, int BMODE, bool K2, int T>
-__global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, unsigned magic, double* ws) {
+__global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int nz, unsigned magic, double* ws) {
   constexpr int TM = T, TN = T, TK = Step<T>::TK;
   constexpr int IW = T / 32;      // MFMA tiles per wave and dimension
   constexpr int NS = T == 128 ? 1 : 2;
@@ -69,13 +69,14 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, unsig
   const double* A = static_cast<const double*>(d.A) + m0 * d.a_m;
   const double* B = static_cast<const double*>(d.B) + n0 * d.b_n;
   long kbeg = 0, kend = d.K;
+  long z = blockIdx.z;  // batch; with split K, batch x chunk
   if (kchunk > 0) {
-    kbeg = (long)blockIdx.z * kchunk;
+    z = blockIdx.z / nz;
+    kbeg = (blockIdx.z - z * nz) * kchunk;
     kend = min(d.K, kbeg + kchunk);
-  } else {
-    A += (long)blockIdx.z * d.a_b;
-    B += (long)blockIdx.z * d.b_b;
   }
+  A += z * d.a_b;
+  B += z * d.b_b;
   const KMap ka{d.a_k, d.a_ko, (unsigned)d.Kin, magic}, kb{d.b_k, d.b_ko, (unsigned)d.Kin, magic};
   const int ma = (int)min((long)TM - 1, d.M - 1 - m0), nb = (int)min((long)TN - 1, d.N - 1 - n0);
   const long nfull = (kend - kbeg) / TK;
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, unsig
 
     // D[i][j] of a 16x16 f64 MFMA tile: lane = j + 16*(i%4), element i/4.
     if (kchunk > 0) {
-      // split-K partial: ws[z][m][n] (dense M x N)
+      // split-K partial: ws[batch][chunk][m][n] (dense M x N)
       double* W = ws + (long)blockIdx.z * d.M * d.N;
 #pragma unroll
       for (int i = 0; i < IW; ++i)
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, unsig
     }
     // per 16-row block: C read (beta != 0) before any of the block's stores,
     // so the loads overlap instead of each waiting behind a store
-    double* C = static_cast<double*>(d.C) + (long)blockIdx.z * d.c_b;
+    double* C = static_cast<double*>(d.C) + z * d.c_b;
 #pragma unroll
     for (int i = 0; i < IW; ++i) {
       double cv[IW][4] = {};
@@ -222,6 +223,8 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_f64(GemmDesc d, int nz, c
   constexpr int E = 256 / G;
   __shared__ double part[G][E];
   const long mn = d.M * d.N;
+  ws += (long)blockIdx.y * nz * mn;
+  double* C = static_cast<double*>(d.C) + (long)blockIdx.y * d.c_b;
   const int x = threadIdx.x % E, g = threadIdx.x / E;
   for (long e0 = (long)blockIdx.x * E; e0 < mn; e0 += (long)gridDim.x * E) {
     const long e = e0 + x;
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_f64(GemmDesc d, int nz, c
         for (int q = 1; q < G; ++q) s += part[q][x];
       }
       const long m = e / d.N, n = e - m * d.N;
-      double* p = static_cast<double*>(d.C) + m * d.c_m + n * d.c_n;
+      double* p = C + m * d.c_m + n * d.c_n;
       double v = d.alpha * s;
       if (d.beta != 0.0) v += d.beta * *p;
       *p = v;
@@ -262,16 +265,16 @@ const char* const kDgemmName[2][2][2][3] = {
 bool two_level(const GemmDesc& d) { return d.Kin > 0 && d.Kin < d.K; }
 
 template <int AM, int BM, int T>
-void launch_f64(const GemmDesc& d, dim3 grid, long kchunk, double* ws, hipStream_t s) {
+void launch_f64(const GemmDesc& d, dim3 grid, long kchunk, int nz, double* ws, hipStream_t s) {
   const bool k2 = two_level(d);
   const unsigned magic =
       k2 ? (unsigned)std::min<unsigned long long>(0xFFFFFFFFull, (1ull << 32) / (unsigned long long)d.Kin) : 0u;
   const int id = prof_begin(kDgemmName[AM][BM][k2 ? 1 : 0][T == 128 ? 0 : (T == 64 ? 1 : 2)],
                             2.0 * d.M * d.N * d.K * d.batch, s);
   if (k2)
-    CCGPU_LAUNCH((k_dgemm<AM, BM, true, T>), grid, dim3(256), 0, s, d, kchunk, magic, ws);
+    CCGPU_LAUNCH((k_dgemm<AM, BM, true, T>), grid, dim3(256), 0, s, d, kchunk, nz, magic, ws);
   else
-    CCGPU_LAUNCH((k_dgemm<AM, BM, false, T>), grid, dim3(256), 0, s, d, kchunk, magic, ws);
+    CCGPU_LAUNCH((k_dgemm<AM, BM, false, T>), grid, dim3(256), 0, s, d, kchunk, nz, magic, ws);
   prof_end(id, s);
 }
 
@@ -300,17 +303,19 @@ double cost_f64(const GemmDesc& d, int T, long nz) {
   const double last = left <= 0.0 ? 0.0 : (full == 0 && left <= 256.0 ? kOne[q] : kTwo[q]);
   const double us = 3.5 + steps / kMhz * (full * kTwo[q] + last) * (two_level(d) ? 1.15 : 1.0);
   const double cbytes = 8.0 * d.batch * (double)d.M * d.N * (d.beta != 0.0 ? 2.0 : 1.0);
-  return std::max(us, cbytes / 4.0e6) + (nz > 1 ? 2.5 + 0.02 * nz + (double)nz * d.M * d.N * 16.0 / 3.0e6 : 0.0);
+  return std::max(us, cbytes / 4.0e6) + (nz > 1 ? 2.5 + 0.02 * nz + (double)nz * d.batch * d.M * d.N * 16.0 / 3.0e6 : 0.0);
 }
 
-// The configuration of least estimated time.
-F64Cfg plan_f64(const GemmDesc& d) {
+// The configuration of least estimated time, of one tile (only) or of all.
+F64Cfg plan_f64(const GemmDesc& d, int only = 0) {
   F64Cfg best;
   double bt = 1e300;
   for (int T : {128, 64, 32}) {
-    // chunks of at least two K steps
-    const long kmax = d.batch == 1 ? std::max<long>(1, d.K / (2 * (2048 / T))) : 1;
-    for (long nz = 1; nz <= std::min<long>(kmax, 256); nz = nz < 4 ? nz + 1 : nz + nz / 3) {
+    if (only && T != only) continue;
+    // chunks of at least two K steps; partials of at most 4 GB
+    const double room = 4.0e9 / (8.0 * d.batch * (double)d.M * d.N);
+    const long kmax = std::max<long>(1, std::min<long>(d.K / (2 * (2048 / T)), (long)std::min(room, 1e6)));
+    for (long nz = 1; nz <= std::min<long>({kmax, 256, 65535 / d.batch}); nz = nz < 4 ? nz + 1 : nz + nz / 3) {
       const double t = cost_f64(d, T, nz);
       if (t < bt) {
         bt = t;
@@ -377,26 +382,26 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
   const int T = cfg.tile;
   const long tiles = (long)cdiv(d.M, T) * cdiv(d.N, T);
   long kchunk = 0;
-  int nz = d.batch;
+  int nz = 1;
   double* ws = nullptr;
-  if (cfg.nz > 1 && d.batch == 1) {
+  if (cfg.nz > 1) {
     const long tk = 2048 / T;  // chunks are whole K steps
     const long chunk = cdiv(cdiv(d.K, cfg.nz), tk) * tk;
     nz = (int)cdiv(d.K, chunk);
     if (nz >= 2) {
       kchunk = chunk;
-      ws = grow_scratch(scratch_for(s).splitk, static_cast<size_t>(nz) * d.M * d.N, s);
+      ws = grow_scratch(scratch_for(s).splitk, static_cast<size_t>(nz) * d.batch * d.M * d.N, s);
     }
   }
-  CCGPU_REQUIRE(nz <= 65535, "gemm: too many batches");
+  CCGPU_REQUIRE((long)nz * d.batch <= 65535, "gemm: too many batches");
   CCGPU_REQUIRE(tiles < (1L << 24), "gemm: too many tiles");
   CCGPU_REQUIRE(!two_level(d) || d.K < (1L << 32), "gemm: two-level K too long");
-  dim3 grid((unsigned)tiles, 1, nz);
+  dim3 grid((unsigned)tiles, 1, (unsigned)(nz * d.batch));
 #define CCGPU_F64_LAUNCH(TT)                                                   \
-  if (am == KFAST && bm == KFAST) launch_f64<KFAST, KFAST, TT>(d, grid, kchunk, ws, s); \
-  else if (am == KFAST) launch_f64<KFAST, RFAST, TT>(d, grid, kchunk, ws, s);          \
-  else if (bm == KFAST) launch_f64<RFAST, KFAST, TT>(d, grid, kchunk, ws, s);          \
-  else launch_f64<RFAST, RFAST, TT>(d, grid, kchunk, ws, s);
+  if (am == KFAST && bm == KFAST) launch_f64<KFAST, KFAST, TT>(d, grid, kchunk, nz, ws, s); \
+  else if (am == KFAST) launch_f64<KFAST, RFAST, TT>(d, grid, kchunk, nz, ws, s);          \
+  else if (bm == KFAST) launch_f64<RFAST, KFAST, TT>(d, grid, kchunk, nz, ws, s);          \
+  else launch_f64<RFAST, RFAST, TT>(d, grid, kchunk, nz, ws, s);
   if (T == 32) {
     CCGPU_F64_LAUNCH(32)
   } else if (T == 64) {
@@ -410,10 +415,10 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
     const long mn = d.M * d.N;
     unsigned nb = static_cast<unsigned>(std::min<long>((mn + 255) / 256, 4096));
     if (nz > 4)
-      CCGPU_LAUNCH(k_splitk_reduce_f64<8>, dim3((unsigned)std::min<long>((mn + 31) / 32, 8192)), dim3(256), 0, s, d, nz,
+      CCGPU_LAUNCH(k_splitk_reduce_f64<8>, dim3((unsigned)std::min<long>((mn + 31) / 32, 8192), d.batch), dim3(256), 0, s, d, nz,
                    ws);
     else
-      CCGPU_LAUNCH(k_splitk_reduce_f64<1>, dim3(nb), dim3(256), 0, s, d, nz, ws);
+      CCGPU_LAUNCH(k_splitk_reduce_f64<1>, dim3(nb, d.batch), dim3(256), 0, s, d, nz, ws);
     CCGPU_HIPX(hipGetLastError());
   }
 }
@@ -421,7 +426,9 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
 // Times every candidate configuration of this shape (the GEMM runs for real,
 // so tuning passes produce throwaway results) and returns the fastest.
 F64Cfg tune_f64(const GemmDesc& d, int am, int bm, hipStream_t s) {
-  const F64Cfg p = plan_f64(d), cands[4] = {p, {128, 1}, {64, 1}, {32, 1}};
+  // each tile with its planned chunks (an unsplit K of a million, one block
+  // walking it, would take a third of a second a run)
+  const F64Cfg cands[3] = {plan_f64(d, 128), plan_f64(d, 64), plan_f64(d, 32)};
   hipEvent_t e0, e1;
   CCGPU_HIP(hipEventCreate(&e0));
   CCGPU_HIP(hipEventCreate(&e1));

@@ -53,6 +53,18 @@ void ladder_vpm(double* vp, double* vm, const double* Y, long ldY, int a0, int a
 void ladder_scatter(double* om2, const double* sp, const double* sm, int a0, int a1, int o, int v,
                     hipStream_t st);
 
+// Fused passes of the residual: contiguous blocks of the dressed factor; the
+// blocks of the dressed Fock matrix (E1 = F_bc, E2 = F_kj, fkc = F_kc,
+// fai[i][a] = F_ai); with X(M)[(i,a),(j,b)] = M[(j,a),(i,b)], Tx = X(T) and
+// U = 2 T - Tx, and out = -P/2 - X(P); C[(i,a),(k,c)] = R[(a,c),(k,i)] and
+// D = -C; Om += X + X^T.
+void split_dressed(double* Bvv, double* Boo, double* BvoT, const double* Bt, int o, int v, long naux, hipStream_t st);
+void fock_blocks(double* E1, double* E2, double* fkc, double* fai, const double* F, int o, int v, hipStream_t st);
+void exchange_tu(double* Tx, double* U, const double* T, int o, int v, hipStream_t st);
+void exchange_ring(double* out, const double* P, int o, int v, hipStream_t st);
+void ring_integrals(double* C, double* D, const double* R, int o, int v, hipStream_t st);
+void add_sym(double* Om, const double* X, long n, hipStream_t st);
+
 // Jd[P] = 2 * sum_k Bt[P][k][k]
 void coulomb_diag(double* Jd, const double* Bt, long naux, int N, int o, hipStream_t st);
 

@@ -158,20 +158,37 @@ double* partials(long n, hipStream_t s) { return grow_scratch(scratch_for(s).par
 }  // namespace
 
 // ------------------------------------------------------------------ gemv
-__global__ void k_gemv_mc(long M, long K, long kchunk, double alpha, const double* A, long lda,
-                          const double* x, double* part) {
-  const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
+// 32 rows m per block, eight groups of threads over this block's K chunk: eight
+// independent chains of strided loads per row instead of one (a K of 110 on
+// 576 rows, one thread per row: 19 us; now 4.8).  With one chunk the result
+// goes straight to y, otherwise to partials summed in chunk order.
+__global__ __launch_bounds__(256) void k_gemv_mc(long M, long K, long kchunk, double alpha, const double* A, long lda,
+                                                 const double* x, double beta, double* y, double* part) {
+  __shared__ double sh[8][32];
+  const int tx = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const long m = (long)blockIdx.x * 32 + tx;
   const long k0 = (long)blockIdx.y * kchunk, k1 = min(K, k0 + kchunk);
   double s = 0.0;
-  for (long k = k0; k < k1; ++k) s += A[k * lda + m] * x[k];
-  part[(long)blockIdx.y * M + m] = alpha * s;
+  if (m < M) {
+#pragma unroll 8
+    for (long k = k0 + g; k < k1; k += 8) s += A[k * lda + m] * x[k];
+  }
+  sh[g][tx] = s;
+  __syncthreads();
+  if (g != 0 || m >= M) return;
+  for (int q = 1; q < 8; ++q) s += sh[q][tx];
+  s *= alpha;
+  if (part)
+    part[(long)blockIdx.y * M + m] = s;
+  else
+    y[m] = (beta != 0.0 ? beta * y[m] : 0.0) + s;
 }
 
 __global__ void k_gemv_finish(long M, int nk, const double* part, double beta, double* y) {
   const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= M) return;
   double s = 0.0;
+#pragma unroll 8
   for (int b = 0; b < nk; ++b) s += part[(long)b * M + m];
   y[m] = (beta != 0.0 ? beta * y[m] : 0.0) + s;
 }
@@ -184,15 +201,16 @@ void gemv_mc(long M, long K, double alpha, const double* A, long lda, const doub
     check_span(x, 0, K - 1, sizeof(double), "gemv x");
   }
   check_span(y, 0, M - 1, sizeof(double), "gemv y");
-  const long mb = (M + 255) / 256;
-  long nk = std::max<long>(1, std::min<long>(std::max<long>(1, 2048 / mb), (K + 255) / 256));
-  const long kchunk = (K + nk - 1) / nk;
-  nk = (K + kchunk - 1) / kchunk;
-  if (nk < 1) nk = 1;
-  double* part = partials(nk * M, st);
-  CCGPU_LAUNCH(k_gemv_mc, dim3((unsigned)mb, (unsigned)nk), dim3(256), 0, st, M, K, kchunk,
-                     alpha, A, lda, x, part);
-  CCGPU_LAUNCH(k_gemv_finish, dim3((unsigned)mb), dim3(256), 0, st, M, (int)nk, part, beta, y);
+  // K chunks: about eight blocks per CU, no chunk below 128
+  const long mb = (M + 31) / 32;
+  long nk = std::max<long>(1, std::min<long>({2048 / mb, K / 128, 65535}));
+  const long kchunk = std::max<long>(1, (K + nk - 1) / nk);
+  nk = std::max<long>(1, (K + kchunk - 1) / kchunk);
+  double* part = nk > 1 ? partials(nk * M, st) : nullptr;
+  CCGPU_LAUNCH(k_gemv_mc, dim3((unsigned)mb, (unsigned)nk), dim3(256), 0, st, M, K, kchunk, alpha, A, lda, x, beta, y,
+               part);
+  if (nk > 1)
+    CCGPU_LAUNCH(k_gemv_finish, dim3(cdiv(M, 256)), dim3(256), 0, st, M, (int)nk, part, beta, y);
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -203,27 +221,35 @@ __global__ void k_pack_sym(double* __restrict__ packed, const double* __restrict
   for (long ai = threadIdx.x; ai <= bj; ai += blockDim.x) packed[base + ai] = F[bj * n + ai];
 }
 
-__global__ void k_unpack_lower(double* __restrict__ F, const double* __restrict__ packed, long n) {
-  const long bj = blockIdx.x;
-  const long base = bj * (bj + 1) / 2;
-  for (long ai = threadIdx.x; ai <= bj; ai += blockDim.x) F[bj * n + ai] = packed[base + ai];
+__device__ __forceinline__ void tri_decode(long p, long& lo, long& hi) {
+  // p = hi*(hi+1)/2 + lo, 0 <= lo <= hi
+  long h = (long)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
+  while (h * (h + 1) / 2 > p) --h;
+  while ((h + 1) * (h + 2) / 2 <= p) ++h;
+  hi = h;
+  lo = p - h * (h + 1) / 2;
 }
 
-// F[c][r] = F[r][c] for c > r (copy lower triangle to upper), 32x32 tiles
-__global__ void k_mirror_lower(double* F, long n) {
+// Both triangles of F from the packed lower one, a 32x32 tile and its mirror
+// image per block.
+__global__ void k_unpack_sym(double* __restrict__ F, const double* __restrict__ packed, long n) {
   __shared__ double tile[32][33];
-  const long tr = blockIdx.y, tc = blockIdx.x;  // source tile (row tr, col tc), tr >= tc
-  if (tc > tr) return;
+  long tr, tc;
+  tri_decode(blockIdx.x, tc, tr);
   const int tx = threadIdx.x, ty = threadIdx.y;
 #pragma unroll
   for (int k = 0; k < 32; k += 8) {
     const long r = tr * 32 + ty + k, c = tc * 32 + tx;
-    if (r < n && c < n) tile[ty + k][tx] = F[r * n + c];
+    if (r < n && c <= r) {
+      const double x = packed[r * (r + 1) / 2 + c];
+      F[r * n + c] = x;
+      tile[ty + k][tx] = x;
+    }
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < 32; k += 8) {
-    const long r = tc * 32 + ty + k, c = tr * 32 + tx;  // destination (row r, col c) = src (c, r)
+    const long r = tc * 32 + ty + k, c = tr * 32 + tx;  // the mirror image of element (c, r)
     if (r < n && c < n && c > r) F[r * n + c] = tile[tx][ty + k];
   }
 }
@@ -240,10 +266,9 @@ void unpack_sym(double* F, const double* packed, long n, hipStream_t st) {
   if (n <= 0) return;
   check_span(packed, 0, n * (n + 1) / 2 - 1, sizeof(double), "unpack_sym packed");
   check_span(F, 0, n * n - 1, sizeof(double), "unpack_sym F");
-  CCGPU_LAUNCH(k_unpack_lower, dim3((unsigned)n), dim3(256), 0, st, F, packed, n);
-  const unsigned nt = cdiv(n, 32);
-  CCGPU_REQUIRE(nt < 65536, "unpack_sym: n too large");
-  CCGPU_LAUNCH(k_mirror_lower, dim3(nt, nt), dim3(32, 8), 0, st, F, n);
+  const long nt = cdiv(n, 32);
+  CCGPU_REQUIRE(nt * (nt + 1) / 2 < (1L << 24), "unpack_sym: n too large");  // 2^32 work-items along x
+  CCGPU_LAUNCH(k_unpack_sym, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(32, 8), 0, st, F, packed, n);
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -439,15 +464,6 @@ void ccsd_energy_packed(double* out, const double* L, const double* t2p, const d
 }
 
 // ------------------------------------------------------------------ ladder helpers
-__device__ __forceinline__ void tri_decode(long p, long& lo, long& hi) {
-  // p = hi*(hi+1)/2 + lo, 0 <= lo <= hi
-  long h = (long)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
-  while (h * (h + 1) / 2 > p) --h;
-  while ((h + 1) * (h + 2) / 2 <= p) ++h;
-  hi = h;
-  lo = p - h * (h + 1) / 2;
-}
-
 __global__ void k_ladder_tau(double* __restrict__ taup, double* __restrict__ taum,
                              const double* __restrict__ Too, int o, int v) {
   const long q = blockIdx.y;  // ij, i <= j
@@ -915,60 +931,75 @@ void multidot_slot(double* dots, const double* diisE, long ld, const int* ctr, i
   CCGPU_HIPX(hipGetLastError());
 }
 
-// One thread: Dalton's bordered DIIS system
+// Dalton's bordered DIIS system
 //   [ B  -1 ] [c]   [ 0]
 //   [-1   0 ] [l] = [-1]
-// solved by Gaussian elimination with partial pivoting.
-__global__ void k_diis_solve(double* Amat, int LD, const double* dots, double* coef, int* ctr, int mx,
-                             double* M) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const int ivec = diis_ivec(ctr[0], mx), nloop = ivec, n = nloop + 1;
-  for (int i = 0; i < nloop; ++i) {
+// solved by Gaussian elimination with partial pivoting, one block, the matrix
+// in LDS up to 31 vectors (in M beyond): element updates in parallel, pivot
+// search and back substitution by one thread (a chain of dependent global
+// accesses in one thread took 25 us for eight vectors; 7 us now).
+constexpr int kDiisLds = 32;
+__global__ __launch_bounds__(256) void k_diis_solve(double* Amat, int LD, const double* dots, double* coef, int* ctr,
+                                                    int mx, double* work) {
+  __shared__ double sm[kDiisLds * (kDiisLds + 1)];
+  __shared__ int piv;
+  const int ivec = diis_ivec(ctr[0], mx), nloop = ivec, n = nloop + 1, t = threadIdx.x;
+  double* M = n <= kDiisLds ? sm : work;
+  double* b = M + n * n;
+  for (int i = t; i < nloop; i += 256) {
     Amat[i * LD + (ivec - 1)] = dots[i];
     Amat[(ivec - 1) * LD + i] = dots[i];
   }
-  double* b = M + n * n;
-  for (int i = 0; i < n; ++i) {
-    for (int j = 0; j < n; ++j) M[i * n + j] = 0.0;
-    b[i] = 0.0;
+  __syncthreads();
+  for (int e = t; e < n * n; e += 256) {
+    const int i = e / n, j = e - i * n;
+    M[e] = (i < nloop && j < nloop) ? Amat[i * LD + j] : (i == nloop && j == nloop ? 0.0 : -1.0);
   }
-  for (int i = 0; i < nloop; ++i) {
-    for (int j = 0; j < nloop; ++j) M[i * n + j] = Amat[i * LD + j];
-    M[i * n + nloop] = -1.0;
-    M[nloop * n + i] = -1.0;
-  }
-  b[nloop] = -1.0;
+  for (int i = t; i < n; i += 256) b[i] = i == nloop ? -1.0 : 0.0;
+  __syncthreads();
   for (int j = 0; j < n; ++j) {
-    int p = j;
-    for (int i = j + 1; i < n; ++i)
-      if (fabs(M[i * n + j]) > fabs(M[p * n + j])) p = i;
-    if (M[p * n + j] == 0.0) {
-      ctr[1] = 1;
-      for (int i = 0; i < nloop; ++i) coef[i] = (i == ivec - 1) ? 1.0 : 0.0;
+    if (t == 0) {
+      int p = j;
+      for (int i = j + 1; i < n; ++i)
+        if (fabs(M[i * n + j]) > fabs(M[p * n + j])) p = i;
+      piv = M[p * n + j] == 0.0 ? -1 : p;
+    }
+    __syncthreads();
+    const int p = piv;
+    if (p < 0) {
+      if (t == 0) ctr[1] = 1;
+      for (int i = t; i < nloop; i += 256) coef[i] = (i == ivec - 1) ? 1.0 : 0.0;
       return;
     }
     if (p != j) {
-      for (int k = 0; k < n; ++k) {
-        const double t = M[j * n + k];
-        M[j * n + k] = M[p * n + k];
-        M[p * n + k] = t;
+      for (int k = t; k <= n; k += 256) {
+        double &x = k < n ? M[j * n + k] : b[j], &y = k < n ? M[p * n + k] : b[p];
+        const double q = x;
+        x = y;
+        y = q;
       }
-      const double t = b[j];
-      b[j] = b[p];
-      b[p] = t;
+      __syncthreads();
     }
-    for (int i = j + 1; i < n; ++i) {
+    const int w = n - j;  // columns j + 1 .. n - 1 and b (column j is not read again)
+    for (int e = t; e < (n - 1 - j) * w; e += 256) {
+      const int i = j + 1 + e / w, k = j + 1 + e % w;
       const double f = M[i * n + j] / M[j * n + j];
-      for (int k = j; k < n; ++k) M[i * n + k] -= f * M[j * n + k];
-      b[i] -= f * b[j];
+      if (k < n)
+        M[i * n + k] -= f * M[j * n + k];
+      else
+        b[i] -= f * b[j];
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    for (int i = n - 1; i >= 0; --i) {
+      double s = b[i];
+      for (int k = i + 1; k < n; ++k) s -= M[i * n + k] * b[k];
+      b[i] = s / M[i * n + i];
     }
   }
-  for (int i = n - 1; i >= 0; --i) {
-    double s = b[i];
-    for (int k = i + 1; k < n; ++k) s -= M[i * n + k] * b[k];
-    b[i] = s / M[i * n + i];
-  }
-  for (int i = 0; i < nloop; ++i) coef[i] = b[i];
+  __syncthreads();
+  for (int i = t; i < nloop; i += 256) coef[i] = b[i];
 }
 
 void diis_solve(double* Amat, int ld, const double* dots, double* coef, int* ctr, int mx, double* work,
@@ -979,7 +1010,7 @@ void diis_solve(double* Amat, int ld, const double* dots, double* coef, int* ctr
   check_span(coef, 0, mx - 1, sizeof(double), "diis_solve coef");
   check_span(work, 0, (long)(mx + 1) * (mx + 2) - 1, sizeof(double), "diis_solve work");
   check_span(ctr, 0, 1, sizeof(int), "diis_solve ctr");
-  CCGPU_LAUNCH(k_diis_solve, dim3(1), dim3(64), 0, st, Amat, ld, dots, coef, ctr, mx, work);
+  CCGPU_LAUNCH(k_diis_solve, dim3(1), dim3(256), 0, st, Amat, ld, dots, coef, ctr, mx, work);
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -1028,6 +1059,205 @@ void report4(double* out, const double* scal, const int* ctr, hipStream_t st) {
   check_span(scal, 0, 1, sizeof(double), "report4 scal");
   check_span(ctr, 0, 1, sizeof(int), "report4 ctr");
   CCGPU_LAUNCH(k_report4, dim3(1), dim3(64), 0, st, out, scal, ctr);
+  CCGPU_HIPX(hipGetLastError());
+}
+}  // namespace ccgpu
+
+namespace ccgpu {
+// ------------------------------------------------ fused passes of the residual
+// Contiguous blocks of the dressed factor: Bvv [P][a][c], Boo [P][k][i],
+// BvoT [P][(i,a)] (transposed through LDS).  blockIdx.y = P; blockIdx.x runs
+// over eight rows of Bvv, eight rows of Boo, or a 32x32 tile of BvoT.
+__global__ void k_split_dressed(double* __restrict__ Bvv, double* __restrict__ Boo, double* __restrict__ BvoT,
+                                const double* __restrict__ Bt, int o, int v, int ga, int gk, int ti) {
+  __shared__ double tile[32][33];
+  const long N = o + v, P = blockIdx.y;
+  const double* S = Bt + P * N * N;
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  int x = blockIdx.x;
+  if (x < ga) {
+    const int a = x * 8 + ty;
+    if (a < v)
+      for (int c = tx; c < v; c += 32) Bvv[(P * v + a) * v + c] = S[(o + a) * N + o + c];
+    return;
+  }
+  x -= ga;
+  if (x < gk) {
+    const int k = x * 8 + ty;
+    if (k < o)
+      for (int i = tx; i < o; i += 32) Boo[(P * o + k) * o + i] = S[k * N + i];
+    return;
+  }
+  x -= gk;
+  const int i0 = (x % ti) * 32, a0 = (x / ti) * 32;
+#pragma unroll
+  for (int q = 0; q < 32; q += 8) {
+    const int a = a0 + ty + q, i = i0 + tx;
+    if (a < v && i < o) tile[ty + q][tx] = S[(o + a) * N + i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 32; q += 8) {
+    const int i = i0 + ty + q, a = a0 + tx;
+    if (a < v && i < o) BvoT[P * o * v + (long)i * v + a] = tile[tx][ty + q];
+  }
+}
+
+void split_dressed(double* Bvv, double* Boo, double* BvoT, const double* Bt, int o, int v, long naux, hipStream_t st) {
+  const long N = o + v;
+  check_span(Bt, 0, naux * N * N - 1, sizeof(double), "split_dressed Bt");
+  check_span(Bvv, 0, naux * v * v - 1, sizeof(double), "split_dressed Bvv");
+  check_span(Boo, 0, naux * o * o - 1, sizeof(double), "split_dressed Boo");
+  check_span(BvoT, 0, naux * o * v - 1, sizeof(double), "split_dressed BvoT");
+  const int ga = (int)cdiv(v, 8), gk = (int)cdiv(o, 8), ti = (int)cdiv(o, 32);
+  const unsigned nx = (unsigned)(ga + gk + ti * (int)cdiv(v, 32));
+  for (long p0 = 0; p0 < naux; p0 += 65535)
+    CCGPU_LAUNCH(k_split_dressed, dim3(nx, (unsigned)std::min<long>(65535, naux - p0)), dim3(32, 8), 0, st,
+                 Bvv + p0 * v * v, Boo + p0 * o * o, BvoT + p0 * o * v, Bt + p0 * N * N, o, v, ga, gk, ti);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+// Blocks of the dressed Fock matrix: E1 = F_bc, E2 = F_kj, fkc = F_kc, fai[i][a] = F_ai.
+__global__ void k_fock_blocks(double* E1, double* E2, double* fkc, double* fai, const double* F, int o, int v) {
+  const long N = o + v;
+  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < N * N; e += (long)gridDim.x * blockDim.x) {
+    const long p = e / N, q = e - p * N;
+    const double x = F[e];
+    if (p < o && q < o)
+      E2[p * o + q] = x;
+    else if (p < o)
+      fkc[p * v + q - o] = x;
+    else if (q < o)
+      fai[q * v + p - o] = x;
+    else
+      E1[(p - o) * v + q - o] = x;
+  }
+}
+
+void fock_blocks(double* E1, double* E2, double* fkc, double* fai, const double* F, int o, int v, hipStream_t st) {
+  const long N = o + v;
+  check_span(F, 0, N * N - 1, sizeof(double), "fock_blocks F");
+  check_span(E1, 0, (long)v * v - 1, sizeof(double), "fock_blocks E1");
+  check_span(E2, 0, (long)o * o - 1, sizeof(double), "fock_blocks E2");
+  check_span(fkc, 0, (long)o * v - 1, sizeof(double), "fock_blocks fkc");
+  check_span(fai, 0, (long)o * v - 1, sizeof(double), "fock_blocks fai");
+  CCGPU_LAUNCH(k_fock_blocks, dim3((unsigned)std::min<long>(4096, cdiv(N * N, 256))), dim3(256), 0, st, E1, E2, fkc, fai,
+               F, o, v);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+// Row (i,a) of M per block and of X(M)[(i,a),(j,b)] = M[(j,a),(i,b)] beside it.
+template <bool TXU>
+__global__ void k_exchange2(double* __restrict__ out, double* __restrict__ out2, const double* __restrict__ M, int o,
+                            int v) {
+  const int nov = o * v, r = blockIdx.x, i = r / v, a = r - i * v;
+  const double* m = M + (long)r * nov;
+  for (int c = threadIdx.x; c < nov; c += blockDim.x) {
+    const int j = c / v, b = c - j * v;
+    const double x = m[c], y = M[(long)(j * v + a) * nov + i * v + b];
+    const long e = (long)r * nov + c;
+    if (TXU) {
+      out[e] = y;
+      out2[e] = 2.0 * x - y;
+    } else {
+      out[e] = -0.5 * x - y;
+    }
+  }
+}
+
+namespace {
+void check_nov(const double* p, int o, int v, const char* what) {
+  const long nov = (long)o * v;
+  CCGPU_REQUIRE(nov < (1L << 24), "residual: o*v too large");
+  check_span(p, 0, nov * nov - 1, sizeof(double), what);
+}
+}  // namespace
+
+// Tx = X(T), U = 2 T - Tx.
+void exchange_tu(double* Tx, double* U, const double* T, int o, int v, hipStream_t st) {
+  check_nov(T, o, v, "exchange T");
+  check_nov(Tx, o, v, "exchange Tx");
+  check_nov(U, o, v, "exchange U");
+  CCGPU_LAUNCH(k_exchange2<true>, dim3((unsigned)(o * v)), dim3(256), 0, st, Tx, U, T, o, v);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+// out = -P/2 - X(P).
+void exchange_ring(double* out, const double* P, int o, int v, hipStream_t st) {
+  check_nov(P, o, v, "exchange P");
+  check_nov(out, o, v, "exchange out");
+  CCGPU_LAUNCH(k_exchange2<false>, dim3((unsigned)(o * v)), dim3(256), 0, st, out, (double*)nullptr, P, o, v);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+// C[(i,a),(k,c)] = R[(a,c),(k,i)], D = -C: per a, the v x o^2 matrix R[a]
+// transposed through LDS.
+__global__ void k_ring_integrals(double* __restrict__ C, double* __restrict__ D, const double* __restrict__ R, int o,
+                                 int v) {
+  __shared__ double tile[32][33];
+  const long a = blockIdx.z, oo = (long)o * o, nov = (long)o * v;
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  const long c0 = (long)blockIdx.x * 32, q0 = (long)blockIdx.y * 32;
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const long c = c0 + ty + k, q = q0 + tx;
+    if (c < v && q < oo) tile[ty + k][tx] = R[(a * v + c) * oo + q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const long q = q0 + ty + k, c = c0 + tx;
+    if (c < v && q < oo) {
+      const long kk = q / o, i = q - kk * o, e = (i * v + a) * nov + kk * v + c;
+      const double x = tile[tx][ty + k];
+      C[e] = x;
+      D[e] = -x;
+    }
+  }
+}
+
+void ring_integrals(double* C, double* D, const double* R, int o, int v, hipStream_t st) {
+  check_nov(C, o, v, "ring C");
+  check_nov(D, o, v, "ring D");
+  check_span(R, 0, (long)v * v * o * o - 1, sizeof(double), "ring R");
+  CCGPU_REQUIRE(v < 65536 && cdiv((long)o * o, 32) < 65536, "ring_integrals: space too large");
+  CCGPU_LAUNCH(k_ring_integrals, dim3(cdiv(v, 32), cdiv((long)o * o, 32), (unsigned)v), dim3(32, 8), 0, st, C, D, R, o,
+               v);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+// Om += X + X^T: a 32x32 tile and its mirror image per block.
+__global__ void k_add_sym(double* __restrict__ Om, const double* __restrict__ X, long n) {
+  __shared__ double lo[32][33], up[32][33];
+  long tr, tc;
+  tri_decode(blockIdx.x, tc, tr);
+  const int tx = threadIdx.x, ty = threadIdx.y;
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    long r = tr * 32 + ty + k, c = tc * 32 + tx;
+    if (r < n && c < n) lo[ty + k][tx] = X[r * n + c];
+    r = tc * 32 + ty + k;
+    c = tr * 32 + tx;
+    if (r < n && c < n) up[ty + k][tx] = X[r * n + c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    long r = tr * 32 + ty + k, c = tc * 32 + tx;
+    if (r < n && c < n) Om[r * n + c] = (Om[r * n + c] + lo[ty + k][tx]) + up[tx][ty + k];
+    if (tr == tc) continue;
+    r = tc * 32 + ty + k;
+    c = tr * 32 + tx;
+    if (r < n && c < n) Om[r * n + c] = (Om[r * n + c] + up[ty + k][tx]) + lo[tx][ty + k];
+  }
+}
+
+void add_sym(double* Om, const double* X, long n, hipStream_t st) {
+  check_span(Om, 0, n * n - 1, sizeof(double), "add_sym Om");
+  check_span(X, 0, n * n - 1, sizeof(double), "add_sym X");
+  const long nt = cdiv(n, 32);
+  CCGPU_REQUIRE(nt * (nt + 1) / 2 < (1L << 24), "add_sym: n too large");
+  CCGPU_LAUNCH(k_add_sym, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(32, 8), 0, st, Om, X, n);
   CCGPU_HIPX(hipGetLastError());
 }
 }  // namespace ccgpu

@@ -42,8 +42,7 @@ void CCSD::ensure_lhtr() {
   Jdb_.alloc(naux);
   Gamb_.alloc((size_t)o * o * o * o);
   G1b_.alloc((size_t)o * o * o * o);
-  taupb_.alloc(dm_.npo * dm_.npv);
-  taumb_.alloc(dm_.npo * dm_.npv);
+  taub_.alloc(2 * dm_.npo * dm_.npv);
   vecb_.alloc(2 * nov);
 }
 
@@ -83,8 +82,7 @@ void CCSD::lhtr_ladder(const double* Xb) {
   const int o = dm_.o, v = dm_.v, naux = dm_.naux;
   const long vv = (long)v * v, npo = dm_.npo, npv = dm_.npv;
   const Gemm bulk{bulk_, st_};
-  fill(taupb_.p, 0.0, npo * npv, st_);
-  fill(taumb_.p, 0.0, npo * npv, st_);
+  fill(taub_.p, 0.0, 2 * npo * npv, st_);
   for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
     const int a0 = lad_batches_[bi], a1 = lad_batches_[bi + 1];
     long rows = 0;
@@ -92,14 +90,13 @@ void CCSD::lhtr_ladder(const double* Xb) {
     const long M = (long)(a1 - a0) * v, Nn = (long)(v - a0) * v;
     const double* Bb = Bvv_.p + (long)a0 * v;
     ladder_y(a0, a1);
-    ladder_vpm(Vp_.p, Vm_.p, Y_.p, Nn, a0, a1, v, st_);
-    ladder_gather(Sp_.p, Sm_.p, Xb, a0, a1, o, v, st_);
-    bulk(npo, npv, rows, 0.5, Sp_.p, 1, npo, Vp_.p, npv, 1, 1.0, taupb_.p, npv, 1);
-    bulk(npo, npv, rows, 0.5, Sm_.p, 1, npo, Vm_.p, npv, 1, 1.0, taumb_.p, npv, 1);
-    bulk(rows, npv, npo, 0.5, Sp_.p, npo, 1, taup_.p, npv, 1, 0.0, Vp_.p, npv, 1);
-    bulk(rows, npv, npo, 0.5, Sm_.p, npo, 1, taum_.p, npv, 1, 0.0, Vm_.p, npv, 1);
+    const long nv = rows * npv, ns = rows * npo, nt = npo * npv;  // the - arrays follow the + ones
+    ladder_vpm(V_.p, V_.p + nv, Y_.p, Nn, a0, a1, v, st_);
+    ladder_gather(S_.p, S_.p + ns, Xb, a0, a1, o, v, st_);
+    bulk(npo, npv, rows, 0.5, S_.p, 1, npo, V_.p, npv, 1, 1.0, taub_.p, npv, 1, 2, ns, nv, nt);
+    bulk(rows, npv, npo, 0.5, S_.p, npo, 1, tau_.p, npv, 1, 0.0, V_.p, npv, 1, 2, ns, nt, nv);
     fill(Y_.p, 0.0, M * Nn, st_);  // entries with b < a stay zero
-    ladder_vpm_adj(Y_.p, Nn, Vp_.p, Vm_.p, a0, a1, v, st_);
+    ladder_vpm_adj(Y_.p, Nn, V_.p, V_.p + nv, a0, a1, v, st_);
     // Y_bar is zero for b < a: the strip [s0, s1) of a sums over b >= s0, that
     // of b over a < s1.  Both sums start and end at multiples of 64, the K
     // padding of the packed operands, so they add the same terms in the same
@@ -194,7 +191,7 @@ void CCSD::lhtr_apply(const double* l1, double* Xb, double* rho1, double* rho2s)
   lhtr_ladder(Xb);
   double* Toob = Db_.p;
   fill(Toob, 0.0, nov2, st_);
-  ladder_tau_adj(Toob, taupb_.p, taumb_.p, o, v, st_);
+  ladder_tau_adj(Toob, taub_.p, taub_.p + dm_.npo * dm_.npv, o, v, st_);
   mark("lhtr_ladder");
 
   // hole ladder: Gam = perm(Boo^T Boo) + Joovv Too^T, LADh = Gam^T Too
@@ -228,9 +225,9 @@ void CCSD::lhtr_apply(const double* l1, double* Xb, double* rho1, double* rho2s)
   g(o, v, (long)naux * N, 1.0, Btb, 1, N, Bt + o, N, 1, 0.0, rho1, v, 1, st_);
   g((long)naux * N, v, o, 1.0, Btb, N, 1, t1, v, 1, 1.0, Btb + o, N, 1, st_);
   g(o, v, (long)naux * N, -1.0, B_.p, N, 1, Btb + o * N, 1, N, 1.0, rho1, v, 1, st_, 1, 0, 0, 0, N, NN, NN);
-  g(o, v, N, 1.0, Fb, 1, N, ht_.p + o, N, 1, 1.0, rho1, v, 1, st_);
+  g(o, v, N, 1.0, Fb, 1, N, Bt + naux * NN + o, N, 1, 1.0, rho1, v, 1, st_);
   g(N, v, o, 1.0, Fb, N, 1, t1, v, 1, 1.0, Fb + o, N, 1, st_);
-  g(o, v, N, -1.0, h_.p, N, 1, Fb + o * N, 1, N, 1.0, rho1, v, 1, st_);
+  g(o, v, N, -1.0, B_.p + naux * NN, N, 1, Fb + o * N, 1, N, 1.0, rho1, v, 1, st_);
   mark("lhtr_fock_dressing");
 
   // packed-storage fold of the doubles gradient
