@@ -17,6 +17,7 @@
 
 #include "bf16x3_tile.h"
 #include "common.h"
+#include "kernels.h"
 
 namespace ccgpu {
 
@@ -30,6 +31,18 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 }
 __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(static_cast<unsigned int>(h) << 16); }
 
+// Two elements split together: packed hi and lo pairs (the conversion
+// instruction rounds to nearest even like f2bf).
+__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{a, b}, bf2v));
+}
+__device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
+  hi = pk_bf16(a, b);
+  lo = pk_bf16(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xFFFF0000u));
+}
+
 struct PackDesc {
   const double* src;
   long rows, K;              // logical operand: rows x K
@@ -39,51 +52,97 @@ struct PackDesc {
   float scale;  // multiplies every element
 };
 
+template <bool K2>
 __device__ __forceinline__ long pk_koff(const PackDesc& p, long k) {
-  if (p.Kin > 0 && p.Kin < p.K) {
+  if (K2) {
     const long ko = k / p.Kin;
     return ko * p.s_ko + (k - ko * p.Kin) * p.s_k;
   }
   return k * p.s_k;
 }
 
-// 32x32 tiles of (row, k); RFAST reads along rows (through LDS), otherwise along k.
-template <bool RFAST_>
-__global__ void k_pack_bf16x2(PackDesc p, unsigned short* __restrict__ hi, unsigned short* __restrict__ lo) {
-  __shared__ float tile[32][33];
-  const long tr = blockIdx.x, tk = blockIdx.y, b = blockIdx.z;
+// Operand order of the source: along rows, along k with unit stride, any.
+enum { PK_R = 0, PK_K1 = 1, PK_ANY = 2 };
+
+// Tile of TR (64 or 32) rows x 64 k per block, every load before the first
+// use (elements past the operand re-read one inside it and become zeros).  A
+// row of the tile is one whole 128-byte line of hi and of lo, written four
+// bytes a lane: with 32 x 32 tiles two blocks, on two XCDs, shared every line.
+// PK_R transposes through LDS.  Bound by HBM: o=32 v=256, 22 operands of a
+// vector function, 3.1 ms before, 2.7 now (12 bytes an element, 3.7 TB/s).
+template <int MODE, bool K2, int TR>
+__global__ __launch_bounds__(256) void k_pack_bf16x2(PackDesc p, unsigned short* __restrict__ hi,
+                                                     unsigned short* __restrict__ lo) {
+  constexpr int NE = TR / 8;  // pairs per thread
+  __shared__ float tile[MODE == PK_R ? 64 : 1][TR + 1];
+  const long r0 = (long)blockIdx.x * TR, k0 = (long)blockIdx.y * 64, b = blockIdx.z;
   const double* src = p.src + b * p.s_b;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  if (RFAST_) {
+  const int t = threadIdx.x, kp = 2 * (t % 32);
+  const bool whole = r0 + TR <= p.rows && k0 + 64 <= p.K;
+  float v[NE][2];
+  if (p.rows <= 0 || p.K <= 0) {
 #pragma unroll
-    for (int q = 0; q < 32; q += 8) {
-      const long r = tr * 32 + tx, k = tk * 32 + ty + q;
-      tile[ty + q][tx] = (r < p.rows && k < p.K) ? p.scale * (float)src[r * p.s_r + pk_koff(p, k)] : 0.0f;  // [k][r]
+    for (int i = 0; i < NE; ++i) v[i][0] = v[i][1] = 0.0f;
+  } else if (MODE == PK_R) {
+    float u[2 * NE];
+    const long r = r0 + t % TR, k = k0 + t / TR;
+    const double* s = src + min(r, p.rows - 1) * p.s_r;
+    if (whole && !K2) {
+      const double* q = s + k * p.s_k;
+      const long st = (256 / TR) * p.s_k;
+#pragma unroll
+      for (int i = 0; i < 2 * NE; ++i) {
+        u[i] = (float)*q;
+        q += st;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2 * NE; ++i) u[i] = (float)s[pk_koff<K2>(p, min(k + (256 / TR) * i, p.K - 1))];
+#pragma unroll
+      for (int i = 0; i < 2 * NE; ++i)
+        if (r >= p.rows || k + (256 / TR) * i >= p.K) u[i] = 0.0f;
     }
+#pragma unroll
+    for (int i = 0; i < 2 * NE; ++i) tile[t / TR + (256 / TR) * i][t % TR] = p.scale * u[i];  // [k][r]
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 32; q += 8) {
-      const long r = tr * 32 + ty + q, k = tk * 32 + tx;
-      if (r < p.Rp && k < p.Kp) {
-        const float f = tile[tx][ty + q];
-        const unsigned short h = f2bf(f);
-        const long o = (b * p.Rp + r) * p.Kp + k;
-        hi[o] = h;
-        lo[o] = f2bf(f - bf2f(h));
-      }
+    for (int i = 0; i < NE; ++i) {
+      v[i][0] = tile[kp][t / 32 + 8 * i];
+      v[i][1] = tile[kp + 1][t / 32 + 8 * i];
     }
   } else {
+    const long k = k0 + kp;
 #pragma unroll
-    for (int q = 0; q < 32; q += 8) {
-      const long r = tr * 32 + ty + q, k = tk * 32 + tx;
-      if (r < p.Rp && k < p.Kp) {
-        const float f = (r < p.rows && k < p.K) ? p.scale * (float)src[r * p.s_r + pk_koff(p, k)] : 0.0f;
-        const unsigned short h = f2bf(f);
-        const long o = (b * p.Rp + r) * p.Kp + k;
-        hi[o] = h;
-        lo[o] = f2bf(f - bf2f(h));
+    for (int i = 0; i < NE; ++i) {
+      const double* s = src + min(r0 + t / 32 + 8 * i, p.rows - 1) * p.s_r;
+      if (MODE == PK_K1 && whole) {
+        typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+        const d2u x = *reinterpret_cast<const d2u*>(s + k);
+        v[i][0] = p.scale * (float)x[0];
+        v[i][1] = p.scale * (float)x[1];
+      } else {
+        v[i][0] = p.scale * (float)s[pk_koff<K2>(p, min(k, p.K - 1))];
+        v[i][1] = p.scale * (float)s[pk_koff<K2>(p, min(k + 1, p.K - 1))];
       }
     }
+    if (!whole) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) {
+        const bool in = r0 + t / 32 + 8 * i < p.rows;
+        if (!in || k >= p.K) v[i][0] = 0.0f;
+        if (!in || k + 1 >= p.K) v[i][1] = 0.0f;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const long r = r0 + t / 32 + 8 * i;
+    if (r >= p.Rp) continue;
+    const long o = (b * p.Rp + r) * p.Kp + k0 + kp;
+    unsigned h, l;
+    split2(v[i][0], v[i][1], h, l);
+    *reinterpret_cast<unsigned*>(hi + o) = h;
+    *reinterpret_cast<unsigned*>(lo + o) = l;
   }
 }
 
@@ -300,14 +359,26 @@ void bf16x3_pack(const double* src, long rows, long K, long s_r, long s_k, long 
   }
   check_span(hi, 0, (long)batch * Rp * Kp - 1, 2, "bf16x3 pack hi");
   check_span(lo, 0, (long)batch * Rp * Kp - 1, 2, "bf16x3 pack lo");
-  const long rt = (Rp + 31) / 32, kt = (Kp + 31) / 32;
-  CCGPU_REQUIRE(kt < 65536 && batch < 65536 && rt < (1L << 27), "bf16x3 pack: grid too large");
-  dim3 grid((unsigned)rt, (unsigned)kt, (unsigned)batch);
-  const bool rfast = s_r == 1 && s_k != 1;
-  if (rfast)
-    CCGPU_LAUNCH(k_pack_bf16x2<true>, grid, dim3(32, 8), 0, s, p, hi, lo);
-  else
-    CCGPU_LAUNCH(k_pack_bf16x2<false>, grid, dim3(32, 8), 0, s, p, hi, lo);
+  const long kt = Kp / 64;
+  // 64-row tiles once they give eight blocks per CU
+  const int tr = cdiv(Rp, 64) * kt * batch >= 2048 ? 64 : 32;
+  CCGPU_REQUIRE(Kp % 64 == 0 && kt < 65536 && batch < 65536 && Rp < (1L << 29), "bf16x3 pack: grid too large");
+  const dim3 grid(cdiv(Rp, tr), (unsigned)kt, (unsigned)batch);
+  const bool k2 = Kin > 0 && Kin < K;
+  const int mode = (s_r == 1 && s_k != 1) ? PK_R : (s_k == 1 && !k2 ? PK_K1 : PK_ANY);
+#define CCGPU_PACK(M, Q)                                                                 \
+  if (mode == M && k2 == Q) {                                                            \
+    if (tr == 64)                                                                        \
+      CCGPU_LAUNCH((k_pack_bf16x2<M, Q, 64>), grid, dim3(256), 0, s, p, hi, lo);          \
+    else                                                                                 \
+      CCGPU_LAUNCH((k_pack_bf16x2<M, Q, 32>), grid, dim3(256), 0, s, p, hi, lo);          \
+  }
+  CCGPU_PACK(PK_R, false)
+  CCGPU_PACK(PK_R, true)
+  CCGPU_PACK(PK_K1, false)
+  CCGPU_PACK(PK_ANY, false)
+  CCGPU_PACK(PK_ANY, true)
+#undef CCGPU_PACK
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -434,60 +505,93 @@ namespace ccgpu {
 // S GEMM: hi/lo[s][r][p] (s = 0: V+, 1: V-; p = d(d+1)/2 + c), row length
 // Kp; the K padding p in [npv, Kp) is written as zeros by the first tile
 // pair of each row.
-__global__ void k_ladder_vpm_pack(unsigned short* __restrict__ hi, unsigned short* __restrict__ lo,
-                                  const float* __restrict__ Y, long ldY, int a0, int a1, int v, long Rp, long Kp) {
-  __shared__ float Mcd[32][33];
-  __shared__ float Mdc[32][33];
-  const long r = blockIdx.y;
-  int a = a0;
-  long off = 0;
-  while (a < a1 && off + (v - a) <= r) {
-    off += v - a;
-    ++a;
+//
+// Block: row r = (a,b), 32 columns d and 128 c (c <= d), both orders of Y
+// staged in LDS (16-byte loads where rows of Y are 16-byte aligned, V4); every
+// d is one run of the packed row, written two bf16 (4 bytes) a lane, the odd
+// elements at its ends alone.  Bound by HBM (16 bytes a pair): o=32 v=256
+// 7.2 ms a vector function with 32 x 32 tiles, 2-byte stores and the tiles of a
+// row spread over the XCDs, 4.7 now (3.7 TB/s).
+template <bool V4>
+__global__ __launch_bounds__(256) void k_ladder_vpm_pack(unsigned short* __restrict__ hi,
+                                                         unsigned short* __restrict__ lo, const float* __restrict__ Y,
+                                                         long ldY, int a0, int v, long rows, long Rp, long Kp) {
+  constexpr int CT = 128;
+  __shared__ float Mcd[CT][33], Mdc[32][CT + 1];
+  // the tiles of a row run one after the other on one XCD (block b runs on XCD
+  // b % 8), whose L2 joins their part lines of Y and of the packed row
+  const int nct = (v + CT - 1) / CT, ntile = nct * ((v + 31) / 32), idx = blockIdx.x / 8, tile = idx % ntile;
+  const int c0 = (tile % nct) * CT, d0 = (tile / nct) * 32;
+  const long r = (long)(idx / ntile) * 8 + blockIdx.x % 8;
+  if (r >= rows) return;
+  const int t = threadIdx.x;
+  unsigned short* const row[4] = {hi + r * Kp, lo + r * Kp, hi + (Rp + r) * Kp, lo + (Rp + r) * Kp};
+  if (tile == 0) {  // K padding
+    const long npv = (long)v * (v + 1) / 2;
+    for (long p = npv + t; p < Kp; p += 256)
+      for (int q = 0; q < 4; ++q) row[q][p] = 0;
   }
-  const int b = a + (int)(r - off);
-  const long bx = blockIdx.x;
-  long td = (long)((sqrt(8.0 * (double)bx + 1.0) - 1.0) * 0.5);
-  while (td * (td + 1) / 2 > bx) --td;
-  while ((td + 1) * (td + 2) / 2 <= bx) ++td;
-  const long tc = bx - td * (td + 1) / 2;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const long c0 = tc * 32, d0 = td * 32;
-  const float* Ya = Y + (long)(a - a0) * v * ldY + (long)(b - a0) * v;
+  if (c0 > d0 + 31) return;
+  int a, b;
+  batch_row_decode(r, a0, v, a, b);
+  const float* Ya = Y + (long)(a - a0) * v * ldY + (long)(b - a0) * v;  // M[c][d] = Ya[c*ldY + d]
+  // all loads before the LDS stores, rows and columns clamped into the block
+  // (elements past the triangle or v are staged and not used)
+  const int cm = min(v - 1, d0 + 31);
+  if constexpr (V4) {
+    f4 mcd[4], mdc[4];  // v is a multiple of four here: groups of four columns do not straddle it
+    const int dc = min(d0 + 4 * (t % 8), v - 4), cc = min(c0 + 4 * (t % 32), cm & ~3);
 #pragma unroll
-  for (int k = 0; k < 32; k += 8) {
-    const long c = c0 + ty + k, d = d0 + tx;
-    Mcd[ty + k][tx] = (c < v && d < v) ? Ya[c * ldY + d] : 0.0f;
-    const long dd = d0 + ty + k, cc = c0 + tx;
-    Mdc[ty + k][tx] = (dd < v && cc < v) ? Ya[dd * ldY + cc] : 0.0f;
+    for (int k = 0; k < 4; ++k)
+      mcd[k] = *reinterpret_cast<const f4*>(Ya + (long)min(c0 + t / 8 + 32 * k, cm) * ldY + dc);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      mdc[k] = *reinterpret_cast<const f4*>(Ya + (long)min(d0 + t / 32 + 8 * k, v - 1) * ldY + cc);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) Mcd[t / 8 + 32 * k][4 * (t % 8) + h] = mcd[k][h];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) Mdc[t / 32 + 8 * k][4 * (t % 32) + h] = mdc[k][h];
+  } else {
+    float mcd[16], mdc[16];
+    const int dc = min(d0 + t % 32, v - 1), cc = min(c0 + t % CT, cm);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mcd[k] = Ya[(long)min(c0 + t / 32 + 8 * k, cm) * ldY + dc];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) mdc[k] = Ya[(long)min(d0 + t / CT + 2 * k, v - 1) * ldY + cc];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) Mcd[t / 32 + 8 * k][t % 32] = mcd[k];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) Mdc[t / CT + 2 * k][t % CT] = mdc[k];
   }
   __syncthreads();
-  const long npv = (long)v * (v + 1) / 2;
-  unsigned short* hp = hi + r * Kp;
-  unsigned short* lp = lo + r * Kp;
-  unsigned short* hm = hi + (Rp + r) * Kp;
-  unsigned short* lm = lo + (Rp + r) * Kp;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+#pragma unroll 2
+  for (int k = 0; k < 8; ++k) {
+    const int dl = wave + 4 * k, d = d0 + dl;
+    if (d >= v) break;
+    const long p0 = (long)d * (d + 1) / 2 + c0;
+    const int n = min(CT, d - c0 + 1);  // elements of this run: c0 .. c0 + n - 1
+    const int sh = (int)(p0 & 1);
+    for (int e = 2 * lane - sh; e < n; e += CT) {  // the aligned pair of elements e, e + 1
+      const int e0 = max(e, 0), e1 = min(e + 1, CT - 1);
+      const float x0 = Mcd[e0][dl], x1 = Mcd[e1][dl], y0 = Mdc[dl][e0], y1 = Mdc[dl][e1];
+      unsigned w[4];
+      split2(x0 + y0, x1 + y1, w[0], w[1]);
+      split2(x0 - y0, x1 - y1, w[2], w[3]);
+      if (e >= 0 && e + 1 < n) {
 #pragma unroll
-  for (int k = 0; k < 32; k += 8) {
-    const long c = c0 + tx, d = d0 + ty + k;
-    if (c < v && d < v && c <= d) {
-      const float x = Mcd[tx][ty + k], y = Mdc[ty + k][tx];
-      const long p = d * (d + 1) / 2 + c;
-      const float vp = x + y, vm = x - y;
-      const unsigned short h1 = f2bf(vp), h2 = f2bf(vm);
-      hp[p] = h1;
-      lp[p] = f2bf(vp - bf2f(h1));
-      hm[p] = h2;
-      lm[p] = f2bf(vm - bf2f(h2));
-    }
-  }
-  if (bx == 0) {
-    const int t = ty * 32 + tx;
-    for (long p = npv + t; p < Kp; p += 256) {
-      hp[p] = 0;
-      lp[p] = 0;
-      hm[p] = 0;
-      lm[p] = 0;
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<unsigned*>(row[q] + p0 + e) = w[q];
+      } else if (e >= 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) row[q][p0 + e] = (unsigned short)w[q];
+      } else if (n > 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) row[q][p0] = (unsigned short)(w[q] >> 16);
+      }
     }
   }
 }
@@ -506,9 +610,13 @@ void ladder_vpm_pack(unsigned short* hi, unsigned short* lo, const float* Y, lon
   check_span(lo, 0, 2 * Rp * Kp - 1, sizeof(unsigned short), "ladder_vpm_pack lo");
   check_span(Y, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(float), "ladder_vpm_pack Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm_pack: ldY too small");
-  const long nt = (v + 31) / 32;
-  CCGPU_LAUNCH(k_ladder_vpm_pack, dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)rows), dim3(32, 8), 0, st, hi, lo,
-               Y, ldY, a0, a1, v, Rp, Kp);
+  CCGPU_REQUIRE(v < 32 * 65536, "ladder_vpm_pack: virtual space too large");
+  const dim3 grid(cdiv(v, 128) * cdiv(v, 32) * cdiv(rows, 8) * 8);
+  CCGPU_REQUIRE((double)cdiv(v, 128) * cdiv(v, 32) * rows < 16.0e6, "ladder_vpm_pack: grid too large");
+  if (v % 4 == 0 && ldY % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0)
+    CCGPU_LAUNCH(k_ladder_vpm_pack<true>, grid, dim3(256), 0, st, hi, lo, Y, ldY, a0, v, rows, Rp, Kp);
+  else
+    CCGPU_LAUNCH(k_ladder_vpm_pack<false>, grid, dim3(256), 0, st, hi, lo, Y, ldY, a0, v, rows, Rp, Kp);
   // padding rows of both halves
   const long pad = (Rp - rows) * Kp;
   if (pad > 0) {

@@ -6,6 +6,19 @@
 
 namespace ccgpu {
 
+// Row r of a particle-ladder a-batch from a0: pairs (a,b), b in [a,v), a-major.
+// With n = a - a0 and w = v - a0, the rows of a start at n w - n (n - 1) / 2;
+// the root of that is at most one off.
+__device__ __forceinline__ void batch_row_decode(long r, int a0, int v, int& a, int& b) {
+  const double w2 = 2.0 * (v - a0) + 1.0;
+  long n = (long)(0.5 * (w2 - sqrt(w2 * w2 - 8.0 * (double)r)));
+  const long w = v - a0;
+  while (n > 0 && n * w - n * (n - 1) / 2 > r) --n;
+  while ((n + 1) * w - (n + 1) * n / 2 <= r) ++n;
+  a = a0 + (int)n;
+  b = a + (int)(r - (n * w - n * (n - 1) / 2));
+}
+
 // out[j0][j1][j2][j3] = alpha * in[j0*s0 + j1*s1 + j2*s2 + j3*s3] + beta * out
 // (row-major out of dims n0..n3; beta == 0 never reads out).
 void permute4(double* out, const double* in, const long n[4], const long s[4], double alpha,

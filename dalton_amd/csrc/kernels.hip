@@ -491,46 +491,47 @@ void ladder_tau(double* taup, double* taum, const double* Too, int o, int v, hip
   CCGPU_HIPX(hipGetLastError());
 }
 
-__device__ __forceinline__ void batch_row_decode(long r, int a0, int a1, int v, int& a, int& b) {
-  int aa = a0;
-  long off = 0;
-  while (aa < a1 && off + (v - aa) <= r) {
-    off += v - aa;
-    ++aa;
-  }
-  a = aa;
-  b = aa + (int)(r - off);
-}
-
-__global__ void k_ladder_vpm(double* __restrict__ vp, double* __restrict__ vm,
-                             const double* __restrict__ Y, long ldY, int a0, int a1, int v) {
-  __shared__ double Mcd[32][33];
-  __shared__ double Mdc[32][33];
-  const long r = blockIdx.y;
+// Block: row r = (a,b), 32 columns d and 64 c (c <= d): rows of 64 of M[d][.]
+// and of 32 of M[.][d] staged in LDS, runs of 64 doubles written.  Bound by
+// HBM (32 bytes a pair): o=21 v=170 2.1 ms with 32 x 32 tiles spread over the
+// XCDs, 1.35 now (5.0 TB/s).
+__global__ __launch_bounds__(256) void k_ladder_vpm(double* __restrict__ vp, double* __restrict__ vm,
+                                                    const double* __restrict__ Y, long ldY, int a0, int v,
+                                                    long rows) {
+  __shared__ double Mcd[64][33], Mdc[32][65];
+  // the tiles of a row run one after the other on one XCD (block b runs on XCD
+  // b % 8), whose L2 joins their part lines of Y, V+ and V-
+  const int nct = (v + 63) / 64, ntile = nct * ((v + 31) / 32), idx = blockIdx.x / 8, tile = idx % ntile;
+  const int c0 = (tile % nct) * 64, d0 = (tile / nct) * 32;
+  const long r = (long)(idx / ntile) * 8 + blockIdx.x % 8;
+  if (r >= rows || c0 > d0 + 31) return;
   int a, b;
-  batch_row_decode(r, a0, a1, v, a, b);
-  long tc, td;
-  tri_decode(blockIdx.x, tc, td);  // tile pair tc <= td
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const long c0 = tc * 32, d0 = td * 32;
+  batch_row_decode(r, a0, v, a, b);
+  const int t = threadIdx.x;
   const double* Ya = Y + (long)(a - a0) * v * ldY + (long)(b - a0) * v;  // M[c][d] = Ya[c*ldY + d]
+  // all loads before the LDS stores, indices clamped into the block (elements
+  // past the triangle or v are staged and not used)
+  double mcd[8], mdc[8];
+  const int cm = min(v - 1, d0 + 31);
 #pragma unroll
-  for (int k = 0; k < 32; k += 8) {
-    const long c = c0 + ty + k, d = d0 + tx;
-    Mcd[ty + k][tx] = (c < v && d < v) ? Ya[c * ldY + d] : 0.0;      // Mcd[c_l][d_l] = M[c][d]
-    const long dd = d0 + ty + k, cc = c0 + tx;
-    Mdc[ty + k][tx] = (dd < v && cc < v) ? Ya[dd * ldY + cc] : 0.0;  // Mdc[d_l][c_l] = M[d][c]
-  }
+  for (int k = 0; k < 8; ++k) mcd[k] = Ya[min(c0 + t / 32 + 8 * k, cm) * ldY + min(d0 + t % 32, v - 1)];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) mdc[k] = Ya[min(d0 + t / 64 + 4 * k, v - 1) * ldY + min(c0 + t % 64, cm)];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) Mcd[t / 32 + 8 * k][t % 32] = mcd[k];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) Mdc[t / 64 + 4 * k][t % 64] = mdc[k];
   __syncthreads();
   const long npv = (long)v * (v + 1) / 2;
 #pragma unroll
-  for (int k = 0; k < 32; k += 8) {
-    const long c = c0 + tx, d = d0 + ty + k;
-    if (c < v && d < v && c <= d) {
-      const double x = Mcd[tx][ty + k], y = Mdc[ty + k][tx];
-      const long p = d * (d + 1) / 2 + c;
-      vp[r * npv + p] = x + y;
-      vm[r * npv + p] = x - y;
+  for (int k = 0; k < 8; ++k) {
+    const int dl = t / 64 + 4 * k, cl = t % 64;
+    const long c = c0 + cl, d = d0 + dl;
+    if (d < v && c <= d) {
+      const double x = Mcd[cl][dl], y = Mdc[dl][cl];
+      const long p = r * npv + d * (d + 1) / 2 + c;
+      vp[p] = x + y;
+      vm[p] = x - y;
     }
   }
 }
@@ -545,26 +546,70 @@ void ladder_vpm(double* vp, double* vm, const double* Y, long ldY, int a0, int a
   check_span(vm, 0, rows * npv_ - 1, sizeof(double), "ladder_vpm vm");
   check_span(Y, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(double), "ladder_vpm Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm: ldY too small");
-  const long nt = (v + 31) / 32;
-  CCGPU_LAUNCH(k_ladder_vpm, dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)rows), dim3(32, 8), 0,
-                     st, vp, vm, Y, ldY, a0, a1, v);
+  CCGPU_REQUIRE(v < 32 * 65536, "ladder_vpm: virtual space too large");
+  const double nblk = (double)cdiv(v, 64) * cdiv(v, 32) * rows;
+  CCGPU_REQUIRE(nblk < 16.0e6, "ladder_vpm: grid too large");
+  CCGPU_LAUNCH(k_ladder_vpm, dim3(cdiv(v, 64) * cdiv(v, 32) * cdiv(rows, 8) * 8), dim3(256), 0, st, vp, vm, Y, ldY, a0,
+               v, rows);
   CCGPU_HIPX(hipGetLastError());
 }
 
-__global__ void k_ladder_scatter(double* __restrict__ om2, const double* __restrict__ sp,
-                                 const double* __restrict__ sm, int a0, int a1, int o, int v) {
-  const long r = blockIdx.y;
-  int a, b;
-  batch_row_decode(r, a0, a1, v, a, b);
-  const long npo = (long)o * (o + 1) / 2, nov = (long)o * v;
-  for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < npo; q += (long)gridDim.x * blockDim.x) {
-    long i, j;
-    tri_decode(q, i, j);
-    const double P = sp[r * npo + q], M = sm[r * npo + q];
-    om2[(i * v + a) * nov + j * v + b] += P + M;
-    if (i != j) om2[(j * v + a) * nov + i * v + b] += P - M;
-    if (a != b) om2[(i * v + b) * nov + j * v + a] += P - M;
-    if (i != j && a != b) om2[(j * v + b) * nov + i * v + a] += P + M;
+// Block: 16 a x 16 b (b >= a) x 16 occupied pairs through LDS, so that S is
+// read along pairs (128 bytes) and Om2 updated along b, then along a (128
+// bytes each).  One thread per element with 8-byte updates o*v apart took
+// 2.2 ms a vector function at o=32 v=256, this 0.5.
+__global__ __launch_bounds__(256) void k_ladder_scatter(double* __restrict__ om2, const double* __restrict__ sp,
+                                                        const double* __restrict__ sm, int a0, int a1, int o, int v,
+                                                        int nq, int ntb) {
+  __shared__ double xs[16][16][17], xd[16][16][17];  // [pair][a][b]: S+ + S-, S+ - S-
+  const long bx = blockIdx.x;
+  const int tq = (int)(bx % nq), tb = (int)(bx / nq % ntb), ta = (int)(bx / nq / ntb);
+  if (tb < ta) return;
+  const long npo = (long)o * (o + 1) / 2, nov = (long)o * v, w = v - a0;
+  const int lo = threadIdx.x % 16, hi = threadIdx.x / 16;
+  {
+    const long q = tq * 16 + lo;
+    const int b = a0 + tb * 16 + hi;
+#pragma unroll 4
+    for (int al = 0; al < 16; ++al) {
+      const int a = a0 + ta * 16 + al;
+      if (q < npo && a < a1 && b < v && b >= a) {
+        const long n = a - a0, r = n * w - n * (n - 1) / 2 + (b - a);
+        const double P = sp[r * npo + q], M = sm[r * npo + q];
+        xs[lo][al][hi] = P + M;
+        xd[lo][al][hi] = P - M;
+      }
+    }
+  }
+  __syncthreads();
+  // along b: lo = b, hi = a; then along a: lo = a, hi = b
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+    const int al = side == 0 ? hi : lo, bl = side == 0 ? lo : hi;
+    const int a = a0 + ta * 16 + al, b = a0 + tb * 16 + bl;
+    if (a >= a1 || b >= v || b < a || (side == 1 && a == b)) continue;
+    const int x = side == 0 ? a : b, y = side == 0 ? b : a;
+#pragma unroll
+    for (int q0 = 0; q0 < 16; q0 += 4) {
+      double* p[8];
+      double u[8];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const long q = tq * 16 + q0 + k;
+        long i = 0, j = 0;
+        if (q < npo) tri_decode(q, i, j);
+        p[2 * k] = q < npo ? om2 + (i * v + x) * nov + j * v + y : nullptr;
+        p[2 * k + 1] = q < npo && i != j ? om2 + (j * v + x) * nov + i * v + y : nullptr;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) u[k] = p[k] ? *p[k] : 0.0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        // (i,j) from S+ + S- on the b side and S+ - S- on the a side; (j,i) the other way round
+        const bool sum = (k % 2 == 0) == (side == 0);
+        if (p[k]) *p[k] = u[k] + (sum ? xs : xd)[q0 + k / 2][al][bl];
+      }
+    }
   }
 }
 
@@ -573,13 +618,14 @@ void ladder_scatter(double* om2, const double* sp, const double* sm, int a0, int
   long rows = 0;
   for (int a = a0; a < a1; ++a) rows += v - a;
   const long npo = (long)o * (o + 1) / 2;
-  const unsigned nbx = (unsigned)std::min<long>(64, (npo + 255) / 256);
   CCGPU_REQUIRE(rows < 65536, "ladder_scatter: batch too large");
   check_span(om2, 0, (long)o * v * o * v - 1, sizeof(double), "ladder_scatter om2");
   check_span(sp, 0, rows * npo - 1, sizeof(double), "ladder_scatter sp");
   check_span(sm, 0, rows * npo - 1, sizeof(double), "ladder_scatter sm");
-  CCGPU_LAUNCH(k_ladder_scatter, dim3(nbx, (unsigned)rows), dim3(256), 0, st, om2, sp, sm, a0,
-                     a1, o, v);
+  const long nq = cdiv(npo, 16), ntb = cdiv(v - a0, 16), nta = cdiv(a1 - a0, 16);
+  CCGPU_REQUIRE(nq * ntb * nta < (1L << 24), "ladder_scatter: too many tiles");
+  CCGPU_LAUNCH(k_ladder_scatter, dim3((unsigned)(nq * ntb * nta)), dim3(256), 0, st, om2, sp, sm, a0, a1, o, v, (int)nq,
+               (int)ntb);
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -696,7 +742,7 @@ __global__ void k_ladder_gather(double* __restrict__ spb, double* __restrict__ s
                                 int a0, int a1, int o, int v) {
   const long r = blockIdx.y;
   int a, b;
-  batch_row_decode(r, a0, a1, v, a, b);
+  batch_row_decode(r, a0, v, a, b);
   const long npo = (long)o * (o + 1) / 2, nov = (long)o * v;
   for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < npo; q += (long)gridDim.x * blockDim.x) {
     long i, j;
@@ -726,14 +772,17 @@ void ladder_gather(double* spb, double* smb, const double* L, int a0, int a1, in
 // one block per (row r = (a,b), tile pair tc <= td); each Ybar element with
 // b >= a is written by exactly one thread (from p = (min, max) of its c, d)
 __global__ void k_ladder_vpm_adj(double* __restrict__ Yb, long ldY, const double* __restrict__ vpb,
-                                 const double* __restrict__ vmb, int a0, int a1, int v) {
+                                 const double* __restrict__ vmb, int a0, int v, long rows) {
   __shared__ double Pp[32][33];
   __shared__ double Pm[32][33];
-  const long r = blockIdx.y;
+  // the tiles of a row on one XCD, one after the other, as in k_ladder_vpm
+  const long nt = (v + 31) / 32, ntp = nt * (nt + 1) / 2, idx = blockIdx.x / 8;
+  const long r = idx / ntp * 8 + blockIdx.x % 8;
+  if (r >= rows) return;
   int a, b;
-  batch_row_decode(r, a0, a1, v, a, b);
+  batch_row_decode(r, a0, v, a, b);
   long tc, td;
-  tri_decode(blockIdx.x, tc, td);
+  tri_decode(idx % ntp, tc, td);
   const int tx = threadIdx.x, ty = threadIdx.y;
   const long c0 = tc * 32, d0 = td * 32;
   const long npv = (long)v * (v + 1) / 2;
@@ -783,8 +832,9 @@ void ladder_vpm_adj(double* Yb, long ldY, const double* vpb, const double* vmb, 
   check_span(Yb, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(double), "ladder_vpm_adj Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm_adj: ldY too small");
   const long nt = (v + 31) / 32;
-  CCGPU_LAUNCH(k_ladder_vpm_adj, dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)rows), dim3(32, 8), 0, st, Yb, ldY,
-               vpb, vmb, a0, a1, v);
+  CCGPU_REQUIRE(nt * (nt + 1) / 2 * rows < (1L << 26), "ladder_vpm_adj: grid too large");
+  CCGPU_LAUNCH(k_ladder_vpm_adj, dim3((unsigned)(nt * (nt + 1) / 2 * cdiv(rows, 8) * 8)), dim3(32, 8), 0, st, Yb, ldY, vpb,
+               vmb, a0, v, rows);
   CCGPU_HIPX(hipGetLastError());
 }
 

@@ -1,14 +1,15 @@
-"""Particle ladder and its adjoint where one a-batch is formed in several
-a-strips (v = 90: three strips, the adjoint two; v odd so that strips and the
-K starts of the adjoint fall off every tile and K-step boundary): residual
-and left transformation against the oracle."""
+"""Particle ladder and its adjoint at the edges of its tiles (32 and 128 virtual
+orbitals, rows of four) and where one a-batch is formed in several a-strips
+(v = 90 and 91: three strips, the adjoint two, off every tile and K-step
+boundary): residual and left transformation against the oracle."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("o,v,naux", [(2, 90, 300), (3, 91, 290)])
+@pytest.mark.parametrize("o,v,naux", [(1, 31, 40), (2, 32, 40), (5, 33, 40), (6, 36, 40), (2, 90, 300), (3, 91, 290),
+                                      (1, 128, 60), (1, 129, 60)])
 def test_strips_match_oracle(o, v, naux):
     import dalton_amd as d
     from dalton_amd.synthetic import make_system
