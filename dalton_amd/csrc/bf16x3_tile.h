@@ -199,6 +199,142 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
 
 }  // namespace bf3
 
+// One 64 x 64 output tile run by four waves of 32 x 32 (2 x 2 MFMA tiles), K
+// step 32, for products with too few larger tiles to fill the chip: a quarter
+// of the 128 tile's work per block, three blocks per CU.  The operands reach
+// LDS with global_load_lds_dwordx4 into three slots (48 KiB): the loads of
+// step g + 2 are issued in step g, so each has two steps to land, and a step
+// has one barrier.  Wave w loads array w (hi, lo of A, then of B).  LDS layout,
+// swizzle and accumulation order are those of the 256 tile below: results
+// are bit-identical.  Bound by LDS bandwidth (48 KiB read and written per 48
+// MFMAs of a block).  A 1521^3 product (o=13 v=117, 144 tiles of 128 for 256
+// CUs): 93 us on the 128 tile, 60 on this.
+namespace bf3s {
+
+constexpr int DT = 64, DTK = 32;
+struct __attribute__((aligned(16))) Smem {
+  unsigned short s[3][4][DT * DTK];
+};
+
+template <typename OutT>
+__device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, Smem& S) {
+  typedef __attribute__((address_space(3))) void lds_void;
+  typedef const __attribute__((address_space(1))) void glb_void;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lr = lane & 15, kc = lane >> 4, lrow = lane >> 2, lslot = lane & 3;
+  constexpr int SARR = DT * DTK, SSLOT = 4 * SARR;
+  f4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+  const int sw = 8 * (kc ^ ((lr >> 1) & 3));
+  const int offA = (wm * 32 + lr) * DTK + sw, offB = (wn * 32 + lr) * DTK + sw;
+  unsigned short* const base = &S.s[0][0][0];
+  // load cursor: the term's panel of this wave's array, and this lane's row
+  const unsigned short* src = nullptr;
+  long rstep = 0;  // elements between the 16-row groups of the panel
+  auto point = [&](int tl) {
+    const BTerm& T = p.t[tl];
+    const unsigned short* q = wave == 0 ? T.Ah : (wave == 1 ? T.Al : (wave == 2 ? T.Bh : T.Bl));
+    const long bs = wave < 2 ? T.a_bs : T.b_bs, r0 = wave < 2 ? m0 : n0;
+    rstep = 16 * T.Kp;
+    src = q + z * bs + (r0 + lrow) * T.Kp + 8 * (lslot ^ ((lrow >> 1) & 3));
+  };
+  long total = 0;
+  for (int tl = 0; tl < p.nterm; ++tl) total += p.t[tl].Kp / DTK;
+  int lt = 0;
+  while (lt < p.nterm && p.t[lt].Kp < DTK) ++lt;
+  long ls = 0, lsteps = lt < p.nterm ? p.t[lt].Kp / DTK : 0;
+  // past the last step the cursor stays put (loads in bounds, never used)
+  auto advance = [&]() {
+    if (ls + 1 < lsteps) {
+      ++ls;
+      src += DTK;
+      return;
+    }
+    int nt = lt + 1;
+    while (nt < p.nterm && p.t[nt].Kp < DTK) ++nt;
+    if (nt < p.nterm) {
+      lt = nt;
+      ls = 0;
+      lsteps = p.t[lt].Kp / DTK;
+      point(lt);
+    }
+  };
+  auto issue = [&](int slot) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      __builtin_amdgcn_global_load_lds((glb_void*)(src + q * rstep),
+                                       (lds_void*)(base + slot * SSLOT + wave * SARR + q * 16 * DTK), 16, 0, 0);
+  };
+  if (total > 0) {
+    point(lt);
+    issue(0);
+    advance();
+    issue(1);
+    advance();
+    int cur = 0;
+    for (long g = 0; g < total; ++g) {
+      __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): this step's loads have landed, the next step's may be in flight
+      __syncthreads();                     // for every wave; and no wave reads the slot loaded next
+      const unsigned short* s = base + cur * SSLOT;
+      issue(cur == 0 ? 2 : cur - 1);
+      advance();
+      bf16x8 ah[2], al[2], bh[2], bl[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        al[u] = *reinterpret_cast<const bf16x8*>(s + SARR + offA + u * 16 * DTK);
+        bh[u] = *reinterpret_cast<const bf16x8*>(s + 2 * SARR + offB + u * 16 * DTK);
+        ah[u] = *reinterpret_cast<const bf16x8*>(s + offA + u * 16 * DTK);
+        bl[u] = *reinterpret_cast<const bf16x8*>(s + 3 * SARR + offB + u * 16 * DTK);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+      cur = cur == 2 ? 0 : cur + 1;
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the loads past the last step
+  }
+  OutT* C = static_cast<OutT*>(p.C) + z * p.c_b;
+  const long M = p.M, N = p.N, c_m = p.c_m, c_n = p.c_n;
+  const double alpha = p.alpha, beta = p.beta;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    OutT cv[2][4] = {};
+    if (beta != 0.0) {  // uniform; indices clamped into C, so the loads need no per-element branch
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          cv[j][r] = C[min(m0 + wm * 32 + i * 16 + kc * 4 + r, M - 1) * c_m + min(n0 + wn * 32 + j * 16 + lr, N - 1) * c_n];
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long m = m0 + wm * 32 + i * 16 + kc * 4 + r, n = n0 + wn * 32 + j * 16 + lr;
+        if (m < M && n < N) {
+          double v = alpha * (double)acc[i][j][r];
+          if (beta != 0.0) v += beta * (double)cv[j][r];
+          C[m * c_m + n * c_n] = static_cast<OutT>(v);
+        }
+      }
+  }
+}
+
+}  // namespace bf3s
+
 // One 256 x 256 output tile of the BF16x3 multi-term product run by eight
 // waves (512 threads, two per SIMD), each a 128 x 64 sub-tile of 8 x 4 MFMA
 // tiles, K step 32, shared by the GEMM launches and the persistent (T)

@@ -186,6 +186,15 @@ __global__ __launch_bounds__(512, 1) void k_gemm_bf16x3_w8(BMulti p) {
   bf3w8::tile<OutT>(p, tm * DT, tn * DT, blockIdx.z, S);
 }
 
+// Small-tile kernel: 64x64 tiles of bf3s::tile.
+template <typename OutT>
+__global__ __launch_bounds__(256, 3) void k_gemm_bf16x3_s(BMulti p) {
+  __shared__ bf3s::Smem S;
+  long tm, tn;
+  tile_of3(blockIdx.x, (p.M + bf3s::DT - 1) / bf3s::DT, (p.N + bf3s::DT - 1) / bf3s::DT, tm, tn, p.gm);
+  bf3s::tile<OutT>(p, tm * bf3s::DT, tn * bf3s::DT, blockIdx.z, S);
+}
+
 // Block-tile kernel: 1 (default) the eight-wave 256x256 direct-to-LDS
 // kernel, 0 the four-wave 128x128 one (CCGPU_BF16X3_VARIANT=0).  At o=64
 // v=512 the 256x256 kernel runs the mixed CCSD iteration in 2.05 s against
@@ -208,10 +217,11 @@ int group_m() {
 }
 
 // Block-tile kernels of a product: the four-wave 128x128 tile (two blocks
-// per CU) or the eight-wave 256x256 one (one block per CU; operands padded to
-// 256 rows, which bf16x3_rpad gives).  Both accumulate every output element
-// in the same order, so the choice never changes a result bit.
-enum BKern { kT128 = 0, kT256 = 1 };
+// per CU), the eight-wave 256x256 one (one block per CU; operands padded to
+// 256 rows, which bf16x3_rpad gives) or the four-wave 64x64 one (three blocks
+// per CU).  All accumulate every output element in the same order, so the
+// choice never changes a result bit.
+enum BKern { kT128 = 0, kT256 = 1, kT64 = 2 };
 
 template <typename OutT>
 void launch_kernel(int kern, const BMulti& p, int batch, hipStream_t s) {
@@ -219,6 +229,10 @@ void launch_kernel(int kern, const BMulti& p, int batch, hipStream_t s) {
     const long ntiles = (p.Mp / DT) * (p.Np / DT);
     CCGPU_REQUIRE(ntiles < (1L << 23), "bf16x3 gemm: grid too large");
     CCGPU_LAUNCH(k_gemm_bf16x3_w8<OutT>, dim3((unsigned)ntiles, 1, (unsigned)batch), dim3(512), 0, s, p);
+  } else if (kern == kT64) {
+    const long ntiles = (long)cdiv(p.M, bf3s::DT) * cdiv(p.N, bf3s::DT);
+    CCGPU_REQUIRE(ntiles < (1L << 23), "bf16x3 gemm: grid too large");
+    CCGPU_LAUNCH(k_gemm_bf16x3_s<OutT>, dim3((unsigned)ntiles, 1, (unsigned)batch), dim3(256), 0, s, p);
   } else {
     const long ntiles = (long)cdiv(p.M, TM) * cdiv(p.N, TN);
     CCGPU_REQUIRE(ntiles < (1L << 23), "bf16x3 gemm: grid too large");
@@ -269,7 +283,11 @@ struct NoTune {
   ~NoTune() { --t_no_tune; }
 };
 
-// Times both tiles on the product itself: an overwriting product (beta = 0)
+// Products of fewer 128x128 tiles than this (two per CU) may take the 64x64 one.
+constexpr long kSmallTiles = 1024;
+long tiles128(const BMulti& p, int batch) { return (long)cdiv(p.M, TM) * cdiv(p.N, TN) * batch; }
+
+// Times the tiles on the product itself: an overwriting product (beta = 0)
 // runs as given, since the real launch that follows rewrites the same
 // values; an accumulating one runs with alpha = 0 and beta = 1, which leaves
 // C as it was (up to the sign of exact zeros).
@@ -283,18 +301,26 @@ int tune(const BMulti& p, int batch, hipStream_t s) {
   hipEvent_t e0, e1;
   CCGPU_HIP(hipEventCreate(&e0));
   CCGPU_HIP(hipEventCreate(&e1));
-  float ms[2] = {0.f, 0.f};
-  for (int k = kT128; k <= kT256; ++k) {
+  float best = 0.f;
+  int kern = -1;
+  for (int k : {kT128, kT256, kT64}) {
+    if (k == kT256 && (p.Mp % DT != 0 || p.Np % DT != 0)) continue;
+    if (k == kT64 && tiles128(p, batch) >= kSmallTiles) continue;
+    float ms = 0.f;
     launch_kernel<OutT>(k, q, batch, s);  // warm-up
     CCGPU_HIP(hipEventRecord(e0, s));
     launch_kernel<OutT>(k, q, batch, s);
     CCGPU_HIP(hipEventRecord(e1, s));
     CCGPU_HIP(hipEventSynchronize(e1));
-    CCGPU_HIP(hipEventElapsedTime(&ms[k], e0, e1));
+    CCGPU_HIP(hipEventElapsedTime(&ms, e0, e1));
+    if (kern < 0 || ms < best) {
+      best = ms;
+      kern = k;
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  return ms[kT256] <= ms[kT128] ? kT256 : kT128;
+  return kern;
 }
 
 template <typename OutT>
@@ -322,7 +348,8 @@ void launch_multi(BMulti p, int batch, hipStream_t s) {
         tu.best[key] = kern;
         ++tu.timed;
       } else {
-        kern = bf16x3_large_tile(p.M, p.N, batch) ? kT256 : kT128;
+        // without a measurement: 64x64 tiles below one 128x128 tile per CU
+        kern = bf16x3_large_tile(p.M, p.N, batch) ? kT256 : (tiles128(p, batch) < 256 ? kT64 : kT128);
       }
     }
   }
