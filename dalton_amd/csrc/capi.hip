@@ -99,8 +99,7 @@ int ccgpu_df_factor_ao(int nbas, int nmo, const double* cmo, const double* eri_a
                   "ccgpu_df_factor_ao: null argument or no vector room");
     SideStream ss;
     bool conv = false;
-    const std::vector<double> f = ccgpu::df_factor_ao(nbas, nmo, cmo, eri_ao, thr, maxvec, naux, &conv, ss.s);
-    if (B != nullptr && !dry) std::memcpy(B, f.data(), f.size() * sizeof(double));
+    ccgpu::df_factor_ao(nbas, nmo, cmo, eri_ao, thr, maxvec, naux, &conv, [&](size_t) { return B; }, ss.s);
     if (!conv) throw ccgpu::Error(4, "ccgpu_df_factor_ao: threshold not reached within maxvec vectors");
   });
 }
@@ -113,9 +112,8 @@ int ccgpu_df_factor_ao_cols(int nbas, int nmo, const double* cmo, const double* 
                   "ccgpu_df_factor_ao_cols: null argument or no vector room");
     SideStream ss;
     bool conv = false;
-    const std::vector<double> f =
-        ccgpu::df_factor_ao_cols(nbas, nmo, cmo, diag, columns, user, thr, maxvec, naux, &conv, ss.s);
-    if (B != nullptr && !dry) std::memcpy(B, f.data(), f.size() * sizeof(double));
+    ccgpu::df_factor_ao_cols(nbas, nmo, cmo, diag, columns, user, thr, maxvec, naux, &conv,
+                             [&](size_t) { return B; }, ss.s);
     if (!conv && !dry) throw ccgpu::Error(4, "ccgpu_df_factor_ao_cols: threshold not reached within maxvec vectors");
   });
 }
@@ -132,7 +130,12 @@ int ccgpu_init_ao(int nocc, int nvir, int nbas, const double* eps, const double*
     {
       SideStream ss;
       bool conv = false;
-      f = ccgpu::df_factor_ao(nbas, nocc + nvir, cmo, eri_ao, thr, 0, naux, &conv, ss.s);
+      ccgpu::df_factor_ao(nbas, nocc + nvir, cmo, eri_ao, thr, 0, naux, &conv,
+                          [&](size_t n) {
+                            f.resize(n);
+                            return f.data();
+                          },
+                          ss.s);
     }
     CCGPU_REQUIRE(*naux > 0 && *naux < (1L << 31), "ccgpu_init_ao: no Cholesky vectors above the threshold");
     auto c = std::make_unique<ccgpu_ctx>();

@@ -20,6 +20,7 @@
 // the final largest diagonal, below the threshold (V is positive semidefinite).
 #include <algorithm>
 #include <cmath>
+#include <functional>
 #include <vector>
 
 #include "common.h"
@@ -122,41 +123,67 @@ __global__ __launch_bounds__(256) void k_argmax_final(const double* __restrict__
 }
 
 // Step j of the panel that starts at vector K0: pivot p = argmax of the
-// remaining diagonal (piv[1], written on the device), then
+// remaining diagonal, then
 //   L[K0 + j][q] = (R[p][q] - sum_{i<j} L[K0+i][p] L[K0+i][q]) / sqrt(d_p),
 //   d[q] -= L[K0 + j][q]^2, d[p] = 0,
 // where R = V minus the vectors of earlier panels.  Stops (st[0] = 1,
 // st[1] = vectors made) once the largest diagonal is below thr.
-// The same pass writes the stage-1 partials of the next pivot search (the
-// updated diagonal) to part; a step after the stop leaves them as they are.
+// Every block reduces the npart stage-1 partials of the last step (pin) to
+// the pivot by itself and writes its own of the updated diagonal to pout, so
+// a vector is one launch; a step after the stop leaves them as they are.
+// Bound by latency: the panel's elements of column p go through LDS and the
+// sum over them reads eight rows at a time.  nbas = 90, 576 steps: 11.4 us
+// and 4.1 us for the pivot before.
 __global__ __launch_bounds__(256) void k_chol_panel_col(double* __restrict__ L, double* __restrict__ d,
-                                                        const double* __restrict__ R, const double* __restrict__ piv,
-                                                        long* __restrict__ st, long M, long K0, int j, double thr,
-                                                        double* __restrict__ part) {
+                                                        const double* __restrict__ R, const double* __restrict__ pin,
+                                                        int npart, long* __restrict__ st, long M, long K0, int j,
+                                                        double thr, double* __restrict__ pout) {
+  __shared__ double cp[64], bestv[4];
+  __shared__ long besti[4];
   if (st[0] != 0) return;
-  const double dp = piv[0];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  double dp = -1.0;
+  long p = M;
+  for (int q = t; q < npart; q += 256) better(dp, p, pin[2 * q], (long)pin[2 * q + 1]);
+  for (int off = 32; off > 0; off >>= 1) {
+    const double ov = __shfl_xor(dp, off, 64);
+    const long oi = __shfl_xor(p, off, 64);
+    better(dp, p, ov, oi);
+  }
+  if (lane == 0) {
+    bestv[wave] = dp;
+    besti[wave] = p;
+  }
+  __syncthreads();
+  dp = bestv[0];
+  p = besti[0];
+  for (int q = 1; q < 4; ++q) better(dp, p, bestv[q], besti[q]);
   if (dp < thr) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (blockIdx.x == 0 && t == 0) {
       st[0] = 1;
       st[1] = K0 + j;
     }
     return;
   }
-  const long p = (long)piv[1];
+  const double* Lp = L + K0 * M;
+  if (t < j) cp[t] = Lp[t * M + p];
+  __syncthreads();
   const double rs = 1.0 / sqrt(dp);
   double bv = -1.0;
   long bi = M;
-  for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < M; q += (long)gridDim.x * blockDim.x) {
+  for (long q = (long)blockIdx.x * 256 + t; q < M; q += (long)gridDim.x * 256) {
     double s = R[p * M + q];
-    for (int i = 0; i < j; ++i) s -= L[(K0 + i) * M + p] * L[(K0 + i) * M + q];
+    const double dq0 = d[q];
+#pragma unroll 8
+    for (int i = 0; i < j; ++i) s -= cp[i] * Lp[i * M + q];
     const double l = s * rs;
     L[(K0 + j) * M + q] = l;
-    const double dq = (q == p) ? 0.0 : d[q] - l * l;
+    const double dq = (q == p) ? 0.0 : dq0 - l * l;
     d[q] = dq;
     better(bv, bi, dq, q);
   }
-  block_best(bv, bi, part);
-  if (blockIdx.x == 0 && threadIdx.x == 0) st[1] = K0 + j + 1;
+  block_best(bv, bi, pout);
+  if (blockIdx.x == 0 && t == 0) st[1] = K0 + j + 1;
 }
 
 // Pivot of one step of a qualified panel: the largest remaining diagonal
@@ -239,11 +266,14 @@ __global__ void k_pairs_to_square(double* __restrict__ S, const double* __restri
 unsigned grid_for(long n) { return (unsigned)std::max<long>(1, std::min<long>(8192, (n + 255) / 256)); }
 
 // B[k][p][q] = sum_{mu,nu} C[mu][p] L_k[mu nu] C[nu][q] for the K pair
-// vectors L (K x M on the device), returned on the host.
-std::vector<double> mo_transform(const double* L, long K, long M, int nbas, int nmo, const double* cmo,
-                                 hipStream_t st) {
-  std::vector<double> B((size_t)K * nmo * nmo);
-  if (K == 0) return B;
+// vectors L (K x M on the device), copied straight to the host array that
+// place(K nmo^2) names (null: not wanted).  At 34 MB a zeroed vector on the
+// way and a copy out of it took longer than the decomposition: 15 of 19.5 ms
+// were the host's at nbas = 90.
+void mo_transform(const double* L, long K, long M, int nbas, int nmo, const double* cmo,
+                  const std::function<double*(size_t)>& place, hipStream_t st) {
+  double* B = place((size_t)K * nmo * nmo);
+  if (K == 0 || B == nullptr) return;
   // AO square per vector, then X = S C and B = C^T X as batched FP64 GEMMs.
   // C[mu][p] = cmo[p * nbas + mu] (the MO coefficients column by column).
   DBuf<double> C((size_t)nbas * nmo), S((size_t)K * nbas * nbas), X((size_t)K * nbas * nmo),
@@ -257,17 +287,16 @@ std::vector<double> mo_transform(const double* L, long K, long M, int nbas, int 
   g(nbas, nmo, nbas, 1.0, S.p, nbas, 1, C.p, 1, nbas, 0.0, X.p, nmo, 1, st, (int)K, nb2, 0, bm);
   // B[k][p][q] = sum_mu C[mu][p] X[k][mu][q]
   g(nmo, nmo, nbas, 1.0, C.p, nbas, 1, X.p, nmo, 1, 0.0, Bd.p, nmo, 1, st, (int)K, 0, bm, mm);
-  CCGPU_HIPX(hipMemcpyAsync(B.data(), Bd.p, Bd.bytes(), hipMemcpyDeviceToHost, st));
+  CCGPU_HIPX(hipMemcpyAsync(B, Bd.p, Bd.bytes(), hipMemcpyDeviceToHost, st));
   CCGPU_HIPX(hipStreamSynchronize(st));
-  return B;
 }
 
 }  // namespace
 
 // MO factor B[k][p][q] = sum_{mu,nu} C[mu][p] L_k[mu nu] C[nu][q] (k < *naux) of the AO
 // integrals; see ccgpu_df_factor_ao.  maxvec <= 0: no limit below the pair count.
-std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const double* eri_ao, double thr, long maxvec,
-                                 long* naux, bool* converged, hipStream_t st) {
+void df_factor_ao(int nbas, int nmo, const double* cmo, const double* eri_ao, double thr, long maxvec, long* naux,
+                  bool* converged, const std::function<double*(size_t)>& place, hipStream_t st) {
   CCGPU_REQUIRE(nbas > 0 && nmo > 0 && nmo <= nbas, "df_factor_ao: bad sizes");
   CCGPU_REQUIRE(thr > 0.0, "df_factor_ao: threshold must be positive");
   const long M = (long)nbas * (nbas + 1) / 2;
@@ -284,10 +313,12 @@ std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const dou
   constexpr int kNb = 64;
   DBuf<long> state(2);
   CCGPU_HIPX(hipMemsetAsync(state.p, 0, state.bytes(), st));
-  // pivot search: stage-1 partials of every block of the column pass, then
-  // one block over them
+  // pivot search: stage-1 partials of every block of the column pass, which
+  // the blocks of the next step reduce while writing the other half
   const unsigned gcol = grid_for(M);
-  DBuf<double> part(2 * (size_t)gcol);
+  DBuf<double> part(4 * (size_t)gcol);
+  double* const half[2] = {part.p, part.p + 2 * (size_t)gcol};
+  long nstep = 0;
   CCGPU_LAUNCH(k_argmax_part, dim3(gcol), dim3(256), 0, st, d.p, M, part.p);
   long K = 0;
   *converged = false;
@@ -295,9 +326,9 @@ std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const dou
     const int nb = (int)std::min<long>(kNb, Kmax - K);
     if (nb > 0) check_span(L.p, 0, (K + nb) * M - 1, sizeof(double), "cholesky L");
     for (int j = 0; j < nb; ++j) {
-      CCGPU_LAUNCH(k_argmax_final, dim3(1), dim3(256), 0, st, part.p, (int)gcol, piv.p);
-      CCGPU_LAUNCH(k_chol_panel_col, dim3(gcol), dim3(256), 0, st, L.p, d.p, V.p, piv.p, state.p, M, K, j, thr,
-                   part.p);
+      CCGPU_LAUNCH(k_chol_panel_col, dim3(gcol), dim3(256), 0, st, L.p, d.p, V.p, half[nstep & 1], (int)gcol, state.p,
+                   M, K, j, thr, half[(nstep + 1) & 1]);
+      ++nstep;
     }
     long h[2] = {0, K + nb};
     CCGPU_HIPX(hipMemcpyAsync(h, state.p, sizeof(h), hipMemcpyDeviceToHost, st));
@@ -326,7 +357,7 @@ std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const dou
   CCGPU_HIPX(hipGetLastError());
   V.release();
   *naux = K;
-  return mo_transform(L.p, K, M, nbas, nmo, cmo, st);
+  mo_transform(L.p, K, M, nbas, nmo, cmo, place, st);
 }
 
 
@@ -338,9 +369,9 @@ std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const dou
 // their columns come from the callback, are corrected for the earlier
 // vectors by one GEMM, and the panel's pivots are chosen among them in
 // decreasing order of the updated diagonal.  Nothing of size M^2 is formed.
-std::vector<double> df_factor_ao_cols(int nbas, int nmo, const double* cmo, const double* diag,
-                                      int (*columns)(void*, int, const long*, double*), void* user, double thr,
-                                      long maxvec, long* naux, bool* converged, hipStream_t st) {
+void df_factor_ao_cols(int nbas, int nmo, const double* cmo, const double* diag,
+                       int (*columns)(void*, int, const long*, double*), void* user, double thr, long maxvec,
+                       long* naux, bool* converged, const std::function<double*(size_t)>& place, hipStream_t st) {
   CCGPU_REQUIRE(nbas > 0 && nmo > 0 && nmo <= nbas, "df_factor_ao_cols: bad sizes");
   CCGPU_REQUIRE(thr > 0.0, "df_factor_ao_cols: threshold must be positive");
   CCGPU_REQUIRE(columns != nullptr && diag != nullptr, "df_factor_ao_cols: null diagonal or column callback");
@@ -416,7 +447,7 @@ std::vector<double> df_factor_ao_cols(int nbas, int nmo, const double* cmo, cons
   }
   CCGPU_HIPX(hipGetLastError());
   *naux = K;
-  return mo_transform(L.p, K, M, nbas, nmo, cmo, st);
+  mo_transform(L.p, K, M, nbas, nmo, cmo, place, st);
 }
 
 }  // namespace ccgpu

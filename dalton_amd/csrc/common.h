@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -205,14 +206,15 @@ void gemm_bf16x3_noalloc(const GemmDesc& d, hipStream_t s);
 double mfma_only_tflops(bool f64);
 
 // MO density-fitting factor of AO integrals by pivoted Cholesky (cholesky.hip):
-// returns naux x nmo x nmo values; maxvec <= 0 allows one vector per AO pair.
-std::vector<double> df_factor_ao(int nbas, int nmo, const double* cmo, const double* eri_ao, double thr, long maxvec,
-                                 long* naux, bool* converged, hipStream_t st);
+// naux x nmo x nmo values into the host array that place(count) returns (null:
+// not wanted); maxvec <= 0 allows one vector per AO pair.
+void df_factor_ao(int nbas, int nmo, const double* cmo, const double* eri_ao, double thr, long maxvec, long* naux,
+                  bool* converged, const std::function<double*(size_t)>& place, hipStream_t st);
 // The same factor from the pair diagonal and integral columns supplied by a
 // callback (qualified panels of at most 64 columns; no M x M array).
-std::vector<double> df_factor_ao_cols(int nbas, int nmo, const double* cmo, const double* diag,
-                                      int (*columns)(void*, int, const long*, double*), void* user, double thr,
-                                      long maxvec, long* naux, bool* converged, hipStream_t st);
+void df_factor_ao_cols(int nbas, int nmo, const double* cmo, const double* diag,
+                       int (*columns)(void*, int, const long*, double*), void* user, double thr, long maxvec,
+                       long* naux, bool* converged, const std::function<double*(size_t)>& place, hipStream_t st);
 
 // Dalton's CC response-vector files (rspfile.hip): the name CC_RWPRE gives
 // list/symmetry/index; writing and reading the records of CC_WVRSP for a

@@ -562,26 +562,36 @@ __global__ __launch_bounds__(256) void k_ladder_scatter(double* __restrict__ om2
                                                         const double* __restrict__ sm, int a0, int a1, int o, int v,
                                                         int nq, int ntb) {
   __shared__ double xs[16][16][17], xd[16][16][17];  // [pair][a][b]: S+ + S-, S+ - S-
+  __shared__ int pi[16], pj[16];
   const long bx = blockIdx.x;
   const int tq = (int)(bx % nq), tb = (int)(bx / nq % ntb), ta = (int)(bx / nq / ntb);
   if (tb < ta) return;
   const long npo = (long)o * (o + 1) / 2, nov = (long)o * v, w = v - a0;
   const int lo = threadIdx.x % 16, hi = threadIdx.x / 16;
   {
-    const long q = tq * 16 + lo;
-    const int b = a0 + tb * 16 + hi;
-#pragma unroll 4
+    const long q = min(tq * 16L + lo, npo - 1);
+    const int b = a0 + tb * 16 + hi, nb = min(b, v - 1) - a0;
+    double P[16], M[16];  // all loads first, indices clamped into S (elements outside are not used)
+#pragma unroll
     for (int al = 0; al < 16; ++al) {
-      const int a = a0 + ta * 16 + al;
-      if (q < npo && a < a1 && b < v && b >= a) {
-        const long n = a - a0, r = n * w - n * (n - 1) / 2 + (b - a);
-        const double P = sp[r * npo + q], M = sm[r * npo + q];
-        xs[lo][al][hi] = P + M;
-        xd[lo][al][hi] = P - M;
-      }
+      const long n = min(min(ta * 16 + al, a1 - 1 - a0), nb), r = n * w - n * (n - 1) / 2 + (nb - n);
+      P[al] = sp[r * npo + q];
+      M[al] = sm[r * npo + q];
+    }
+    if (hi == 0) {
+      long i, j;
+      tri_decode(q, i, j);
+      pi[lo] = (int)i;
+      pj[lo] = (int)j;
+    }
+#pragma unroll
+    for (int al = 0; al < 16; ++al) {
+      xs[lo][al][hi] = P[al] + M[al];
+      xd[lo][al][hi] = P[al] - M[al];
     }
   }
   __syncthreads();
+  const int nqt = (int)min(16L, npo - tq * 16L);
   // along b: lo = b, hi = a; then along a: lo = a, hi = b
 #pragma unroll
   for (int side = 0; side < 2; ++side) {
@@ -590,24 +600,23 @@ __global__ __launch_bounds__(256) void k_ladder_scatter(double* __restrict__ om2
     if (a >= a1 || b >= v || b < a || (side == 1 && a == b)) continue;
     const int x = side == 0 ? a : b, y = side == 0 ? b : a;
 #pragma unroll
-    for (int q0 = 0; q0 < 16; q0 += 4) {
-      double* p[8];
-      double u[8];
+    for (int q0 = 0; q0 < 16; q0 += 8) {
+      if (q0 >= nqt) break;
+      double u[16];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const long q = tq * 16 + q0 + k;
-        long i = 0, j = 0;
-        if (q < npo) tri_decode(q, i, j);
-        p[2 * k] = q < npo ? om2 + (i * v + x) * nov + j * v + y : nullptr;
-        p[2 * k + 1] = q < npo && i != j ? om2 + (j * v + x) * nov + i * v + y : nullptr;
+      for (int k = 0; k < 8; ++k) {  // (a pair past the list re-reads the last one)
+        const long i = pi[q0 + k], j = pj[q0 + k];
+        u[2 * k] = om2[(i * v + x) * nov + j * v + y];
+        u[2 * k + 1] = om2[(j * v + x) * nov + i * v + y];
       }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) u[k] = p[k] ? *p[k] : 0.0;
-#pragma unroll
       for (int k = 0; k < 8; ++k) {
+        if (q0 + k >= nqt) break;
+        const long i = pi[q0 + k], j = pj[q0 + k];
         // (i,j) from S+ + S- on the b side and S+ - S- on the a side; (j,i) the other way round
-        const bool sum = (k % 2 == 0) == (side == 0);
-        if (p[k]) *p[k] = u[k] + (sum ? xs : xd)[q0 + k / 2][al][bl];
+        const double s = xs[q0 + k][al][bl], d = xd[q0 + k][al][bl];
+        om2[(i * v + x) * nov + j * v + y] = u[2 * k] + (side == 0 ? s : d);
+        if (i != j) om2[(j * v + x) * nov + i * v + y] = u[2 * k + 1] + (side == 0 ? d : s);
       }
     }
   }
