@@ -10,15 +10,18 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 
 enum { KFAST = 0, RFAST = 1 };  // loader order: k fastest / row (m or n) fastest
 
-// K steps and LDS staging of a T x T block tile: TK = 2048 / T columns of
-// K per step, so that every thread stages eight elements per operand whatever
-// the tile.  An operand loaded k-fastest is stored [row][k] with row stride
-// TK + 2, one loaded row-fastest [k][row] with stride T + 16 (the 32 tile:
-// stride 32, odd k with row bit 4 flipped, so that two blocks fit a CU); the
-// 8-byte fragment reads of a half wave then fall on all 64 banks once.
+// K steps and LDS staging of a T x T block tile: TK columns of K per step, of
+// which every thread stages EPT elements per operand.  Steps of 16 (32 tile:
+// 32) are short enough that a product over K = v of a small molecule is not
+// mostly padding, and leave the registers and LDS for more than two of the
+// small tiles per CU: with steps twice as long, v^3 products at v = 93..170
+// took 1.1-1.4x the time.  An operand loaded k-fastest is stored [row][k] with
+// row stride TK + 2, one loaded row-fastest [k][row] with stride T + 16 (the
+// 32 tile: stride 32, odd k with row bit 4 flipped); the 8-byte fragment
+// reads of a half wave then fall on all 64 banks once.
 template <int T>
 struct Step {
-  static constexpr int TK = 2048 / T, LDK = TK + 2, LDR = T == 32 ? T : T + 16;
+  static constexpr int TK = T == 32 ? 32 : 16, EPT = T * TK / 256, LDK = TK + 2, LDR = T == 32 ? T : T + 16;
 };
 template <int MODE, int T>
 struct Stage;
@@ -52,11 +55,11 @@ __device__ __forceinline__ long koff(const KMap& m, long k) {
   return (long)q * m.s_ko + (long)r * m.s_k;
 }
 
-// This thread's eight elements of one K step of an operand tile whose first
+// This thread's EPT elements of one K step of an operand tile whose first
 // row is at base: k-fastest, column tid % TK of rows tid / TK + (256 / TK) i;
 // row-fastest, row tid % T of columns tid / T + (256 / T) i.  One pointer per
-// operand walks K (two-level K recomputes it per step) and the eight
-// elements are uniform steps from it.  An element past the matrix (EDGE;
+// operand walks K (two-level K recomputes it per step) and the elements
+// are uniform steps from it.  An element past the matrix (EDGE;
 // rmax = last row of the tile inside it) re-reads a row inside it, whose
 // results are never stored; only the last, partial step (TAIL) compares k
 // with kend, re-reads a column inside and takes zeros.
@@ -77,7 +80,7 @@ struct Cursor {
     if (!K2) p += (kbeg + c0) * km.s_k;
   }
   template <bool TAIL>
-  __device__ __forceinline__ void load(double (&v)[8], long k0, long kend) {
+  __device__ __forceinline__ void load(double (&v)[Step<T>::EPT], long k0, long kend) {
     const long k = k0 + c0;
     if (MODE == KFAST) {
       P q = p;
@@ -88,7 +91,7 @@ struct Cursor {
       const long st = NR * s_r;
       int r = r0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < Step<T>::EPT; ++i) {
         v[i] = *q;
         if (EDGE) {
           r += NR;
@@ -99,11 +102,11 @@ struct Cursor {
       }
       if (TAIL && k >= kend) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = 0.0;
+        for (int i = 0; i < Step<T>::EPT; ++i) v[i] = 0.0;
       }
     } else if (K2) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < Step<T>::EPT; ++i) {
         const long ki = k + NR * i;
         const double x = p[koff<true>(km, TAIL ? min(ki, kend - 1) : ki)];
         v[i] = (TAIL && ki >= kend) ? 0.0 : x;
@@ -113,7 +116,7 @@ struct Cursor {
       if (TAIL && k >= kend) q -= (k - (kend - 1)) * km.s_k;
       const long st = NR * km.s_k;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < Step<T>::EPT; ++i) {
         const double x = *q;
         v[i] = (TAIL && k + NR * i >= kend) ? 0.0 : x;
         if (TAIL)
@@ -127,10 +130,10 @@ struct Cursor {
 };
 
 template <int MODE, int T>
-__device__ __forceinline__ void stage8(Stage<MODE, T>& S, const double (&v)[8], int tid) {
+__device__ __forceinline__ void stage_step(Stage<MODE, T>& S, const double (&v)[Step<T>::EPT], int tid) {
   constexpr int TK = Step<T>::TK;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < Step<T>::EPT; ++i) {
     if (MODE == KFAST)
       S.at(tid / TK + (256 / TK) * i, tid % TK) = v[i];
     else

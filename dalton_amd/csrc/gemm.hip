@@ -47,19 +47,20 @@ __device__ __forceinline__ void tile_of(long b, long tiles_m, long tiles_n, long
 
 // Block tile T x T (T = 128, 64 or 32), 2x2 waves of (T/2)x(T/2), each wave
 // (T/32)x(T/32) MFMA 16x16 tiles.  The next step's global loads are in
-// flight while the current step's MFMAs run.  The 128 tile, which is bound
-// by the matrix cores, has one LDS stage (two barriers a step); the smaller
-// tiles, bound by the latency of a step, two stages and one barrier.
+// flight while the current step's MFMAs run; one LDS stage, two barriers a
+// step: a second stage saves a barrier but costs the blocks that hide it
+// (128 tile 61 against 68 TFLOP/s; 64 tile, two blocks a CU instead of four,
+// 1150^3 to 3570^3 products 1.2-1.3x the time).
 template <int AMODE, int BMODE, bool K2, int T>
-__global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int nz, unsigned magic, double* ws) {
+__global__ __launch_bounds__(256, T == 128 ? 2 : (T == 64 ? 4 : 5)) void k_dgemm(GemmDesc d, long kchunk, int nz,
+                                                                               unsigned magic, double* ws) {
   constexpr int TM = T, TN = T, TK = Step<T>::TK;
   constexpr int IW = T / 32;      // MFMA tiles per wave and dimension
-  constexpr int NS = T == 128 ? 1 : 2;
   // both operands [row][k]: a lane takes two consecutive k of a group of
   // eight for two MFMAs in turn, in 16-byte reads
   constexpr bool PAIR = AMODE == KFAST && BMODE == KFAST;
-  __shared__ Stage<AMODE, T> As[NS];
-  __shared__ Stage<BMODE, T> Bs[NS];
+  __shared__ Stage<AMODE, T> As;
+  __shared__ Stage<BMODE, T> Bs;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const long tiles_m = (d.M + TM - 1) / TM, tiles_n = (d.N + TN - 1) / TN;
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int n
     for (int i = 0; i < IW; ++i)
 #pragma unroll
       for (int j = 0; j < IW; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    double ra[8], rb[8];
+    double ra[Step<T>::EPT], rb[Step<T>::EPT];
     Cursor<AMODE, K2, T, E> ca(A, d.a_m, ka, ma, kbeg, tid);
     Cursor<BMODE, K2, T, E> cb(B, d.b_n, kb, nb, kbeg, tid);
     auto load = [&](long k0, auto tail) {
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int n
       ca.template load<TL>(ra, k0, kend);
       cb.template load<TL>(rb, k0, kend);
     };
-    auto mfma8 = [&](int st, int k) {  // k .. k + 7 of the staged step
+    auto mfma8 = [&](int k) {  // k .. k + 7 of the staged step
       d2 pa[IW], pb[IW];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -109,14 +110,14 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int n
           const int ra0 = wm * (T / 2) + t * 16 + lr, rb0 = wn * (T / 2) + t * 16 + lr;
           if constexpr (PAIR) {
             if (h == 0) {
-              pa[t] = *reinterpret_cast<const d2*>(&As[st].at(ra0, k + 2 * lk));
-              pb[t] = *reinterpret_cast<const d2*>(&Bs[st].at(rb0, k + 2 * lk));
+              pa[t] = *reinterpret_cast<const d2*>(&As.at(ra0, k + 2 * lk));
+              pb[t] = *reinterpret_cast<const d2*>(&Bs.at(rb0, k + 2 * lk));
             }
             a[t] = pa[t][h];
             b[t] = pb[t][h];
           } else {
-            a[t] = As[st].at(ra0, k + 4 * h + lk);
-            b[t] = Bs[st].at(rb0, k + 4 * h + lk);
+            a[t] = As.at(ra0, k + 4 * h + lk);
+            b[t] = Bs.at(rb0, k + 4 * h + lk);
           }
         }
 #pragma unroll
@@ -131,34 +132,17 @@ __global__ __launch_bounds__(256, 2) void k_dgemm(GemmDesc d, long kchunk, int n
       load(kbeg, std::false_type{});
     else if (rem > 0)
       load(kbeg, std::true_type{});
-    if constexpr (NS == 2) {
-      if (nstep > 0) {
-        stage8(As[0], ra, tid);
-        stage8(Bs[0], rb, tid);
-      }
-      __syncthreads();
-    }
     for (long s = 0; s < nstep; ++s) {
-      const int st = NS == 2 ? (int)(s & 1) : 0;
-      if constexpr (NS == 1) {
-        __syncthreads();
-        stage8(As[0], ra, tid);
-        stage8(Bs[0], rb, tid);
-        __syncthreads();
-      }
+      __syncthreads();
+      stage_step(As, ra, tid);
+      stage_step(Bs, rb, tid);
+      __syncthreads();
       if (s + 1 < nfull)
         load(kbeg + (s + 1) * TK, std::false_type{});
       else if (s + 1 < nstep)
         load(kbeg + (s + 1) * TK, std::true_type{});
 #pragma unroll
-      for (int k = 0; k < TK; k += 8) mfma8(st, k);
-      if constexpr (NS == 2) {
-        if (s + 1 < nstep) {
-          stage8(As[st ^ 1], ra, tid);
-          stage8(Bs[st ^ 1], rb, tid);
-        }
-        __syncthreads();
-      }
+      for (int k = 0; k < TK; k += 8) mfma8(k);
     }
 
 
@@ -284,26 +268,31 @@ struct F64Cfg {
   int nz = 1;
 };
 
-// Estimated time (microseconds) of block tile T with K in nz chunks.  Two
-// blocks of any tile are resident per CU (256 CUs): a K step takes kOne
-// cycles while one block has a CU to itself and kTwo when two share it, the
-// blocks beyond whole rounds of 512 take a shared round again; a split adds a
-// launch and the pass over the partials, and C bounds the time from below.
-// The step times are measured (o = 5..32, v = 19..256 products of a vector
-// function): the 128 tile runs at 68 TFLOP/s in full rounds, the 64 tile at
-// 52 and the 32 tile at 37, but 64 x 64 and 32 x 32 tiles fill the chip, or
-// leave it sooner, where 128 x 128 ones are few or mostly padding.
+int step_k(int T) { return T == 32 ? Step<32>::TK : Step<64>::TK; }
+
+// Estimated time (microseconds) of block tile T with K in nz chunks.  kRes
+// blocks of the tile are resident per CU (256 CUs); with c of them a K step
+// takes kBase + kPer c cycles, and the blocks beyond whole rounds of 256 kRes
+// take a round of their own.  A two-level K costs kTwoK, a split adds a launch
+// and the pass over the partials, and C bounds the time from below (the
+// shorter of the two adds a little: first loads and last stores are not
+// overlapped).  The constants are measured (1648 runs, the products of a
+// vector function for o = 5..21, v = 19..170; the configuration of least
+// estimate is on average within 1% of the fastest one measured): in full
+// rounds the 128 tile runs at 64 TFLOP/s, the 64 tile at 59 and the 32 tile at
+// 45, but 64 x 64 and 32 x 32 tiles fill the chip, or leave it sooner, where
+// 128 x 128 ones are few or mostly padding.
 double cost_f64(const GemmDesc& d, int T, long nz) {
   const int q = T == 128 ? 0 : (T == 64 ? 1 : 2);
-  constexpr double kOne[3] = {5900.0, 4200.0, 2700.0}, kTwo[3] = {9300.0, 5800.0, 3900.0}, kMhz = 2300.0;
-  const double tiles = (double)cdiv(d.M, T) * cdiv(d.N, T) * d.batch;
-  const double blocks = tiles * nz, steps = (double)cdiv(cdiv(d.K, nz), 2048 / T);
-  const long full = (long)(blocks / 512.0);
-  const double left = blocks - 512.0 * full;
-  const double last = left <= 0.0 ? 0.0 : (full == 0 && left <= 256.0 ? kOne[q] : kTwo[q]);
-  const double us = 3.5 + steps / kMhz * (full * kTwo[q] + last) * (two_level(d) ? 1.15 : 1.0);
-  const double cbytes = 8.0 * d.batch * (double)d.M * d.N * (d.beta != 0.0 ? 2.0 : 1.0);
-  return std::max(us, cbytes / 4.0e6) + (nz > 1 ? 2.5 + 0.02 * nz + (double)nz * d.batch * d.M * d.N * 16.0 / 3.0e6 : 0.0);
+  constexpr double kBase[3] = {2400.0, 1000.0, 700.0}, kPer[3] = {3100.0, 1050.0, 650.0}, kTwoK[3] = {1.05, 1.08, 1.25};
+  constexpr double kMhz = 2300.0;
+  constexpr long kRes[3] = {2, 5, 8};
+  const long blocks = (long)cdiv(d.M, T) * cdiv(d.N, T) * d.batch * nz, steps = cdiv(cdiv(d.K, nz), step_k(T));
+  const long round = 256 * kRes[q], full = blocks / round, left = cdiv(blocks - full * round, 256);
+  const double cycles = full * (kBase[q] + kPer[q] * kRes[q]) + (left > 0 ? kBase[q] + kPer[q] * left : 0.0);
+  const double us = 3.8 + steps * cycles / kMhz * (two_level(d) ? kTwoK[q] : 1.0);
+  const double mn = (double)d.batch * d.M * d.N, cus = 8.0 * mn * (d.beta != 0.0 ? 2.0 : 1.0) / 4.5e6;
+  return std::max(us, cus) + 0.15 * std::min(us, cus) + (nz > 1 ? 2.3 + 0.02 * nz + nz * mn * 16.0 / 3.5e6 : 0.0);
 }
 
 // The configuration of least estimated time, of one tile (only) or of all.
@@ -314,7 +303,7 @@ F64Cfg plan_f64(const GemmDesc& d, int only = 0) {
     if (only && T != only) continue;
     // chunks of at least two K steps; partials of at most 4 GB
     const double room = 4.0e9 / (8.0 * d.batch * (double)d.M * d.N);
-    const long kmax = std::max<long>(1, std::min<long>(d.K / (2 * (2048 / T)), (long)std::min(room, 1e6)));
+    const long kmax = std::max<long>(1, std::min<long>(d.K / (2 * (step_k(T))), (long)std::min(room, 1e6)));
     for (long nz = 1; nz <= std::min<long>({kmax, 256, 65535 / d.batch}); nz = nz < 4 ? nz + 1 : nz + nz / 3) {
       const double t = cost_f64(d, T, nz);
       if (t < bt) {
@@ -385,7 +374,7 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
   int nz = 1;
   double* ws = nullptr;
   if (cfg.nz > 1) {
-    const long tk = 2048 / T;  // chunks are whole K steps
+    const long tk = step_k(T);  // chunks are whole K steps
     const long chunk = cdiv(cdiv(d.K, cfg.nz), tk) * tk;
     nz = (int)cdiv(d.K, chunk);
     if (nz >= 2) {

@@ -112,8 +112,8 @@ __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, lo
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) ra[i] *= al;
-    stage8<AM, T>(SA, ra, tid);
-    stage8<BM, T>(SB, rb, tid);
+    stage_step<AM, T>(SA, ra, tid);
+    stage_step<BM, T>(SB, rb, tid);
     __syncthreads();
     if (k0 + TK < K) load(k0 + TK);
 #pragma unroll
