@@ -4,7 +4,8 @@
 //
 // A cooperative launch of as many blocks as the device holds at once walks
 // the triples of the launch in order.  Per triple q three GEMM passes build
-// W_q (G1: W[a][(b,c)] with beta = 0; G2: batched over a, W[a][b][c] += ...;
+// W_q (G1: W[a][(b,c)] with beta = 0; G2: W[a][b][c] += ..., rows b, batched
+// over a in the mixed passes, columns (a,c) in FP64;
 // G3: W[(a,b)][c] += ...; four of the twelve terms each, one 128 x 128
 // output tile per item) and an energy pass (E, one item per group of
 // canonical 8x8x8 virtual blocks) reads it.  The passes form a software
@@ -44,59 +45,64 @@ namespace ccgpu {
 namespace {
 
 // ------------------------------------------------------------ FP64 tiles
-// One term of a multi-term FP64 product: A(m,k) of batch z at
-// A + m a_m + k a_k + z a_b, B(n,k) at B + n b_n + k b_k + z b_b.
+// One term of a multi-term FP64 product: A(m,k) at A + m a_m + k a_k, B(n,k)
+// at B + n b_n + k b_k.
 struct DTerm {
   const double* A;
   const double* B;
-  long a_m, a_k, a_b;
-  long b_n, b_k, b_b;
+  long a_m, a_k;
+  long b_n, b_k;
   long K;
   double alpha;
   int akf;  // 1: A is read along k and B along n; 0: A along m and B along k
 };
-// C(m,n) of batch z (at C + m c_m + n c_n + z c_b) = sum_t alpha_t A_t B_t^T + beta C
+// C(m,n) (at C + m c_m + (n % nin) + (n / nin) c_no) = sum_t alpha_t A_t B_t^T + beta C
 struct DMulti {
   DTerm t[4];
   int nterm;
   long M, N;
   double beta;
   double* C;
-  long c_m, c_n, c_b;
+  long c_m, c_no;
+  int nin;
 };
 
 namespace dt {
-// Tile 128 x 128, K step 16, 256 threads as 2 x 2 waves of 64 x 64
-// (4 x 4 v_mfma_f64_16x16x4f64 tiles each); operands staged
-// global -> registers -> LDS as in the FP64 GEMM (one pointer per operand
-// walks K, rows past the matrix re-read a row inside it, only a last partial
-// K step compares k with K), the next step's loads issued before the MFMAs.
-constexpr int T = 128, TK = Step<T>::TK, IW = 4;
+// Tile 128 x 128, K step 16, 256 threads; operands staged global -> registers ->
+// LDS as in the FP64 GEMM (one pointer per operand walks K, rows past the
+// matrix re-read a row inside it, only a last partial K step compares k with
+// K), the next step's loads issued before the MFMAs.  The four waves lie side
+// by side along the long dimension (n for X, m for !X): the other one is
+// v, and its 16-row parts past v are left out of the products of all waves
+// alike (2 x 2 waves: only the waves that own them, and the others set the
+// time of a step; o=12 v=101 full list 17.5 against 16.0 ms).  A 64 x 64 tile
+// with four blocks per CU took 16.8 ms.
+constexpr int T = 128, TK = Step<T>::TK;
 struct __attribute__((aligned(16))) Smem {
-  double A[TK * Step<T>::LDR];
-  double B[TK * Step<T>::LDR];
+  static constexpr size_t N = std::max(sizeof(Stage<KFAST, T>), sizeof(Stage<RFAST, T>)) / sizeof(double);
+  double A[N];
+  double B[N];
 };
-static_assert(sizeof(Stage<KFAST, T>) <= sizeof(double) * TK * Step<T>::LDR &&
-                  sizeof(Stage<RFAST, T>) <= sizeof(double) * TK * Step<T>::LDR,
-              "pt: operand stages");
 
 // E: the tile reaches past M or N.
-template <bool AKF, bool E>
-__device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, long n0, long z, d4 (&acc)[IW][IW],
-                                     Smem& S) {
+template <bool X, bool AKF, bool E>
+__device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, long n0,
+                                     d4 (&acc)[X ? T / 16 : T / 64][X ? T / 64 : T / 16], Smem& S) {
   constexpr int AM = AKF ? KFAST : RFAST, BM = AKF ? RFAST : KFAST;
+  constexpr int IM = X ? T / 16 : T / 64, IN = X ? T / 64 : T / 16;
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // thread-index arithmetic stays inside the item (not hoisted into the claim loop)
   const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = X ? 0 : wave * (T / 4), wn = X ? wave * (T / 4) : 0;
+  const int nv = (X ? ma : nb) / 16 + 1;  // 16-row parts inside the matrix
   const long K = t.K;
   const double al = t.alpha;
   using GP = const CCGPU_GLOBAL double*;
-  Cursor<AM, false, T, E, GP> ca(gptr(t.A + z * t.a_b + m0 * t.a_m), t.a_m, KMap{t.a_k, 0, 0u, 0u}, ma, 0, tid);
-  Cursor<BM, false, T, E, GP> cb(gptr(t.B + z * t.b_b + n0 * t.b_n), t.b_n, KMap{t.b_k, 0, 0u, 0u}, nb, 0, tid);
+  Cursor<AM, false, T, E, GP> ca(gptr(t.A + m0 * t.a_m), t.a_m, KMap{t.a_k, 0, 0u, 0u}, ma, 0, tid);
+  Cursor<BM, false, T, E, GP> cb(gptr(t.B + n0 * t.b_n), t.b_n, KMap{t.b_k, 0, 0u, 0u}, nb, 0, tid);
   Stage<AM, T>& SA = *reinterpret_cast<Stage<AM, T>*>(S.A);
   Stage<BM, T>& SB = *reinterpret_cast<Stage<BM, T>*>(S.B);
-  double ra[8], rb[8];
+  double ra[Step<T>::EPT], rb[Step<T>::EPT];
   auto load = [&](long k0) {
     if (k0 + TK <= K) {
       ca.template load<false>(ra, k0, K);
@@ -111,23 +117,28 @@ __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, lo
   for (long k0 = 0; k0 < K; k0 += TK) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ra[i] *= al;
+    for (int i = 0; i < Step<T>::EPT; ++i) ra[i] *= al;
     stage_step<AM, T>(SA, ra, tid);
     stage_step<BM, T>(SB, rb, tid);
     __syncthreads();
     if (k0 + TK < K) load(k0 + TK);
 #pragma unroll
     for (int kk = 0; kk < TK / 4; ++kk) {
-      double a[IW], b[IW];
+      if (k0 + kk * 4 >= K) break;
+      double a[IM], b[IN];
 #pragma unroll
-      for (int u = 0; u < IW; ++u) {
-        a[u] = SA.at(wm * 64 + u * 16 + lr, kk * 4 + lk);
-        b[u] = SB.at(wn * 64 + u * 16 + lr, kk * 4 + lk);
+      for (int u = 0; u < IM; ++u) a[u] = SA.at(wm + u * 16 + lr, kk * 4 + lk);
+#pragma unroll
+      for (int u = 0; u < IN; ++u) b[u] = SB.at(wn + u * 16 + lr, kk * 4 + lk);
+#pragma unroll
+      for (int i = 0; i < (X ? IM : IN); ++i) {
+        if (E && i >= nv) break;
+#pragma unroll
+        for (int j = 0; j < (X ? IN : IM); ++j) {
+          d4& c = X ? acc[i][j] : acc[j][i];
+          c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[X ? i : j], b[X ? j : i], c, 0, 0, 0);
+        }
       }
-#pragma unroll
-      for (int i = 0; i < IW; ++i)
-#pragma unroll
-        for (int j = 0; j < IW; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
     }
   }
 }
@@ -136,50 +147,54 @@ __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, lo
 // other two the other way; the sequence is static so the accumulators stay
 // in registers from term to term.
 template <bool X, bool E>
-__device__ __forceinline__ void tile4(const DMulti& p, long m0, long n0, long z, Smem& S) {
-  d4 acc[IW][IW];
+__device__ __forceinline__ void tile4(const DMulti& p, long m0, long n0, Smem& S) {
+  constexpr int IM = X ? T / 16 : T / 64, IN = X ? T / 64 : T / 16;
+  d4 acc[IM][IN];
 #pragma unroll
-  for (int i = 0; i < IW; ++i)
+  for (int i = 0; i < IM; ++i)
 #pragma unroll
-    for (int j = 0; j < IW; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int j = 0; j < IN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   const int ma = (int)min((long)T - 1, p.M - 1 - m0), nb = (int)min((long)T - 1, p.N - 1 - n0);
-  term<X, E>(p.t[0], ma, nb, m0, n0, z, acc, S);
-  term<X, E>(p.t[1], ma, nb, m0, n0, z, acc, S);
-  term<!X, E>(p.t[2], ma, nb, m0, n0, z, acc, S);
-  term<!X, E>(p.t[3], ma, nb, m0, n0, z, acc, S);
+  term<X, X, E>(p.t[0], ma, nb, m0, n0, acc, S);
+  term<X, X, E>(p.t[1], ma, nb, m0, n0, acc, S);
+  term<X, !X, E>(p.t[2], ma, nb, m0, n0, acc, S);
+  term<X, !X, E>(p.t[3], ma, nb, m0, n0, acc, S);
   __syncthreads();  // the next item reuses the LDS
   // D[i][j] of a 16x16 f64 MFMA tile: lane = j + 16*(i%4), element i/4.
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1, lr = lane & 15, lk = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int wm = X ? 0 : wave * (T / 4), wn = X ? wave * (T / 4) : 0;
+  // the descriptor's fields are read once (a store through C could alias them)
+  CCGPU_GLOBAL double* C = gptr(p.C);
+  const long c_m = p.c_m, c_no = p.c_no;
+  const int nin = p.nin;
+  const double beta = p.beta;
+  long co[IN];  // column offsets, clamped into C
+#pragma unroll
+  for (int j = 0; j < IN; ++j) {
+    const int n = (int)n0 + min(wn + j * 16 + lr, nb), q = n / nin;
+    co[j] = q * c_no + (n - q * nin);
+  }
   // per 16-row block: C read (beta != 0) before any of the block's stores,
   // so the loads overlap instead of each waiting behind a store
-  // the descriptor's fields are read once (a store through C could alias them)
-  CCGPU_GLOBAL double* C = gptr(p.C + z * p.c_b);
-  const long M = p.M, N = p.N, c_m = p.c_m, c_n = p.c_n;
-  const double beta = p.beta;
 #pragma unroll
-  for (int i = 0; i < IW; ++i) {
-    double cv[IW][4] = {};
+  for (int i = 0; i < IM; ++i) {
+    if (E && wm + i * 16 > ma) break;
+    double cv[IN][4] = {};
     if (beta != 0.0) {  // uniform; indices clamped into C: no per-element branch
 #pragma unroll
-      for (int j = 0; j < IW; ++j)
+      for (int j = 0; j < IN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const long m = min(m0 + wm * 64 + i * 16 + r * 4 + lk, M - 1);
-          const long n = min(n0 + wn * 64 + j * 16 + lr, N - 1);
-          cv[j][r] = C[m * c_m + n * c_n];
-        }
+        for (int r = 0; r < 4; ++r) cv[j][r] = C[(m0 + min(wm + i * 16 + r * 4 + lk, ma)) * c_m + co[j]];
     }
 #pragma unroll
-    for (int j = 0; j < IW; ++j)
+    for (int j = 0; j < IN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const long m = m0 + wm * 64 + i * 16 + r * 4 + lk;
-        const long n = n0 + wn * 64 + j * 16 + lr;
-        if (m < M && n < N) {
+        const int m = wm + i * 16 + r * 4 + lk;
+        if (m <= ma && wn + j * 16 + lr <= nb) {
           double v = acc[i][j][r];
           if (beta != 0.0) v += beta * cv[j][r];
-          C[m * c_m + n * c_n] = v;
+          C[(m0 + m) * c_m + co[j]] = v;
         }
       }
   }
@@ -507,14 +522,14 @@ __device__ __forceinline__ void pass_tile(const PtRun& r, long q, int ph, long t
     const bool inside = m0 + 128 <= d.M && n0 + 128 <= d.N;
     if (ph < 2) {
       if (inside)
-        dt::tile4<true, false>(d, m0, n0, z, GS);
+        dt::tile4<true, false>(d,m0, n0, GS);
       else
-        dt::tile4<true, true>(d, m0, n0, z, GS);
+        dt::tile4<true, true>(d,m0, n0, GS);
     } else {
       if (inside)
-        dt::tile4<false, false>(d, m0, n0, z, GS);
+        dt::tile4<false, false>(d,m0, n0, GS);
       else
-        dt::tile4<false, true>(d, m0, n0, z, GS);
+        dt::tile4<false, true>(d,m0, n0, GS);
     }
   }
 }
@@ -626,45 +641,53 @@ __global__ __launch_bounds__(PtShape<MIXED>::NT, MIXED ? 1 : 2) void k_pt_persis
 // The same W passes and energy evaluation as plain launches (stream order
 // instead of in-kernel dependencies).
 
-// Tile of block b: each XCD (block b runs on XCD b % 8) gets a contiguous
-// range of tiles, walked in groups of 8 m-tiles.
-__device__ __forceinline__ void tile_xcd(long b, long tiles_m, long tiles_n, long& tm, long& tn) {
-  const long nt = tiles_m * tiles_n;
-  const long per = nt / 8, full = per * 8;
-  tile_grouped((b < full) ? (b % 8) * per + b / 8 : b, tiles_m, tiles_n, tm, tn);
+// Tile and batch of block b of a triple, nx = grid_xcd(tiles) blocks a triple:
+// each XCD (block b runs on XCD b % 8) gets a contiguous range of batches and,
+// in a batch, of tiles walked in groups of 8 m-tiles, the same range for every
+// triple.  false: a block past the range.
+__device__ __forceinline__ bool tile_xcd(long b, long nx, long tiles_m, long tiles_n, long batch, long& tm, long& tn,
+                                         long& z) {
+  const long per = nx / 8, t = (b % 8) * per + b / 8, nt = tiles_m * tiles_n;
+  if (t >= nt * batch) return false;
+  z = t / nt;
+  tile_grouped(t - z * nt, tiles_m, tiles_n, tm, tn);
+  return true;
 }
+unsigned grid_xcd(long tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
 
 // One W pass of several triples: blockIdx.y takes the triple (its descriptor
-// in list), blockIdx.z the batch, blockIdx.x the tile.  Bound by the matrix
-// cores once the chip is full, which a single triple's pass does not do below
-// v = 256 (80 to 101 blocks at v = 101, 50 us a launch).  The full list at
-// o=12 v=101, FP64: 87.9 ms in 1760 launches one triple at a time, 18.6 ms in
-// 70 with 26 triples each.
+// in list), blockIdx.x the tile.  Bound by the matrix cores once the chip is
+// full, which a single triple's pass does not do below v = 256 (80 blocks at
+// v = 101, 50 us a launch).  The full list at o=12 v=101, FP64: 87.9 ms in
+// 1760 launches one triple at a time, 18.6 ms with 26 triples each, 16.0 with
+// the columns of G2 flat (v batches of v x v pad both sides: 470 against 400
+// us a launch) and the waves along the long side, 15.0 with 25 triples.
 template <bool X>
 __global__ __launch_bounds__(256, 2) void k_dtile4(const DMulti* list, long tiles_m, long tiles_n) {
   __shared__ dt::Smem S;
   const DMulti& p = list[blockIdx.y];
-  long tm, tn;
-  tile_xcd(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const long m0 = tm * 128, n0 = tn * 128;
-  if (m0 + 128 <= p.M && n0 + 128 <= p.N)
-    dt::tile4<X, false>(p, m0, n0, blockIdx.z, S);
+  long tm, tn, z;
+  if (!tile_xcd(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1, tm, tn, z)) return;
+  const long m0 = tm * dt::T, n0 = tn * dt::T;
+  if (m0 + dt::T <= p.M && n0 + dt::T <= p.N)
+    dt::tile4<X, false>(p, m0, n0, S);
   else
-    dt::tile4<X, true>(p, m0, n0, blockIdx.z, S);
+    dt::tile4<X, true>(p, m0, n0, S);
 }
 
 // The mixed passes: the 256x256 tile (W8) or the 128x128 one.
 template <bool W8>
-__global__ __launch_bounds__(W8 ? 512 : 256, W8 ? 1 : 2) void k_btile4(const BMulti* list, long tiles_m, long tiles_n) {
+__global__ __launch_bounds__(W8 ? 512 : 256, W8 ? 1 : 2) void k_btile4(const BMulti* list, long tiles_m, long tiles_n,
+                                                                       long batch) {
   const BMulti& p = list[blockIdx.y];
-  long tm, tn;
-  tile_xcd(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  long tm, tn, z;
+  if (!tile_xcd(blockIdx.x, gridDim.x, tiles_m, tiles_n, batch, tm, tn, z)) return;
   if constexpr (W8) {
     __shared__ bf3w8::Smem S;
-    bf3w8::tile<float, true>(p, tm * bf3w8::DT, tn * bf3w8::DT, blockIdx.z, S);
+    bf3w8::tile<float, true>(p, tm * bf3w8::DT, tn * bf3w8::DT, z, S);
   } else {
     __shared__ bf3::Smem<2> S;
-    bf3::tile<float, 2>(p, tm * 128, tn * 128, blockIdx.z, S);
+    bf3::tile<float, 2>(p, tm * 128, tn * 128, z, S);
   }
 }
 
@@ -692,13 +715,14 @@ __global__ void k_zero_u64(unsigned long long* p, int n) {
 }
 
 // FP64 descriptor with every operand span checked.
-DMulti d_desc(std::initializer_list<DTerm> terms, long M, long N, int batch, double* C, long c_m, long c_n,
-              long c_b, double beta) {
+DMulti d_desc(std::initializer_list<DTerm> terms, long M, long N, double* C, long c_m, long nin, long c_no,
+              double beta) {
   DMulti p{};
   CCGPU_REQUIRE(terms.size() >= 1 && terms.size() <= 4, "pt: 1..4 terms");
+  CCGPU_REQUIRE(N < (1L << 31) && nin > 0 && N % nin == 0, "pt: columns in whole rows of C");
   for (const DTerm& t : terms) {
-    check_span(t.A, 0, (M - 1) * t.a_m + (t.K - 1) * t.a_k + (batch - 1) * t.a_b, sizeof(double), "pt A");
-    check_span(t.B, 0, (N - 1) * t.b_n + (t.K - 1) * t.b_k + (batch - 1) * t.b_b, sizeof(double), "pt B");
+    check_span(t.A, 0, (M - 1) * t.a_m + (t.K - 1) * t.a_k, sizeof(double), "pt A");
+    check_span(t.B, 0, (N - 1) * t.b_n + (t.K - 1) * t.b_k, sizeof(double), "pt B");
     p.t[p.nterm++] = t;
   }
   CCGPU_REQUIRE(p.nterm == 4 && p.t[0].akf == p.t[1].akf && p.t[2].akf == p.t[3].akf && p.t[0].akf != p.t[2].akf,
@@ -708,9 +732,9 @@ DMulti d_desc(std::initializer_list<DTerm> terms, long M, long N, int batch, dou
   p.beta = beta;
   p.C = C;
   p.c_m = c_m;
-  p.c_n = c_n;
-  p.c_b = c_b;
-  check_span(C, 0, (M - 1) * c_m + (N - 1) * c_n + (batch - 1) * c_b, sizeof(double), "pt C");
+  p.c_no = c_no;
+  p.nin = (int)nin;
+  check_span(C, 0, (M - 1) * c_m + (N / nin - 1) * c_no + nin - 1, sizeof(double), "pt C");
   return p;
 }
 
@@ -741,14 +765,14 @@ long env_long(const char* name, long dflt) {
   return (e && *e) ? std::atol(e) : dflt;
 }
 
-// Tiles of the three W passes: G1 v x v^2, G2 v batches of v x v, G3 v^2 x v.
+// Tiles of the three W passes: G1 v x v^2, G2 v x v^2 (mixed: v batches of v x v), G3 v^2 x v.
 struct PassShape {
   long M[3], N[3], tm[3], tn[3], batch[3], ng[3];
 };
 PassShape pass_shape(bool mixed, int v) {
   PassShape ps{};
   const long vv = (long)v * v;
-  const long Ms[3] = {v, v, vv}, Ns[3] = {vv, v, v}, Bs[3] = {1, v, 1};
+  const long Ms[3] = {v, v, vv}, Ns[3] = {vv, mixed ? v : vv, v}, Bs[3] = {1, mixed ? v : 1, 1};
   for (int g = 0; g < 3; ++g) {
     // mixed: 256 x 256 tiles over operands padded to 256 rows; FP64: 128 x 128
     ps.tm[g] = mixed ? cdiv(bf16x3_rpad(Ms[g]), bf3w8::DT) : cdiv(Ms[g], 128);
@@ -811,21 +835,22 @@ void CCSD::pt_descs(int i, int j, int k, int slot, unsigned char* out) {
     DMulti* d = reinterpret_cast<DMulti*>(out);
     // the same twelve terms; A read along k and B along n for the G terms of G1 and G2, the other way round
     // for their occupied terms; the reverse in G3
-    d[0] = d_desc({DTerm{Td(i, j), Gk, nov, 1, 0, 1, vv, 0, v, 1.0, 1},
-                   DTerm{Td(i, k), Gp_.p + (long)j * vvv, nov, 1, 0, 1, vv, 0, v, 1.0, 1},
-                   DTerm{Qd(i, k), Pd(j), 1, v, 0, o, 1, 0, o, -1.0, 0},
-                   DTerm{Qd(i, j), Sd(k), 1, v, 0, o, 1, 0, o, -1.0, 0}},
-                  v, vv, 1, Wq, vv, 1, 0, 0.0);
-    d[1] = d_desc({DTerm{Td(j, i), Gk, nov, 1, 0, 1, vv, v, v, 1.0, 1},
-                   DTerm{Td(j, k), Gp_.p + (long)i * vvv, nov, 1, 0, 1, vv, v, v, 1.0, 1},
-                   DTerm{Qd(j, k), Pd(i), 1, v, 0, o, 1, (long)v * o, o, -1.0, 0},
-                   DTerm{Qd(j, i), Sd(k), 1, v, 0, o, 1, (long)v * o, o, -1.0, 0}},
-                  v, v, v, Wq, v, 1, vv, 1.0);
-    d[2] = d_desc({DTerm{G_.p + (long)j * vvv, Td(k, i), 1, vv, 0, nov, 1, 0, v, 1.0, 0},
-                   DTerm{Gp_.p + (long)i * vvv, Td(k, j), 1, vv, 0, nov, 1, 0, v, 1.0, 0},
-                   DTerm{Pd(i), Qd(k, j), o, 1, 0, 1, v, 0, o, -1.0, 1},
-                   DTerm{Sd(j), Qd(k, i), o, 1, 0, 1, v, 0, o, -1.0, 1}},
-                  vv, v, 1, Wq, v, 1, 0, 1.0);
+    d[0] = d_desc({DTerm{Td(i, j), Gk, nov, 1, 1, vv, v, 1.0, 1},
+                   DTerm{Td(i, k), Gp_.p + (long)j * vvv, nov, 1, 1, vv, v, 1.0, 1},
+                   DTerm{Qd(i, k), Pd(j), 1, v, o, 1, o, -1.0, 0},
+                   DTerm{Qd(i, j), Sd(k), 1, v, o, 1, o, -1.0, 0}},
+                  v, vv, Wq, vv, vv, 0, 0.0);
+    // G2: the columns are (a, c), a slowest, as they lie in the B operands
+    d[1] = d_desc({DTerm{Td(j, i), Gk, nov, 1, 1, vv, v, 1.0, 1},
+                   DTerm{Td(j, k), Gp_.p + (long)i * vvv, nov, 1, 1, vv, v, 1.0, 1},
+                   DTerm{Qd(j, k), Pd(i), 1, v, o, 1, o, -1.0, 0},
+                   DTerm{Qd(j, i), Sd(k), 1, v, o, 1, o, -1.0, 0}},
+                  v, vv, Wq, v, v, vv, 1.0);
+    d[2] = d_desc({DTerm{G_.p + (long)j * vvv, Td(k, i), 1, vv, nov, 1, v, 1.0, 0},
+                   DTerm{Gp_.p + (long)i * vvv, Td(k, j), 1, vv, nov, 1, v, 1.0, 0},
+                   DTerm{Pd(i), Qd(k, j), o, 1, 1, v, o, -1.0, 1},
+                   DTerm{Sd(j), Qd(k, i), o, 1, 1, v, o, -1.0, 1}},
+                  vv, v, Wq, v, v, 0, 1.0);
   }
 }
 
@@ -836,14 +861,15 @@ EArgs energy_args(const int* ctab, const double* J, const double* t1, const doub
 }
 }  // namespace
 
-// Triples per launch of the W passes: enough for four waves of blocks over the
-// CUs (two 128 x 128 blocks or one 256 x 256 block per CU), at most 64, with
-// their W slots inside 256 MB, about what the last-level cache holds (G2, G3
-// and the energy re-read W).  One at v = 512.
+// Triples per launch of the W passes: just below four waves of blocks over the
+// CUs (two 128 x 128 blocks or one 256 x 256 block per CU; just above, a fifth
+// one is nearly empty: v=101 26 triples 16.0 ms the full list, 25 15.0), at
+// most 64, with their W slots inside 256 MB, about what the last-level cache
+// holds (G2, G3 and the energy re-read W).  One at v = 512.
 long CCSD::pt_group(bool mixed) const {
   const PassShape ps = pass_shape(mixed, dm_.v);
   const long fewest = std::min(std::min(ps.ng[0], ps.ng[1]), ps.ng[2]), vvv = (long)dm_.v * dm_.v * dm_.v;
-  const long fill = ((mixed ? 1024 : 2048) + fewest - 1) / fewest;
+  const long fill = (mixed ? 1024 : 2048) / fewest;
   const long room = (256L << 20) / (vvv * (long)(mixed ? sizeof(float) : sizeof(double)));
   return std::max<long>(1, std::min<long>({fill, room, 64, pt_ntriples()}));
 }
@@ -897,7 +923,7 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
       for (int g = 0; g < 3; ++g) {
         const unsigned char* list = ptdesc_.p + (g * nr + q0) * dsz;
         const unsigned nb = (unsigned)ps.batch[g];
-        CCGPU_REQUIRE(ps.tm[g] * ps.tn[g] < (1L << 23) && ps.batch[g] < 65536, "pt: grid too large");
+        CCGPU_REQUIRE(ps.tm[g] * ps.tn[g] * ps.batch[g] < (1L << 22), "pt: grid too large");
         if (mixed) {
           const BMulti* d = reinterpret_cast<const BMulti*>(list);
           // the 256 tile where padding to 256 rows does not cost more than its higher rate gives
@@ -906,14 +932,14 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
           const bool w8 = bf16x3_large_tile(ps.M[g], ps.N[g], (long)gn * nb);
           const int id = prof_begin("k_gemm_bf16x3", fg * gn, st_);
           if (w8)
-            CCGPU_LAUNCH(k_btile4<true>, dim3((unsigned)(ps.tm[g] * ps.tn[g]), gn, nb), dim3(512), 0, st_, d,
-                         ps.tm[g], ps.tn[g]);
+            CCGPU_LAUNCH(k_btile4<true>, dim3(grid_xcd(ps.tm[g] * ps.tn[g] * nb), gn), dim3(512), 0, st_, d, ps.tm[g],
+                         ps.tn[g], (long)nb);
           else
-            CCGPU_LAUNCH(k_btile4<false>, dim3((unsigned)(tm1 * tn1), gn, nb), dim3(256), 0, st_, d, tm1, tn1);
+            CCGPU_LAUNCH(k_btile4<false>, dim3(grid_xcd(tm1 * tn1 * nb), gn), dim3(256), 0, st_, d, tm1, tn1, (long)nb);
           prof_end(id, st_);
         } else {
           const DMulti* d = reinterpret_cast<const DMulti*>(list);
-          const dim3 grid((unsigned)(ps.tm[g] * ps.tn[g]), gn, nb);
+          const dim3 grid(grid_xcd(ps.tm[g] * ps.tn[g] * nb), gn);
           const int id = prof_begin(g < 2 ? "k_dtile4<true>" : "k_dtile4<false>", fg * gn, st_);
           if (g < 2)
             CCGPU_LAUNCH(k_dtile4<true>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
