@@ -243,10 +243,10 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
     src = q + z * bs + (r0 + lrow) * T.Kp + 8 * (lslot ^ ((lrow >> 1) & 3));
   };
   long total = 0;
-  for (int tl = 0; tl < p.nterm; ++tl) total += p.t[tl].Kp / DTK;
+  for (int tl = 0; tl < p.nterm; ++tl) total += p.t[tl].Kc / DTK;
   int lt = 0;
-  while (lt < p.nterm && p.t[lt].Kp < DTK) ++lt;
-  long ls = 0, lsteps = lt < p.nterm ? p.t[lt].Kp / DTK : 0;
+  while (lt < p.nterm && p.t[lt].Kc < DTK) ++lt;
+  long ls = 0, lsteps = lt < p.nterm ? p.t[lt].Kc / DTK : 0;
   // past the last step the cursor stays put (loads in bounds, never used)
   auto advance = [&]() {
     if (ls + 1 < lsteps) {
@@ -255,11 +255,11 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
       return;
     }
     int nt = lt + 1;
-    while (nt < p.nterm && p.t[nt].Kp < DTK) ++nt;
+    while (nt < p.nterm && p.t[nt].Kc < DTK) ++nt;
     if (nt < p.nterm) {
       lt = nt;
       ls = 0;
-      lsteps = p.t[lt].Kp / DTK;
+      lsteps = p.t[lt].Kc / DTK;
       point(lt);
     }
   };
@@ -413,10 +413,10 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
     }
   };
   long total = 0;  // K steps of all terms
-  for (int tl = 0; tl < p.nterm; ++tl) total += p.t[tl].Kp / DTK;
+  for (int tl = 0; tl < p.nterm; ++tl) total += p.t[tl].Kc / DTK;
   int lt = 0;
-  while (lt < p.nterm && p.t[lt].Kp < DTK) ++lt;
-  long ls = 0, lsteps = lt < p.nterm ? p.t[lt].Kp / DTK : 0;
+  while (lt < p.nterm && p.t[lt].Kc < DTK) ++lt;
+  long ls = 0, lsteps = lt < p.nterm ? p.t[lt].Kc / DTK : 0;
   // past the last step the cursor stays put: the loads re-read the last K
   // slice into the free stage (in bounds, never read)
   auto advance = [&]() {
@@ -427,11 +427,11 @@ __device__ __forceinline__ void tile(const BMulti& p, long m0, long n0, long z, 
       return;
     }
     int nt = lt + 1;
-    while (nt < p.nterm && p.t[nt].Kp < DTK) ++nt;
+    while (nt < p.nterm && p.t[nt].Kc < DTK) ++nt;
     if (nt < p.nterm) {
       lt = nt;
       ls = 0;
-      lsteps = p.t[lt].Kp / DTK;
+      lsteps = p.t[lt].Kc / DTK;
       point(lt);
     }
   };

@@ -348,13 +348,13 @@ void CCSD::ladder_mixed(double* Om) {
     for (size_t q = 0; q + 1 < strips.size(); ++q) {
       const long s0 = strips[q], Ms = (strips[q + 1] - s0) * v, Ns = (v - s0) * v;
       const unsigned short *bh = lpBh_.p + s0 * v * KpB, *bl = lpBl_.p + s0 * v * KpB;
-      const BTerm ty{bh, bl, bh, bl, KpB, 0, 0};
+      const BTerm ty{bh, bl, bh, bl, KpB, 0, 0, bf16x3_kcols(naux)};
       bf16x3_multi(&ty, 1, Ms, Ns, 1, Y32 + (s0 - a0) * v * (ldY + 1), true, ldY, 1, 0, 1.0, 0.0, 2.0 * Ms * Ns * naux,
                    st_);
     }
     const long Rp = bf16x3_rpad(rows);
     ladder_vpm_pack(lpVh_.p, lpVl_.p, Y32, ldY, a0, a1, v, Rp, KpT, st_);
-    const BTerm ts{lpVh_.p, lpVl_.p, lpTh_.p, lpTl_.p, KpT, Rp * KpT, RpT * KpT};
+    const BTerm ts{lpVh_.p, lpVl_.p, lpTh_.p, lpTl_.p, KpT, Rp * KpT, RpT * KpT, bf16x3_kcols(npv)};
     bf16x3_multi(&ts, 1, rows, npo, 2, Sp, false, npo, 1, maxr * npo, 1.0, 0.0, 4.0 * rows * npo * npv, st_);
     ladder_scatter(Om, Sp, Sm, a0, a1, o, v, st_);
   }

@@ -166,6 +166,7 @@ struct BTerm {
   const unsigned short *Ah, *Al, *Bh, *Bl;
   long Kp;         // row length (padded K) of this term's A and B
   long a_bs, b_bs;  // batch strides (elements) of the packed A and B
+  long Kc = 0;      // columns to multiply, a multiple of 32 (0: Kp); those from Kc to Kp hold zeros
 };
 struct BMulti {
   BTerm t[4];
@@ -177,6 +178,7 @@ struct BMulti {
   long c_m, c_n, c_b;
 };
 long bf16x3_kpad(long K);
+long bf16x3_kcols(long K);  // K padded to the 32 columns of a matrix instruction (BTerm::Kc)
 long bf16x3_rpad(long R);
 // Whether the cost model takes the 256 x 256 tile for batch products of M x N.
 bool bf16x3_large_tile(long M, long N, long batch);

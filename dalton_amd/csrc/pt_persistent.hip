@@ -797,16 +797,16 @@ void CCSD::pt_descs(int i, int j, int k, int slot, unsigned char* out) {
   const long nov = dm_.nov, vv = (long)v * v, vvv = vv * v;
   if (mixed) {
     const long Kpv = bf16x3_kpad(v), Kpo = bf16x3_kpad(o), Rv = bf16x3_rpad(v), Rvv = bf16x3_rpad(vv) + 256;
-    const long gk = vv * Kpv;
+    const long gk = vv * Kpv, Kcv = bf16x3_kcols(v), Kco = bf16x3_kcols(o);
     auto Tm = [&](int p, int q, bool hi) { return (hi ? ppH_[0].p : ppL_[0].p) + ((long)p * o + q) * Rv * Kpv; };
     auto Qm = [&](int p, int q, bool hi) { return (hi ? ppH_[1].p : ppL_[1].p) + ((long)p * o + q) * Rv * Kpo; };
     auto Pm = [&](int p, bool hi) { return (hi ? ppH_[2].p : ppL_[2].p) + (long)p * Rvv * Kpo; };
     auto Sm = [&](int p, bool hi) { return (hi ? ppH_[3].p : ppL_[3].p) + (long)p * Rvv * Kpo; };
     auto TT = [&](int p, int q, const unsigned short* Bh, const unsigned short* Bl, long bbs) {  // T(p,q) x G
-      return BTerm{Tm(p, q, true), Tm(p, q, false), Bh, Bl, Kpv, 0, bbs};
+      return BTerm{Tm(p, q, true), Tm(p, q, false), Bh, Bl, Kpv, 0, bbs, Kcv};
     };
     auto QP = [&](int p, int q, const unsigned short* Bh, const unsigned short* Bl, long bbs) {  // Q_pq x Tvvo
-      return BTerm{Qm(p, q, true), Qm(p, q, false), Bh, Bl, Kpo, 0, bbs};
+      return BTerm{Qm(p, q, true), Qm(p, q, false), Bh, Bl, Kpo, 0, bbs, Kco};
     };
     float* Wq = W32_.p + slot * vvv;
     const unsigned short *GTk = GTh_.p + k * gk, *GTkl = GTl_.p + k * gk;
@@ -820,10 +820,10 @@ void CCSD::pt_descs(int i, int j, int k, int slot, unsigned char* out) {
                          QP(j, k, Pm(i, true), Pm(i, false), v * Kpo), QP(j, i, Sm(k, true), Sm(k, false), v * Kpo)};
     d[1] = bf16x3_desc(g2, 4, v, v, v, Wq, true, v, 1, vv, 1.0, 1.0);
     // G3: W[(a,b)][c] += (ad|bj) t_ki^{cd} + (bd|ai) t_kj^{cd} - t_il^{ab} (ck|lj) - t_jl^{ba} (ck|li)
-    const BTerm g3[4] = {BTerm{GTh_.p + j * gk, GTl_.p + j * gk, Tm(k, i, true), Tm(k, i, false), Kpv, 0, 0},
-                         BTerm{GpTh_.p + i * gk, GpTl_.p + i * gk, Tm(k, j, true), Tm(k, j, false), Kpv, 0, 0},
-                         BTerm{Pm(i, true), Pm(i, false), Qm(k, j, true), Qm(k, j, false), Kpo, 0, 0},
-                         BTerm{Sm(j, true), Sm(j, false), Qm(k, i, true), Qm(k, i, false), Kpo, 0, 0}};
+    const BTerm g3[4] = {BTerm{GTh_.p + j * gk, GTl_.p + j * gk, Tm(k, i, true), Tm(k, i, false), Kpv, 0, 0, Kcv},
+                         BTerm{GpTh_.p + i * gk, GpTl_.p + i * gk, Tm(k, j, true), Tm(k, j, false), Kpv, 0, 0, Kcv},
+                         BTerm{Pm(i, true), Pm(i, false), Qm(k, j, true), Qm(k, j, false), Kpo, 0, 0, Kco},
+                         BTerm{Sm(j, true), Sm(j, false), Qm(k, i, true), Qm(k, i, false), Kpo, 0, 0, Kco}};
     d[2] = bf16x3_desc(g3, 4, vv, v, 1, Wq, true, v, 1, 0, 1.0, 1.0);
   } else {
     auto Td = [&](int p, int q) { return T_.p + (long)p * v * nov + (long)q * v; };  // [x][d], row stride nov
