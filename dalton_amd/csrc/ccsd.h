@@ -158,6 +158,8 @@ class CCSD {
   void ladder_mixed(double* Om);
   std::vector<int> ladder_strips(int a0, int a1, long rows, long tiles) const;
   void ladder_y(int a0, int a1);
+  void ladder_pack_b();
+  void ladder_y_packed(int a0, int a1, void* Y, bool y_float, long ldY);
   void mark(const char* name);
   void ensure_work();
   // (T) drivers: launches per group of triples of the pre-packed three-pass W

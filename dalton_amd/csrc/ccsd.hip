@@ -306,6 +306,29 @@ void CCSD::ladder_y(int a0, int a1) {
   }
 }
 
+// Bvv split into bf16 hi/lo, a row per (a,c), K = naux: once per ladder.
+void CCSD::ladder_pack_b() {
+  const long vv = (long)dm_.v * dm_.v, naux = dm_.naux;
+  // every batch reads rows up to a0*v + rpad(...) < vv + (row padding)
+  const long RpB = bf16x3_rpad(vv + bf16x3_rpad(1) - 1), KpB = bf16x3_kpad(naux);
+  lpBh_.ensure((size_t)RpB * KpB);
+  lpBl_.ensure((size_t)RpB * KpB);
+  bf16x3_pack(Bvv_.p, vv, naux, 1, vv, 0, 1, RpB, KpB, 1.0f, lpBh_.p, lpBl_.p, st_);
+}
+
+// ladder_y from the packed factor into float or double Y of row length ldY.
+void CCSD::ladder_y_packed(int a0, int a1, void* Y, bool y_float, long ldY) {
+  const long v = dm_.v, Nn = (v - a0) * v, KpB = bf16x3_kpad(dm_.naux);
+  const std::vector<int> strips = ladder_strips(a0, a1, Nn, 1024);
+  for (size_t q = 0; q + 1 < strips.size(); ++q) {
+    const long s0 = strips[q], Ms = (strips[q + 1] - s0) * v, Ns = (v - s0) * v, off = (s0 - a0) * v * (ldY + 1);
+    const unsigned short *bh = lpBh_.p + s0 * v * KpB, *bl = lpBl_.p + s0 * v * KpB;
+    const BTerm ty{bh, bl, bh, bl, KpB, 0, 0, bf16x3_kcols(dm_.naux)};
+    void* C = y_float ? (void*)(static_cast<float*>(Y) + off) : (void*)(static_cast<double*>(Y) + off);
+    bf16x3_multi(&ty, 1, Ms, Ns, 1, C, y_float, ldY, 1, 0, 1.0, 0.0, 2.0 * Ms * Ns * dm_.naux, st_);
+  }
+}
+
 // The same ladder with BF16x3 products.  The dressed factor Bvv and tau+/-
 // are split into bf16 hi/lo once per call (not per batch); each batch forms
 // Y in FP32 straight from the packed factor, and V+/- goes from Y directly
@@ -319,18 +342,14 @@ void CCSD::ladder_mixed(double* Om) {
     for (int a = lad_batches_[bi]; a < lad_batches_[bi + 1]; ++a) rows += v - a;
     maxr = std::max(maxr, rows);
   }
-  // rows of the packed factor: every batch reads a0*v + rpad(...) < vv + (row padding) rows
-  const long RpB = bf16x3_rpad(vv + bf16x3_rpad(1) - 1), KpB = bf16x3_kpad(naux);
   const long RpT = bf16x3_rpad(npo), KpT = bf16x3_kpad(npv);
   const long RpV = bf16x3_rpad(maxr);
-  lpBh_.ensure((size_t)RpB * KpB);
-  lpBl_.ensure((size_t)RpB * KpB);
   lpTh_.ensure((size_t)2 * RpT * KpT);
   lpTl_.ensure((size_t)2 * RpT * KpT);
   lpVh_.ensure((size_t)2 * RpV * KpT);
   lpVl_.ensure((size_t)2 * RpV * KpT);
   S2_.ensure((size_t)2 * maxr * npo);
-  bf16x3_pack(Bvv_.p, vv, naux, 1, vv, 0, 1, RpB, KpB, 1.0f, lpBh_.p, lpBl_.p, st_);
+  ladder_pack_b();
   bf16x3_pack(tau_.p, npo, npv, npv, 1, npo * npv, 2, RpT, KpT, 1.0f, lpTh_.p, lpTl_.p, st_);
   float* Y32 = reinterpret_cast<float*>(Y_.p);
   double* Sp = S2_.p;
@@ -344,14 +363,7 @@ void CCSD::ladder_mixed(double* Om) {
     // memory channel (v = 256: 6.9 -> 6.4 ms of V+/-)
     const long ldY = Nn % 512 ? Nn : Nn + 32;
     CCGPU_REQUIRE((size_t)(M * ldY) <= 2 * Y_.n, "ladder_mixed: Y block exceeds its buffer");
-    const std::vector<int> strips = ladder_strips(a0, a1, Nn, 1024);
-    for (size_t q = 0; q + 1 < strips.size(); ++q) {
-      const long s0 = strips[q], Ms = (strips[q + 1] - s0) * v, Ns = (v - s0) * v;
-      const unsigned short *bh = lpBh_.p + s0 * v * KpB, *bl = lpBl_.p + s0 * v * KpB;
-      const BTerm ty{bh, bl, bh, bl, KpB, 0, 0, bf16x3_kcols(naux)};
-      bf16x3_multi(&ty, 1, Ms, Ns, 1, Y32 + (s0 - a0) * v * (ldY + 1), true, ldY, 1, 0, 1.0, 0.0, 2.0 * Ms * Ns * naux,
-                   st_);
-    }
+    ladder_y_packed(a0, a1, Y32, true, ldY);
     const long Rp = bf16x3_rpad(rows);
     ladder_vpm_pack(lpVh_.p, lpVl_.p, Y32, ldY, a0, a1, v, Rp, KpT, st_);
     const BTerm ts{lpVh_.p, lpVl_.p, lpTh_.p, lpTl_.p, KpT, Rp * KpT, RpT * KpT, bf16x3_kcols(npv)};

@@ -83,6 +83,7 @@ void coulomb_diag(double* Jd, const double* Bt, long naux, int N, int o, hipStre
 
 // small helpers
 void fill(double* p, double val, long n, hipStream_t st);
+void zero_rect(double* p, long rows, long cols, long ld, hipStream_t st);
 void axpy(double* y, double a, const double* x, long n, hipStream_t st);
 
 }  // namespace ccgpu

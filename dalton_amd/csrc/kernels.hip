@@ -659,6 +659,12 @@ __global__ void k_fill(double* p, double val, long n) {
     p[e] = val;
 }
 
+// Zeros in a block of rows (blockIdx.y) of leading dimension ld.
+__global__ void k_fill_rect(double* p, long cols, long ld) {
+  double* q = p + blockIdx.y * ld;
+  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < cols; e += (long)gridDim.x * blockDim.x) q[e] = 0.0;
+}
+
 __global__ void k_axpy(double* y, double a, const double* x, long n) {
   for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
     y[e] += a * x[e];
@@ -669,6 +675,15 @@ void fill(double* p, double val, long n, hipStream_t st) {
   check_span(p, 0, n - 1, sizeof(double), "fill");
   CCGPU_LAUNCH(k_fill, dim3((unsigned)std::min<long>(65536, (n + 255) / 256)), dim3(256), 0, st, p,
                      val, n);
+  CCGPU_HIPX(hipGetLastError());
+}
+
+void zero_rect(double* p, long rows, long cols, long ld, hipStream_t st) {
+  if (rows <= 0 || cols <= 0) return;
+  check_span(p, 0, (rows - 1) * ld + cols - 1, sizeof(double), "zero_rect");
+  const unsigned nx = (unsigned)std::min<long>(4096, (cols + 1023) / 1024);
+  for (long r = 0; r < rows; r += 65535)
+    CCGPU_LAUNCH(k_fill_rect, dim3(nx, (unsigned)std::min<long>(65535, rows - r)), dim3(256), 0, st, p + r * ld, cols, ld);
   CCGPU_HIPX(hipGetLastError());
 }
 

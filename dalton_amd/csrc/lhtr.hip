@@ -83,19 +83,29 @@ void CCSD::lhtr_ladder(const double* Xb) {
   const long vv = (long)v * v, npo = dm_.npo, npv = dm_.npv;
   const Gemm bulk{bulk_, st_};
   fill(taub_.p, 0.0, 2 * npo * npv, st_);
+  if (bulk_ == GemmPrec::BF16X3) ladder_pack_b();
   for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
     const int a0 = lad_batches_[bi], a1 = lad_batches_[bi + 1];
     long rows = 0;
     for (int a = a0; a < a1; ++a) rows += v - a;
     const long M = (long)(a1 - a0) * v, Nn = (long)(v - a0) * v;
     const double* Bb = Bvv_.p + (long)a0 * v;
-    ladder_y(a0, a1);
+    if (bulk_ == GemmPrec::BF16X3)
+      ladder_y_packed(a0, a1, Y_.p, false, Nn);
+    else
+      ladder_y(a0, a1);
     const long nv = rows * npv, ns = rows * npo, nt = npo * npv;  // the - arrays follow the + ones
     ladder_vpm(V_.p, V_.p + nv, Y_.p, Nn, a0, a1, v, st_);
     ladder_gather(S_.p, S_.p + ns, Xb, a0, a1, o, v, st_);
     bulk(npo, npv, rows, 0.5, S_.p, 1, npo, V_.p, npv, 1, 1.0, taub_.p, npv, 1, 2, ns, nv, nt);
     bulk(rows, npv, npo, 0.5, S_.p, npo, 1, tau_.p, npv, 1, 0.0, V_.p, npv, 1, 2, ns, nt, nv);
-    fill(Y_.p, 0.0, M * Nn, st_);  // entries with b < a stay zero
+    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::BF16X3 ? 512 : 64);
+    // Entries with b < a: zeros where the sums below read them, the blocks of
+    // a strip by itself and of its K padding (v = 192: 1.8 ms of all of Y).
+    for (size_t q = 0; q + 1 < sa.size(); ++q) {
+      const long r0 = (long)(sa[q] - a0) * v, c1 = (long)(sa[q + 1] - a0) * v, k0 = r0 / 64 * 64;
+      zero_rect(Y_.p + r0 * Nn + k0, std::min(M, (c1 + 63) / 64 * 64) - r0, c1 - k0, Nn, st_);
+    }
     ladder_vpm_adj(Y_.p, Nn, V_.p, V_.p + nv, a0, a1, v, st_);
     // Y_bar is zero for b < a: the strip [s0, s1) of a sums over b >= s0, that
     // of b over a < s1.  Both sums start and end at multiples of 64, the K
@@ -103,7 +113,6 @@ void CCSD::lhtr_ladder(const double* Xb) {
     // groups as the whole sums do.  K is the long side here and is not split in
     // BF16x3: there a strip keeps one wave of output tiles (512).
     double* Bbb = Bvvb_.p + (long)a0 * v;
-    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::BF16X3 ? 512 : 64);
     for (size_t q = 0; q + 1 < sa.size(); ++q) {
       const long r0 = (long)(sa[q] - a0) * v, nr = (long)(sa[q + 1] - sa[q]) * v, k0 = r0 / 64 * 64;
       bulk(naux, nr, Nn - k0, 1.0, Bb + k0, vv, 1, Y_.p + r0 * Nn + k0, 1, Nn, 1.0, Bbb + r0, vv, 1);
