@@ -71,8 +71,8 @@ namespace dt {
 // Tile 128 x 128, K step 16, 256 threads; operands staged global -> registers ->
 // LDS as in the FP64 GEMM (one pointer per operand walks K, rows past the
 // matrix re-read a row inside it, only a last partial K step compares k with
-// K), the next step's loads issued before the MFMAs.  The four waves lie side
-// by side along the long dimension (n for X, m for !X): the other one is
+// K), the next step's loads issued before the MFMAs.  LONG: the four waves lie
+// side by side along the long dimension (n for X, m for !X): the other one is
 // v, and its 16-row parts past v are left out of the products of all waves
 // alike (2 x 2 waves: only the waves that own them, and the others set the
 // time of a step; o=12 v=101 full list 17.5 against 16.0 ms).  A 64 x 64 tile
@@ -84,16 +84,22 @@ struct __attribute__((aligned(16))) Smem {
   double B[N];
 };
 
+// Waves of a tile and their 16 x 16 parts: all along the long side, or 2 x 2.
+template <bool X, bool LONG>
+struct Waves {
+  static constexpr int WM = LONG ? (X ? 1 : 4) : 2, WN = 4 / WM, IM = T / 16 / WM, IN = T / 16 / WN;
+};
+
 // E: the tile reaches past M or N.
-template <bool X, bool AKF, bool E>
+template <bool X, bool AKF, bool E, bool LONG>
 __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, long n0,
-                                     d4 (&acc)[X ? T / 16 : T / 64][X ? T / 64 : T / 16], Smem& S) {
-  constexpr int AM = AKF ? KFAST : RFAST, BM = AKF ? RFAST : KFAST;
-  constexpr int IM = X ? T / 16 : T / 64, IN = X ? T / 64 : T / 16;
+                                     d4 (&acc)[Waves<X, LONG>::IM][Waves<X, LONG>::IN], Smem& S) {
+  using W = Waves<X, LONG>;
+  constexpr int AM = AKF ? KFAST : RFAST, BM = AKF ? RFAST : KFAST, IM = W::IM, IN = W::IN;
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // thread-index arithmetic stays inside the item (not hoisted into the claim loop)
   const int lane = tid & 63, wave = tid >> 6;
-  const int wm = X ? 0 : wave * (T / 4), wn = X ? wave * (T / 4) : 0;
+  const int wm = wave / W::WN * (IM * 16), wn = wave % W::WN * (IN * 16);
   const int nv = (X ? ma : nb) / 16 + 1;  // 16-row parts inside the matrix
   const long K = t.K;
   const double al = t.alpha;
@@ -132,7 +138,7 @@ __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, lo
       for (int u = 0; u < IN; ++u) b[u] = SB.at(wn + u * 16 + lr, kk * 4 + lk);
 #pragma unroll
       for (int i = 0; i < (X ? IM : IN); ++i) {
-        if (E && i >= nv) break;
+        if (E && LONG && i >= nv) break;
 #pragma unroll
         for (int j = 0; j < (X ? IN : IM); ++j) {
           d4& c = X ? acc[i][j] : acc[j][i];
@@ -146,23 +152,24 @@ __device__ __forceinline__ void term(const DTerm& t, int ma, int nb, long m0, lo
 // Four terms, the first two read with A along k (X) or along m (!X), the
 // other two the other way; the sequence is static so the accumulators stay
 // in registers from term to term.
-template <bool X, bool E>
+template <bool X, bool E, bool LONG>
 __device__ __forceinline__ void tile4(const DMulti& p, long m0, long n0, Smem& S) {
-  constexpr int IM = X ? T / 16 : T / 64, IN = X ? T / 64 : T / 16;
+  using W = Waves<X, LONG>;
+  constexpr int IM = W::IM, IN = W::IN;
   d4 acc[IM][IN];
 #pragma unroll
   for (int i = 0; i < IM; ++i)
 #pragma unroll
     for (int j = 0; j < IN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   const int ma = (int)min((long)T - 1, p.M - 1 - m0), nb = (int)min((long)T - 1, p.N - 1 - n0);
-  term<X, X, E>(p.t[0], ma, nb, m0, n0, acc, S);
-  term<X, X, E>(p.t[1], ma, nb, m0, n0, acc, S);
-  term<X, !X, E>(p.t[2], ma, nb, m0, n0, acc, S);
-  term<X, !X, E>(p.t[3], ma, nb, m0, n0, acc, S);
+  term<X, X, E, LONG>(p.t[0], ma, nb, m0, n0, acc, S);
+  term<X, X, E, LONG>(p.t[1], ma, nb, m0, n0, acc, S);
+  term<X, !X, E, LONG>(p.t[2], ma, nb, m0, n0, acc, S);
+  term<X, !X, E, LONG>(p.t[3], ma, nb, m0, n0, acc, S);
   __syncthreads();  // the next item reuses the LDS
   // D[i][j] of a 16x16 f64 MFMA tile: lane = j + 16*(i%4), element i/4.
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
-  const int wm = X ? 0 : wave * (T / 4), wn = X ? wave * (T / 4) : 0;
+  const int wm = wave / W::WN * (IM * 16), wn = wave % W::WN * (IN * 16);
   // the descriptor's fields are read once (a store through C could alias them)
   CCGPU_GLOBAL double* C = gptr(p.C);
   const long c_m = p.c_m, c_no = p.c_no;
@@ -522,14 +529,14 @@ __device__ __forceinline__ void pass_tile(const PtRun& r, long q, int ph, long t
     const bool inside = m0 + 128 <= d.M && n0 + 128 <= d.N;
     if (ph < 2) {
       if (inside)
-        dt::tile4<true, false>(d,m0, n0, GS);
+        dt::tile4<true, false, true>(d,m0, n0, GS);
       else
-        dt::tile4<true, true>(d,m0, n0, GS);
+        dt::tile4<true, true, true>(d,m0, n0, GS);
     } else {
       if (inside)
-        dt::tile4<false, false>(d,m0, n0, GS);
+        dt::tile4<false, false, true>(d,m0, n0, GS);
       else
-        dt::tile4<false, true>(d,m0, n0, GS);
+        dt::tile4<false, true, true>(d,m0, n0, GS);
     }
   }
 }
@@ -662,7 +669,7 @@ unsigned grid_xcd(long tiles) { return (unsigned)((tiles + 7) / 8 * 8); }
 // 1760 launches one triple at a time, 18.6 ms with 26 triples each, 16.0 with
 // the columns of G2 flat (v batches of v x v pad both sides: 470 against 400
 // us a launch) and the waves along the long side, 15.0 with 25 triples.
-template <bool X>
+template <bool X, bool LONG>
 __global__ __launch_bounds__(256, 2) void k_dtile4(const DMulti* list, long tiles_m, long tiles_n) {
   __shared__ dt::Smem S;
   const DMulti& p = list[blockIdx.y];
@@ -670,9 +677,9 @@ __global__ __launch_bounds__(256, 2) void k_dtile4(const DMulti* list, long tile
   if (!tile_xcd(blockIdx.x, gridDim.x, tiles_m, tiles_n, 1, tm, tn, z)) return;
   const long m0 = tm * dt::T, n0 = tn * dt::T;
   if (m0 + dt::T <= p.M && n0 + dt::T <= p.N)
-    dt::tile4<X, false>(p, m0, n0, S);
+    dt::tile4<X, false, LONG>(p, m0, n0, S);
   else
-    dt::tile4<X, true>(p, m0, n0, S);
+    dt::tile4<X, true, LONG>(p, m0, n0, S);
 }
 
 // The mixed passes: the 256x256 tile (W8) or the 128x128 one.
@@ -941,10 +948,13 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
           const DMulti* d = reinterpret_cast<const DMulti*>(list);
           const dim3 grid(grid_xcd(ps.tm[g] * ps.tn[g] * nb), gn);
           const int id = prof_begin(g < 2 ? "k_dtile4<true>" : "k_dtile4<false>", fg * gn, st_);
-          if (g < 2)
-            CCGPU_LAUNCH(k_dtile4<true>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
-          else
-            CCGPU_LAUNCH(k_dtile4<false>, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
+          // The waves side by side read a quarter more from LDS (2 x 2 is 3% faster at v = 256, 384 and
+          // 512): only where they leave out more than that of the 16-row parts.
+          const long parts = cdiv(v, 16), all = 8L * cdiv(v, 128);
+          const bool lng = 24 * (all - parts) >= all;
+          auto* kern = g < 2 ? (lng ? k_dtile4<true, true> : k_dtile4<true, false>)
+                             : (lng ? k_dtile4<false, true> : k_dtile4<false, false>);
+          CCGPU_LAUNCH(kern, grid, dim3(256), 0, st_, d, ps.tm[g], ps.tn[g]);
           prof_end(id, st_);
         }
       }
