@@ -529,14 +529,14 @@ __device__ __forceinline__ void pass_tile(const PtRun& r, long q, int ph, long t
     const bool inside = m0 + 128 <= d.M && n0 + 128 <= d.N;
     if (ph < 2) {
       if (inside)
-        dt::tile4<true, false, true>(d,m0, n0, GS);
+        dt::tile4<true, false, true>(d, m0, n0, GS);
       else
-        dt::tile4<true, true, true>(d,m0, n0, GS);
+        dt::tile4<true, true, true>(d, m0, n0, GS);
     } else {
       if (inside)
-        dt::tile4<false, false, true>(d,m0, n0, GS);
+        dt::tile4<false, false, true>(d, m0, n0, GS);
       else
-        dt::tile4<false, true, true>(d,m0, n0, GS);
+        dt::tile4<false, true, true>(d, m0, n0, GS);
     }
   }
 }
