@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "common.h"
+#include "chol_panel.h"
 #include "ops.h"
 
 namespace ccgpu {
@@ -43,40 +44,6 @@ __global__ void k_unpack_pairs(double* __restrict__ V, const double* __restrict_
 __global__ void k_diag(double* __restrict__ d, const double* __restrict__ V, long M) {
   for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < M; q += (long)gridDim.x * blockDim.x)
     d[q] = V[q * M + q];
-}
-
-// Largest remaining diagonal and its index (smallest index on ties), in two
-// stages so that the search spreads over the whole chip: every block of a
-// grid-stride pass writes the best (value, index) of its elements to
-// part[2 b], part[2 b + 1], and one block reduces the nb partials in a fixed
-// order (the pivot is the same as that of a sequential scan).
-__device__ __forceinline__ void better(double& bv, long& bi, double ov, long oi) {
-  if (ov > bv || (ov == bv && oi < bi)) {
-    bv = ov;
-    bi = oi;
-  }
-}
-
-// Block reduction of (bv, bi) over 256 threads into part[2 blockIdx.x ...].
-__device__ __forceinline__ void block_best(double bv, long bi, double* __restrict__ part) {
-  __shared__ double sv[4];
-  __shared__ long si[4];
-  for (int off = 32; off > 0; off >>= 1) {
-    const double ov = __shfl_down(bv, off, 64);
-    const long oi = __shfl_down(bi, off, 64);
-    better(bv, bi, ov, oi);
-  }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) {
-    sv[w] = bv;
-    si[w] = bi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int q = 1; q < (int)(blockDim.x >> 6); ++q) better(bv, bi, sv[q], si[q]);
-    part[2 * (long)blockIdx.x] = bv;
-    part[2 * (long)blockIdx.x + 1] = (double)bi;
-  }
 }
 
 // Stage 1 on its own (the first pivot, and the check at the vector limit).
@@ -120,70 +87,6 @@ __global__ __launch_bounds__(256) void k_argmax_final(const double* __restrict__
     out[0] = sv[0];
     out[1] = (double)si[0];
   }
-}
-
-// Step j of the panel that starts at vector K0: pivot p = argmax of the
-// remaining diagonal, then
-//   L[K0 + j][q] = (R[p][q] - sum_{i<j} L[K0+i][p] L[K0+i][q]) / sqrt(d_p),
-//   d[q] -= L[K0 + j][q]^2, d[p] = 0,
-// where R = V minus the vectors of earlier panels.  Stops (st[0] = 1,
-// st[1] = vectors made) once the largest diagonal is below thr.
-// Every block reduces the npart stage-1 partials of the last step (pin) to
-// the pivot by itself and writes its own of the updated diagonal to pout, so
-// a vector is one launch; a step after the stop leaves them as they are.
-// Bound by latency: the panel's elements of column p go through LDS and the
-// sum over them reads eight rows at a time.  nbas = 90, 576 steps: 11.4 us
-// and 4.1 us for the pivot before.
-__global__ __launch_bounds__(256) void k_chol_panel_col(double* __restrict__ L, double* __restrict__ d,
-                                                        const double* __restrict__ R, const double* __restrict__ pin,
-                                                        int npart, long* __restrict__ st, long M, long K0, int j,
-                                                        double thr, double* __restrict__ pout) {
-  __shared__ double cp[64], bestv[4];
-  __shared__ long besti[4];
-  if (st[0] != 0) return;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  double dp = -1.0;
-  long p = M;
-  for (int q = t; q < npart; q += 256) better(dp, p, pin[2 * q], (long)pin[2 * q + 1]);
-  for (int off = 32; off > 0; off >>= 1) {
-    const double ov = __shfl_xor(dp, off, 64);
-    const long oi = __shfl_xor(p, off, 64);
-    better(dp, p, ov, oi);
-  }
-  if (lane == 0) {
-    bestv[wave] = dp;
-    besti[wave] = p;
-  }
-  __syncthreads();
-  dp = bestv[0];
-  p = besti[0];
-  for (int q = 1; q < 4; ++q) better(dp, p, bestv[q], besti[q]);
-  if (dp < thr) {
-    if (blockIdx.x == 0 && t == 0) {
-      st[0] = 1;
-      st[1] = K0 + j;
-    }
-    return;
-  }
-  const double* Lp = L + K0 * M;
-  if (t < j) cp[t] = Lp[t * M + p];
-  __syncthreads();
-  const double rs = 1.0 / sqrt(dp);
-  double bv = -1.0;
-  long bi = M;
-  for (long q = (long)blockIdx.x * 256 + t; q < M; q += (long)gridDim.x * 256) {
-    double s = R[p * M + q];
-    const double dq0 = d[q];
-#pragma unroll 8
-    for (int i = 0; i < j; ++i) s -= cp[i] * Lp[i * M + q];
-    const double l = s * rs;
-    L[(K0 + j) * M + q] = l;
-    const double dq = (q == p) ? 0.0 : dq0 - l * l;
-    d[q] = dq;
-    better(bv, bi, dq, q);
-  }
-  block_best(bv, bi, pout);
-  if (blockIdx.x == 0 && t == 0) st[1] = K0 + j + 1;
 }
 
 // Pivot of one step of a qualified panel: the largest remaining diagonal
