@@ -73,7 +73,10 @@ class CCSD {
   void enqueue_iteration(double* report);
   double finish_iteration(double* omnm);
   // Host bookkeeping after an iteration enqueued elsewhere (graph replay).
-  void note_iteration() { ++iter_; lhtr_ready_ = false; }
+  void note_iteration() {
+    ++iter_;
+    amplitudes_changed();
+  }
   // Bytes per particle-ladder batch buffer (V+/-, Y); applies from the next
   // workspace allocation.
   void set_ladder_budget(double bytes) { ladder_budget_ = bytes; }
@@ -162,10 +165,14 @@ class CCSD {
   void ladder_y_packed(int a0, int a1, void* Y, bool y_float, long ldY);
   void mark(const char* name);
   void ensure_work();
+  // t1 or T was written: what is kept of the old amplitudes is made again when next needed
+  void amplitudes_changed() { lhtr_ready_ = pt_amps_ = false; }
   // (T) drivers: launches per group of triples of the pre-packed three-pass W
   // build and blocked energy (default); the same as one persistent kernel
   enum class PtPath { Launch = 0, Persistent = 1 };
   void pt_prepare(GemmPrec mode, PtPath path);
+  void pt_integrals(GemmPrec mode, PtPath path);
+  void pt_amplitudes();
   void pt_energy_persistent(long first, long n, long stride, double* e4, double* e5);
   void pt_energy_launches(long first, long n, long stride, double* e4, double* e5);
   void pt_descs(int i, int j, int k, int slot, unsigned char* out);
@@ -187,7 +194,7 @@ class CCSD {
   int diis_off_ = 0;  // DIIS cycle restarts after the history was released
   bool work_ = false;
   GemmPrec bulk_ = GemmPrec::F64;
-  bool pt_ready_ = false;
+  bool pt_ready_ = false, pt_amps_ = false;  // buffers and integral layouts; amplitude layouts
   std::vector<int> tri_i_, tri_j_, tri_k_;
   hipStream_t st_ = nullptr;
 

@@ -457,7 +457,7 @@ double CCSD::mp2_start() {
   CCGPU_HIPX(hipStreamSynchronize(st_));
   iter_ = 1;
   diis_off_ = 0;
-  lhtr_ready_ = false;
+  amplitudes_changed();
   reset_cycle();
   return e;
 }
@@ -563,7 +563,7 @@ void CCSD::set_amplitudes(const double* t1_host, const double* t2p_host) {
   CCGPU_HIPX(hipStreamSynchronize(st_));
   iter_ = 1;
   diis_off_ = 0;
-  lhtr_ready_ = false;
+  amplitudes_changed();
   reset_cycle();
 }
 

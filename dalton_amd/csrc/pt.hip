@@ -50,14 +50,19 @@ void CCSD::pt_release() {
   TvvoS_.release();
   ptdesc_.release();
   W32_.release();
-  pt_ready_ = false;
+  pt_ready_ = pt_amps_ = false;
 }
 
-// Integral and amplitude layouts for the triple loop (built once per call
-// sequence; the iteration workspace is released first to make room): every
-// per-triple operand pre-packed, and the W slots.
+// Integral and amplitude layouts for the triple loop (the iteration workspace
+// is released first to make room): every per-triple operand pre-packed, and the
+// W slots.  The integral layouts and the buffers are kept from call to call,
+// the amplitude layouts until the amplitudes change.
 void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
-  if (pt_ready_ && pt_mode_ == mode && pt_path_ == path) return;
+  if (!(pt_ready_ && pt_mode_ == mode && pt_path_ == path)) pt_integrals(mode, path);
+  if (!pt_amps_) pt_amplitudes();
+}
+
+void CCSD::pt_integrals(GemmPrec mode, PtPath path) {
   pt_release();
   release_work();
   const int o = dm_.o, v = dm_.v, naux = dm_.naux;
@@ -110,39 +115,22 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
     perm(Q_.p, R.p, o, o, o, v, (long)v * o * o, 1, o, (long)o * o, 1.0, 0.0, st_);
     CCGPU_HIPX(hipStreamSynchronize(st_));
   }
-  // Tvvo[i][a][b][l] = t_il^ab = T[(i,a),(l,b)]
-  perm(Tvvo_.p, T_.p, o, v, v, o, (long)v * nov, nov, 1, v, 1.0, 0.0, st_);
-  {
-    if (!mixed) {
-      // TvvoS[p][x][y][l] = Tvvo[p][y][x][l]
-      perm(TvvoS_.p, Tvvo_.p, o, v, v, o, vv * o, o, (long)v * o, 1, 1.0, 0.0, st_);
-    } else {
-      const long Kpv = bf16x3_kpad(v), Kpo = bf16x3_kpad(o), Rv = bf16x3_rpad(v), Rvv = bf16x3_rpad(vv) + 256;
-      CCGPU_REQUIRE(o <= 255 && v <= 65535, "pt: occupied or virtual space too large for the packed slices");
-      const size_t n0 = (size_t)o * o * Rv * Kpv, n1 = (size_t)o * o * Rv * Kpo, n2 = (size_t)o * Rvv * Kpo;
-      const size_t nn[4] = {n0, n1, n2, n2};
-      for (int q = 0; q < 4; ++q) {
-        ppH_[q].alloc(nn[q]);
-        ppL_[q].alloc(nn[q]);
-      }
-      // slot tails past v*v rows of the swapped -Tvvo are read by edge tiles only: keep them finite
-      for (DBuf<unsigned short>* b : {&ppH_[3], &ppL_[3]})
-        CCGPU_LAUNCH(k_zero_u16, dim3(4096), dim3(256), 0, st_, b->p, (long)b->n);
-      for (int p = 0; p < o; ++p) {
-        // T(p,q)[x][d] = t_pq^{xd} for every q: [(p,q)][x][d]
-        const size_t ot = (size_t)p * o * Rv * Kpv;
-        bf16x3_pack(T_.p + (long)p * v * nov, v, v, nov, 1, v, o, Rv, Kpv, 1.0f, ppH_[0].p + ot, ppL_[0].p + ot,
-                    st_);
-        // [x][c][l] = -Tvvo_p[c][x][l]
-        const size_t os = (size_t)p * Rvv * Kpo;
-        bf16x3_pack(Tvvo_.p + (long)p * vv * o, v, o, (long)v * o, 1, o, v, v, Kpo, -1.0f, ppH_[3].p + os,
-                    ppL_[3].p + os, st_);
-      }
-      // Q_rq[z][l] = (zr|lq) for every (r,q)
-      bf16x3_pack(Q_.p, v, o, 1, v, (long)o * v, o * o, Rv, Kpo, 1.0f, ppH_[1].p, ppL_[1].p, st_);
-      // [(x,y)][l] = -Tvvo_p[x][y][l]
-      bf16x3_pack(Tvvo_.p, vv, o, o, 1, vv * o, o, Rvv, Kpo, -1.0f, ppH_[2].p, ppL_[2].p, st_);
+  if (mixed) {
+    const long Kpv = bf16x3_kpad(v), Kpo = bf16x3_kpad(o), Rv = bf16x3_rpad(v), Rvv = bf16x3_rpad(vv) + 256;
+    CCGPU_REQUIRE(o <= 255 && v <= 65535, "pt: occupied or virtual space too large for the packed slices");
+    const size_t n0 = (size_t)o * o * Rv * Kpv, n1 = (size_t)o * o * Rv * Kpo, n2 = (size_t)o * Rvv * Kpo;
+    const size_t nn[4] = {n0, n1, n2, n2};
+    for (int q = 0; q < 4; ++q) {
+      ppH_[q].alloc(nn[q]);
+      ppL_[q].alloc(nn[q]);
     }
+    // slot tails past v*v rows of the swapped -Tvvo are read by edge tiles only: keep them finite
+    for (DBuf<unsigned short>* b : {&ppH_[3], &ppL_[3]})
+      CCGPU_LAUNCH(k_zero_u16, dim3(4096), dim3(256), 0, st_, b->p, (long)b->n);
+    // Q_rq[z][l] = (zr|lq) for every (r,q)
+    bf16x3_pack(Q_.p, v, o, 1, v, (long)o * v, o * o, Rv, Kpo, 1.0f, ppH_[1].p, ppL_[1].p, st_);
+  }
+  {
     // canonical 8x8x8 blocks A <= B <= C of the virtual cube, A | B << 10 | C << 20
     const long nb = cdiv(v, 8);
     CCGPU_REQUIRE(nb <= 1023, "pt: virtual space too large for the block table");
@@ -168,6 +156,31 @@ void CCSD::pt_prepare(GemmPrec mode, PtPath path) {
   pt_mode_ = mode;
   pt_path_ = path;
   pt_ready_ = true;
+}
+
+void CCSD::pt_amplitudes() {
+  const int o = dm_.o, v = dm_.v;
+  const long nov = dm_.nov, vv = (long)v * v;
+  // Tvvo[i][a][b][l] = t_il^ab = T[(i,a),(l,b)]
+  perm(Tvvo_.p, T_.p, o, v, v, o, (long)v * nov, nov, 1, v, 1.0, 0.0, st_);
+  if (pt_mode_ != GemmPrec::BF16X3) {
+    // TvvoS[p][x][y][l] = Tvvo[p][y][x][l]
+    perm(TvvoS_.p, Tvvo_.p, o, v, v, o, vv * o, o, (long)v * o, 1, 1.0, 0.0, st_);
+  } else {
+    const long Kpv = bf16x3_kpad(v), Kpo = bf16x3_kpad(o), Rv = bf16x3_rpad(v), Rvv = bf16x3_rpad(vv) + 256;
+    for (int p = 0; p < o; ++p) {
+      // T(p,q)[x][d] = t_pq^{xd} for every q: [(p,q)][x][d]
+      const size_t ot = (size_t)p * o * Rv * Kpv;
+      bf16x3_pack(T_.p + (long)p * v * nov, v, v, nov, 1, v, o, Rv, Kpv, 1.0f, ppH_[0].p + ot, ppL_[0].p + ot, st_);
+      // [x][c][l] = -Tvvo_p[c][x][l]
+      const size_t os = (size_t)p * Rvv * Kpo;
+      bf16x3_pack(Tvvo_.p + (long)p * vv * o, v, o, (long)v * o, 1, o, v, v, Kpo, -1.0f, ppH_[3].p + os,
+                  ppL_[3].p + os, st_);
+    }
+    // [(x,y)][l] = -Tvvo_p[x][y][l]
+    bf16x3_pack(Tvvo_.p, vv, o, o, 1, vv * o, o, Rvv, Kpo, -1.0f, ppH_[2].p, ppL_[2].p, st_);
+  }
+  pt_amps_ = true;
 }
 
 // (T) driver from CCGPU_PT_PATH: "launch" (default: launches of the pass
