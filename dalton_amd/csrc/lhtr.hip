@@ -99,7 +99,7 @@ void CCSD::lhtr_ladder(const double* Xb) {
     ladder_gather(S_.p, S_.p + ns, Xb, a0, a1, o, v, st_);
     bulk(npo, npv, rows, 0.5, S_.p, 1, npo, V_.p, npv, 1, 1.0, taub_.p, npv, 1, 2, ns, nv, nt);
     bulk(rows, npv, npo, 0.5, S_.p, npo, 1, tau_.p, npv, 1, 0.0, V_.p, npv, 1, 2, ns, nt, nv);
-    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::BF16X3 ? 512 : 64);
+    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::F64 ? 64 : 512);
     // Entries with b < a: zeros where the sums below read them, the blocks of
     // a strip by itself and of its K padding (v = 192: 1.8 ms of all of Y).
     for (size_t q = 0; q + 1 < sa.size(); ++q) {
@@ -110,8 +110,11 @@ void CCSD::lhtr_ladder(const double* Xb) {
     // Y_bar is zero for b < a: the strip [s0, s1) of a sums over b >= s0, that
     // of b over a < s1.  Both sums start and end at multiples of 64, the K
     // padding of the packed operands, so they add the same terms in the same
-    // groups as the whole sums do.  K is the long side here and is not split in
-    // BF16x3: there a strip keeps one wave of output tiles (512).
+    // groups as the whole sums do.  K is the long side here and only the FP64
+    // GEMM splits it: the others keep one wave of output tiles a strip (512).
+    // FP32, one left transformation at o=7 v=171 / o=24 v=192 / o=32 v=256: with
+    // 64 tiles a strip 56.3 / 100.4 / 384 ms, 512 40.1 / 85.4 / 302, no strips
+    // 43.8 / 92.3 / 306.
     double* Bbb = Bvvb_.p + (long)a0 * v;
     for (size_t q = 0; q + 1 < sa.size(); ++q) {
       const long r0 = (long)(sa[q] - a0) * v, nr = (long)(sa[q + 1] - sa[q]) * v, k0 = r0 / 64 * 64;
