@@ -3,6 +3,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -481,7 +482,14 @@ int dgemm_impl(ccgpu::GemmPrec prec, char transa, char transb, int m, int n, int
     CCGPU_HIPX(hipMemcpy(B.p, b, nb * sizeof(double), hipMemcpyHostToDevice));
     CCGPU_HIPX(hipMemcpy(C.p, c, nc * sizeof(double), hipMemcpyHostToDevice));
     d.A = A.p; d.B = B.p; d.C = C.p;
-    ccgpu::gemm(d, prec, nullptr);
+    {
+      // Calls of several threads share the null stream and its scratch (packed
+      // operands, partial sums of a split K): the launches of one product stay
+      // together on the stream, and the scratch does not grow between them.
+      static std::mutex mu;
+      std::lock_guard<std::mutex> lk(mu);
+      ccgpu::gemm(d, prec, nullptr);
+    }
     CCGPU_HIPX(hipDeviceSynchronize());
     CCGPU_HIPX(hipMemcpy(c, C.p, nc * sizeof(double), hipMemcpyDeviceToHost));
   });
