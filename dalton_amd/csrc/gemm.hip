@@ -268,6 +268,8 @@ struct F64Cfg {
   int nz = 1;
 };
 
+constexpr long kMaxTiles = 1L << 24;
+
 int step_k(int T) { return T == 32 ? Step<32>::TK : Step<64>::TK; }
 
 // Estimated time (microseconds) of block tile T with K in nz chunks.  kRes
@@ -301,6 +303,9 @@ F64Cfg plan_f64(const GemmDesc& d, int only = 0) {
   double bt = 1e300;
   for (int T : {128, 64, 32}) {
     if (only && T != only) continue;
+    // a grid holds 2^24 blocks of 256 threads: long thin products past that
+    // with the small tiles (540e6 x 1, K = 17) keep the 128 one
+    if (T != 128 && (long)cdiv(d.M, T) * cdiv(d.N, T) >= kMaxTiles) continue;
     // chunks of at least two K steps; partials of at most 4 GB
     const double room = 4.0e9 / (8.0 * d.batch * (double)d.M * d.N);
     const long kmax = std::max<long>(1, std::min<long>(d.K / (2 * (step_k(T))), (long)std::min(room, 1e6)));
@@ -383,7 +388,7 @@ void run_f64(const GemmDesc& d, const F64Cfg& cfg, int am, int bm, hipStream_t s
     }
   }
   CCGPU_REQUIRE((long)nz * d.batch <= 65535, "gemm: too many batches");
-  CCGPU_REQUIRE(tiles < (1L << 24), "gemm: too many tiles");
+  CCGPU_REQUIRE(tiles < kMaxTiles, "gemm: too many tiles");
   CCGPU_REQUIRE(!two_level(d) || d.K < (1L << 32), "gemm: two-level K too long");
   dim3 grid((unsigned)tiles, 1, (unsigned)(nz * d.batch));
 #define CCGPU_F64_LAUNCH(TT)                                                   \
