@@ -180,8 +180,6 @@ struct BMulti {
 long bf16x3_kpad(long K);
 long bf16x3_kcols(long K);  // K padded to the 32 columns of a matrix instruction (BTerm::Kc)
 long bf16x3_rpad(long R);
-// Whether the cost model takes the 256 x 256 tile for batch products of M x N.
-bool bf16x3_large_tile(long M, long N, long batch);
 // Pack scale * A(r,k) (element at src + r*s_r + koff(k) + b*s_b) into hi/lo.
 void bf16x3_pack(const double* src, long rows, long K, long s_r, long s_k, long s_b, int batch, long Rp, long Kp,
                  float scale, unsigned short* hi, unsigned short* lo, hipStream_t s, long s_ko = 0, long Kin = 0);

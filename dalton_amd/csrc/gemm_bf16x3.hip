@@ -323,6 +323,17 @@ int tune(const BMulti& p, int batch, hipStream_t s) {
   return kern;
 }
 
+// Without a measurement: the 256x256 tile computes M x N padded to 256,
+// the 128x128 one ceil(M/128) x ceil(N/128) tiles, at 361 against 307
+// TFLOP/s measured on square products; the 256 tile also needs a wave of
+// tiles over the CUs to be worth its larger grain.
+bool large_tile(long M, long N, long batch) {
+  const double a256 = (double)bf16x3_rpad(M) * (double)bf16x3_rpad(N);
+  const double a128 = (double)cdiv(M, TM) * TM * (double)cdiv(N, TN) * TN;
+  const long t256 = (bf16x3_rpad(M) / DT) * (bf16x3_rpad(N) / DT) * batch;
+  return a256 * 307.0 <= a128 * 361.0 && t256 >= 256;
+}
+
 template <typename OutT>
 void launch_multi(BMulti p, int batch, hipStream_t s) {
   p.gm = group_m();
@@ -349,7 +360,7 @@ void launch_multi(BMulti p, int batch, hipStream_t s) {
         ++tu.timed;
       } else {
         // without a measurement: 64x64 tiles below one 128x128 tile per CU
-        kern = bf16x3_large_tile(p.M, p.N, batch) ? kT256 : (tiles128(p, batch) < 256 ? kT64 : kT128);
+        kern = large_tile(p.M, p.N, batch) ? kT256 : (tiles128(p, batch) < 256 ? kT64 : kT128);
       }
     }
   }
@@ -366,18 +377,6 @@ long bf16x3_kcols(long K) { return std::max<long>(32, (K + 31) / 32 * 32); }
 long bf16x3_rpad(long R) {
   const long t = variant() != 0 ? DT : TM;  // rows padded to the block tile in use
   return (R + t - 1) / t * t;
-}
-
-// Without a measurement: the 256x256 tile computes M x N padded to 256,
-// the 128x128 one ceil(M/128) x ceil(N/128) tiles, at 361 against 307
-// TFLOP/s measured on square products; the 256 tile also needs a wave of
-// tiles over the CUs to be worth its larger grain.
-bool bf16x3_large_tile(long M, long N, long batch) {
-  if (variant() != 1) return false;  // operands padded to 128 rows only
-  const double a256 = (double)bf16x3_rpad(M) * (double)bf16x3_rpad(N);
-  const double a128 = (double)cdiv(M, TM) * TM * (double)cdiv(N, TN) * TN;
-  const long t256 = (bf16x3_rpad(M) / DT) * (bf16x3_rpad(N) / DT) * batch;
-  return a256 * 307.0 <= a128 * 361.0 && t256 >= 256;
 }
 
 void bf16x3_pack(const double* src, long rows, long K, long s_r, long s_k, long s_b, int batch, long Rp, long Kp,

@@ -868,6 +868,19 @@ EArgs energy_args(const int* ctab, const double* J, const double* t1, const doub
 }
 }  // namespace
 
+namespace {
+// The 256 tile where its whole rounds of blocks (one a CU) take no longer than
+// those of the 128 tile (two a CU), at 361 against 307 TFLOP/s in full rounds.
+// A launch of few triples is a round or two, where padding to 256 rows and a
+// part-filled chip matter less than a second round: with the area rule of the
+// BF16x3 GEMM (and a full round of 256 tiles) one triple took 261 us at v = 200
+// and 343 at v = 230, now 214 and 287; full groups take the same tile as before.
+bool pt_large_tile(long t256, long t128) {
+  if (bf16x3_rpad(1) != bf3w8::DT) return false;  // operands padded to 128 rows only
+  return cdiv(t256, 256) * 4.0 / 361.0 <= cdiv(t128, 512) * 2.0 / 307.0;
+}
+}  // namespace
+
 // Triples per launch of the W passes: just below four waves of blocks over the
 // CUs (two 128 x 128 blocks or one 256 x 256 block per CU; just above, a fifth
 // one is nearly empty: v=101 26 triples 16.0 ms the full list, 25 15.0), at
@@ -902,13 +915,17 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
   constexpr long kRange = 4096;  // triples whose descriptors are held at once
   const long nr = std::min(n, kRange);
   const size_t dsz = pt_desc_bytes();
-  if (n > 0) {
-    ptdesc_.ensure(3 * nr * dsz);
-    pttri_.ensure(3 * (size_t)nr);
-    check_span(pttri_.p, 0, 3 * nr - 1, sizeof(int), "pt triples");
-  }
-  std::vector<unsigned char> hd(3 * nr * dsz), one(3 * dsz);
-  std::vector<int> ht(3 * nr);
+  const size_t dend = 3 * nr * dsz;  // the indices follow the descriptors: one copy
+  if (n > 0) ptdesc_.ensure(dend + 3 * nr * sizeof(int));
+  std::vector<unsigned char> hd(dend + 3 * nr * sizeof(int)), one(3 * dsz);
+  int* const ht = reinterpret_cast<int*>(hd.data() + dend);
+  const int* const tri = reinterpret_cast<const int*>(ptdesc_.p + dend);
+  struct Drain {  // an error on the way leaves with the copy done
+    hipStream_t s;
+    ~Drain() {
+      if (!dryrun()) (void)hipStreamSynchronize(s);
+    }
+  } drain{st_};
   for (long r0 = 0; r0 < n; r0 += kRange) {
     const long nq = std::min(kRange, n - r0);
     for (long q = 0; q < nq; ++q) {
@@ -920,11 +937,10 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
       pt_descs(i, j, k, (int)(q % ng), one.data());
       for (int g = 0; g < 3; ++g) std::memcpy(hd.data() + (g * nr + q) * dsz, one.data() + g * dsz, dsz);
     }
-    // the previous range's launches precede the copies on the stream, and the
-    // host arrays are refilled only after the copies have left them
+    // the previous range's launches precede the copy on the stream, and the
+    // host array is refilled only after the copy has left it
     CCGPU_HIPX(hipMemcpyAsync(ptdesc_.p, hd.data(), hd.size(), hipMemcpyHostToDevice, st_));
-    CCGPU_HIPX(hipMemcpyAsync(pttri_.p, ht.data(), 3 * nq * sizeof(int), hipMemcpyHostToDevice, st_));
-    CCGPU_HIPX(hipStreamSynchronize(st_));
+    if (r0 + nq < n) CCGPU_HIPX(hipStreamSynchronize(st_));
     for (long q0 = 0; q0 < nq; q0 += ng) {
       const unsigned gn = (unsigned)std::min(ng, nq - q0);
       for (int g = 0; g < 3; ++g) {
@@ -933,10 +949,8 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
         CCGPU_REQUIRE(ps.tm[g] * ps.tn[g] * ps.batch[g] < (1L << 22), "pt: grid too large");
         if (mixed) {
           const BMulti* d = reinterpret_cast<const BMulti*>(list);
-          // the 256 tile where padding to 256 rows does not cost more than its higher rate gives
-          // (cost model of the BF16x3 GEMM) and the group fills the CUs with it
           const long tm1 = cdiv(ps.M[g], 128), tn1 = cdiv(ps.N[g], 128);
-          const bool w8 = bf16x3_large_tile(ps.M[g], ps.N[g], (long)gn * nb);
+          const bool w8 = pt_large_tile(ps.tm[g] * ps.tn[g] * nb * gn, tm1 * tn1 * nb * gn);
           const int id = prof_begin("k_gemm_bf16x3", fg * gn, st_);
           if (w8)
             CCGPU_LAUNCH(k_btile4<true>, dim3(grid_xcd(ps.tm[g] * ps.tn[g] * nb), gn), dim3(512), 0, st_, d, ps.tm[g],
@@ -961,10 +975,10 @@ void CCSD::pt_energy_launches(long first, long n, long stride, double* e4, doubl
       const int id = prof_begin(mixed ? "k_pt_energy_blocked<float>" : "k_pt_energy_blocked<double>", 0.0, st_);
       const dim3 egrid((unsigned)ea.nE, gn);
       if (mixed)
-        CCGPU_LAUNCH(k_pt_energy_blocked<float>, egrid, dim3(256), 0, st_, ea, W32_.p, vvv, pttri_.p + 3 * q0,
+        CCGPU_LAUNCH(k_pt_energy_blocked<float>, egrid, dim3(256), 0, st_, ea, W32_.p, vvv, tri + 3 * q0,
                      ptpart_.p);
       else
-        CCGPU_LAUNCH(k_pt_energy_blocked<double>, egrid, dim3(256), 0, st_, ea, Wt_.p, vvv, pttri_.p + 3 * q0,
+        CCGPU_LAUNCH(k_pt_energy_blocked<double>, egrid, dim3(256), 0, st_, ea, Wt_.p, vvv, tri + 3 * q0,
                      ptpart_.p);
       prof_end(id, st_);
       CCGPU_LAUNCH(k_reduce_pairs, dim3(gn), dim3(256), 0, st_, ptpart_.p, ea.nE, etrip_.p + 2 * (r0 + q0));
