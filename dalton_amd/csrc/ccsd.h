@@ -160,8 +160,12 @@ class CCSD {
   void ladder(const double* T, double* Om);
   void ladder_mixed(double* Om);
   std::vector<int> ladder_strips(int a0, int a1, long rows, long tiles) const;
+  std::vector<int> adjoint_strips(int a0, int a1, GemmPrec prec) const;
   void ladder_y(int a0, int a1);
   void ladder_pack_b();
+  // rows of the largest a-batch; elements of each packed operand (hi or lo)
+  long ladder_maxrows() const;
+  size_t ladder_b_size() const;
   void ladder_y_packed(int a0, int a1, void* Y, bool y_float, long ldY);
   void mark(const char* name);
   void ensure_work();
@@ -182,7 +186,10 @@ class CCSD {
   void ensure_diis();
   void reset_cycle();
   void ensure_lhtr();
-  void lhtr_prepare();
+  void lhtr_prepare(GemmPrec transforms, double extra = 0.0);
+  ScratchNeed lhtr_scratch(GemmPrec transforms) const;
+  void lhtr_scratch(ScratchNeed& n, GemmPrec prec) const;
+  double lhtr_need(GemmPrec transforms) const;
   void lhtr_apply(const double* l1, double* Xb, double* rho1, double* rho2s);
   void lhtr_ladder(const double* Xb);
   void lhtr_packed(const double* x, double* y);
@@ -238,6 +245,7 @@ class CCSD {
   // left transformation: cotangents (suffix b) of the residual's intermediates
   int lam_counts_[2] = {0, 0};
   bool lhtr_ready_ = false;
+  unsigned lhtr_room_ = 0;  // bit 3 * forward + transformation arithmetic: room was made for its buffers
   GemmPrec lhtr_prec_ = GemmPrec::F64;
   DBuf<double> Tb_, Ub_, Txb_, Db_, Btb_, Bvvb_, Boob_, BvoTb_, Zb_, Wb_, Fb_, E1b_, E2b_, Jdb_, Gamb_, G1b_,
       taub_, vecb_;

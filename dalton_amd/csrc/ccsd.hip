@@ -199,6 +199,7 @@ void CCSD::release_work() {
   for (DBuf<unsigned short>* b : {&lpBh_, &lpBl_, &lpTh_, &lpTl_, &lpVh_, &lpVl_}) b->release();
   work_ = false;
   lhtr_ready_ = false;
+  lhtr_room_ = 0;
   diis_off_ = iter_ > 0 ? iter_ - 1 : 0;  // the DIIS history is gone: restart the cycle
 }
 
@@ -214,7 +215,10 @@ void CCSD::side_stream() {
 }
 
 CCSD::~CCSD() {
-  if (dryrun()) return;
+  if (dryrun()) {
+    release_scratch(st_);
+    return;
+  }
   if (cst_) {
     (void)hipStreamSynchronize(cst_);
     for (int q = 0; q < 2; ++q) {
@@ -306,13 +310,26 @@ void CCSD::ladder_y(int a0, int a1) {
   }
 }
 
+long CCSD::ladder_maxrows() const {
+  long maxr = 0;
+  for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
+    long rows = 0;
+    for (int a = lad_batches_[bi]; a < lad_batches_[bi + 1]; ++a) rows += dm_.v - a;
+    maxr = std::max(maxr, rows);
+  }
+  return maxr;
+}
+
+// every batch reads rows up to a0*v + rpad(...) < vv + (row padding)
+size_t CCSD::ladder_b_size() const {
+  return (size_t)bf16x3_rpad((long)dm_.v * dm_.v + bf16x3_rpad(1) - 1) * bf16x3_kpad(dm_.naux);
+}
+
 // Bvv split into bf16 hi/lo, a row per (a,c), K = naux: once per ladder.
 void CCSD::ladder_pack_b() {
-  const long vv = (long)dm_.v * dm_.v, naux = dm_.naux;
-  // every batch reads rows up to a0*v + rpad(...) < vv + (row padding)
-  const long RpB = bf16x3_rpad(vv + bf16x3_rpad(1) - 1), KpB = bf16x3_kpad(naux);
-  lpBh_.ensure((size_t)RpB * KpB);
-  lpBl_.ensure((size_t)RpB * KpB);
+  const long vv = (long)dm_.v * dm_.v, naux = dm_.naux, KpB = bf16x3_kpad(naux), RpB = ladder_b_size() / KpB;
+  lpBh_.ensure(ladder_b_size());
+  lpBl_.ensure(ladder_b_size());
   bf16x3_pack(Bvv_.p, vv, naux, 1, vv, 0, 1, RpB, KpB, 1.0f, lpBh_.p, lpBl_.p, st_);
 }
 
@@ -334,14 +351,8 @@ void CCSD::ladder_y_packed(int a0, int a1, void* Y, bool y_float, long ldY) {
 // Y in FP32 straight from the packed factor, and V+/- goes from Y directly
 // into the packed operand of one batched (+ and -) S GEMM.
 void CCSD::ladder_mixed(double* Om) {
-  const int o = dm_.o, v = dm_.v, naux = dm_.naux;
-  const long vv = (long)v * v, npo = dm_.npo, npv = dm_.npv;
-  long maxr = 0;
-  for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
-    long rows = 0;
-    for (int a = lad_batches_[bi]; a < lad_batches_[bi + 1]; ++a) rows += v - a;
-    maxr = std::max(maxr, rows);
-  }
+  const int o = dm_.o, v = dm_.v;
+  const long npo = dm_.npo, npv = dm_.npv, maxr = ladder_maxrows();
   const long RpT = bf16x3_rpad(npo), KpT = bf16x3_kpad(npv);
   const long RpV = bf16x3_rpad(maxr);
   lpTh_.ensure((size_t)2 * RpT * KpT);

@@ -35,7 +35,9 @@ struct Error : std::runtime_error {
 // layout-kernel launch still has its address span checked against the
 // allocation it points into.  This lets the whole host orchestration be
 // bounds-checked on a machine without a GPU, at any problem size.
+// CCGPU_DRYRUN_MB sets the size of the device memory that it allocates from.
 bool& dryrun();
+size_t device_free();  // bytes of device memory not allocated
 void* dry_alloc(size_t bytes);
 void register_alloc(const void* p, size_t bytes);
 void unregister_alloc(const void* p);
@@ -129,6 +131,14 @@ T* grow_scratch(DBuf<T>& b, size_t n, hipStream_t s) {
   return b.p;
 }
 
+// Elements of a stream's scratch that products need (gemm_scratch takes the
+// largest of several); what they still have to allocate, and allocating it.
+struct ScratchNeed {
+  size_t splitk = 0, pack[4] = {0, 0, 0, 0};
+};
+size_t scratch_growth(const ScratchNeed& n, hipStream_t s);  // bytes
+void reserve_scratch(const ScratchNeed& n, hipStream_t s);
+
 // ------------------------------------------------------------------ GEMM API
 // C(m,n) = alpha * sum_k A(m,k) B(k,n) + beta * C(m,n), all operands given by
 // element strides, optionally batched (blockIdx.z) and with a two-level K
@@ -150,6 +160,8 @@ struct GemmDesc {
 enum class GemmPrec { F64 = 0, F32 = 1, BF16X3 = 2 };
 
 void gemm(const GemmDesc& d, GemmPrec prec, hipStream_t s);
+// Raises n to what a product of this shape needs (FP64: with its planned split of K).
+void gemm_scratch(ScratchNeed& n, long M, long N, long K, int batch, double beta, GemmPrec prec);
 
 // FP64 GEMM autotuner.  While enabled, the first call of every new shape
 // class (M, N, K, two-level K, batch, operand orders) with fewer than 1024

@@ -449,8 +449,8 @@ F64Cfg tune_f64(const GemmDesc& d, int am, int bm, hipStream_t s) {
 
 namespace {
 // plan_f64 through a small direct-mapped table per thread (the plan depends
-// on the key and beta alone, and takes about as long as a launch).
-F64Cfg planned(const GemmDesc& d, const ShapeKey& key) {
+// on the sizes and beta alone, and takes about as long as a launch).
+F64Cfg planned(const GemmDesc& d) {
   struct Entry {
     ShapeKey key{};
     bool acc = false, set = false;
@@ -458,6 +458,7 @@ F64Cfg planned(const GemmDesc& d, const ShapeKey& key) {
   };
   static thread_local Entry table[256];
   const bool acc = d.beta != 0.0;
+  const ShapeKey key{d.M, d.N, d.K, two_level(d) ? d.Kin : 0, d.batch, 0, 0};
   unsigned long h = 1469598103934665603ul;
   for (long x : {key.M, key.N, key.K, key.Kin, (long)key.batch, acc ? 1L : 0L}) h = (h ^ (unsigned long)x) * 1099511628211ul;
   Entry& e = table[(h ^ (h >> 32)) & 255];
@@ -497,12 +498,28 @@ void gemm_f64(const GemmDesc& d, hipStream_t s) {
     std::lock_guard<std::mutex> lk(tu.mu);
     tu.best[key] = cfg;
   }
-  if (!found) cfg = planned(d, key);
+  if (!found) cfg = planned(d);
   run_f64(d, cfg, am, bm, s);
 }
 
 void gemm_bf16x3(const GemmDesc& d, hipStream_t s);
 void gemm_f32(const GemmDesc& d, hipStream_t s);
+void bf16x3_scratch(ScratchNeed& n, long M, long N, long K, int batch);
+void f32_scratch(ScratchNeed& n, long M, long N, long K, int batch);
+
+void gemm_scratch(ScratchNeed& n, long M, long N, long K, int batch, double beta, GemmPrec prec) {
+  if (M <= 0 || N <= 0 || batch <= 0) return;
+  if (prec == GemmPrec::BF16X3) return bf16x3_scratch(n, M, N, K, batch);
+  if (prec == GemmPrec::F32) return f32_scratch(n, M, N, K, batch);
+  GemmDesc d;
+  d.M = M;
+  d.N = N;
+  d.K = K;
+  d.batch = std::min(batch, 65535);
+  d.beta = beta;
+  const int nz = planned(d).nz;  // (asked for again by the product itself)
+  if (nz > 1) n.splitk = std::max(n.splitk, (size_t)nz * d.batch * M * N);
+}
 
 void gemm(const GemmDesc& d, GemmPrec prec, hipStream_t s) {
   if (prec == GemmPrec::BF16X3) {

@@ -457,6 +457,13 @@ void bf16x3_run(const BMulti& p, int batch, bool c_float, double flops, hipStrea
 
 void check_gemm(const GemmDesc& d, size_t esz);
 
+// The packed operands of gemm_bf16x3, hi and lo of A and of B.
+void bf16x3_scratch(ScratchNeed& n, long M, long N, long K, int batch) {
+  const long Kp = bf16x3_kpad(K);
+  const size_t na = (size_t)batch * bf16x3_rpad(M) * Kp, nb = (size_t)batch * bf16x3_rpad(N) * Kp;
+  for (int q = 0; q < 4; ++q) n.pack[q] = std::max(n.pack[q], q < 2 ? na : nb);
+}
+
 void gemm_bf16x3(const GemmDesc& d, hipStream_t s) {
   if (d.M <= 0 || d.N <= 0 || d.batch <= 0) return;
   check_gemm(d, sizeof(double));

@@ -218,6 +218,13 @@ void pack_f32(const double* src, long rows, long K, long s_r, long s_k, long s_b
 
 void check_gemm(const GemmDesc& d, size_t esz);
 
+// The packed operands of gemm_f32 (a float in two of the bf16 buffer's elements).
+void f32_scratch(ScratchNeed& n, long M, long N, long K, int batch) {
+  const long Kp = f32_kpad(K);
+  n.pack[0] = std::max(n.pack[0], (size_t)2 * batch * f32_rpad(M) * Kp);
+  n.pack[2] = std::max(n.pack[2], (size_t)2 * batch * f32_rpad(N) * Kp);
+}
+
 void gemm_f32(const GemmDesc& d, hipStream_t s) {
   if (d.M <= 0 || d.N <= 0 || d.batch <= 0) return;
   check_gemm(d, sizeof(double));

@@ -162,15 +162,18 @@ int CCSD::lambda_solve(double thr, int maxit, int maxred, double* l1, double* l2
   // forward intermediates in FP64 for both modes: the BF16x3 transforms of
   // the refinement use them with BF16x3 bulk products
   set_precision(GemmPrec::F64);
-  lhtr_prepare();
-  ensure_lhtr();
   // space for eta, r, w, lambda, the FP64 residual, the correction and 2 x
   // maxred vectors, within the free memory
   constexpr long kFixed = 6;
-  if (!dryrun()) {
-    size_t fr = 0, tot = 0;
-    CCGPU_HIP(hipMemGetInfo(&fr, &tot));
-    const long fit = (long)((0.9 * (double)fr / (8.0 * (double)n) - kFixed) / 2.0);
+  lhtr_prepare(user, (kFixed + 2.0 * maxred) * 8.0 * n / 0.9);
+  {
+    // what the transformations allocate comes before the space that takes the rest
+    reserve_scratch(lhtr_scratch(user), st_);
+    if (user == GemmPrec::BF16X3) {
+      lpBh_.ensure(ladder_b_size());
+      lpBl_.ensure(ladder_b_size());
+    }
+    const long fit = (long)((0.9 * (double)device_free() / (8.0 * (double)n) - kFixed) / 2.0);
     maxred = (int)std::min<long>(maxred, fit);
     CCGPU_REQUIRE(maxred >= 2, "ccgpu_lambda_solve: not enough device memory for the reduced space");
   }
@@ -319,8 +322,7 @@ void CCSD::onedens_host(const double* l1, const double* l2p, double* D, bool dal
   CCGPU_REQUIRE(iter_ >= 1, "ccgpu_onedens: no amplitudes (run the CCSD iterations or set amplitudes first)");
   const long n = dm_.ntamp, nov = dm_.nov, N = dm_.N, NN = N * N;
   const int o = dm_.o, v = dm_.v;
-  lhtr_prepare();
-  ensure_lhtr();
+  lhtr_prepare(bulk_, 16.0 * n + 8.0 * NN);
   DBuf<double> x((size_t)2 * n), Dd((size_t)NN);
   CCGPU_HIPX(hipMemcpyAsync(x.p, l1, nov * sizeof(double), hipMemcpyHostToDevice, st_));
   CCGPU_HIPX(hipMemcpyAsync(x.p + nov, l2p, (n - nov) * sizeof(double), hipMemcpyHostToDevice, st_));

@@ -46,27 +46,99 @@ void CCSD::ensure_lhtr() {
   vecb_.alloc(2 * nov);
 }
 
-// Forward pass at the current amplitudes: leaves Bt, Bvv, Boo, BvoT, F, h~,
-// Jd, Tx, U, C, D, Gam, E1, E2, Z, W, F_kc and tau+/- on the device.
-void CCSD::lhtr_prepare() {
-  if (lhtr_ready_ && lhtr_prec_ == bulk_) return;
-  if (diisS_.p && !Tb_.p) {
-    // The DIIS history stays when the cotangent buffers and the trial-vector
-    // staging fit beside it (with 4 GB to spare); otherwise it is released,
-    // as the converged ground state needs none (a later iterate restarts
-    // the DIIS cycle).
-    const int o = dm_.o, v = dm_.v, naux = dm_.naux;
-    const double N = (double)dm_.N, nov = (double)dm_.nov, oo = (double)o * o;
-    const double need = 8.0 * (4.0 * dm_.nov2 + naux * (N * N + (double)v * v + oo + 2.0 * nov + 1.0) +
-                               oo * nov + N * N + (double)v * v + oo + 2.0 * oo * oo +
-                               2.0 * dm_.npo * dm_.npv + 2.0 * nov + 4.0 * dm_.ntamp) + 4.0e9;
-    size_t fr = 0, tot = 0;
-    if (!dryrun()) CCGPU_HIP(hipMemGetInfo(&fr, &tot));
-    if (!dryrun() && (double)fr < need) {
-      diisS_.release();
-      diisE_.release();
+// a-strips of the sums of the adjoint ladder.  K is the long side there and only
+// the FP64 GEMM splits it: the others keep one wave of output tiles a strip
+// (512).  FP32, one left transformation at o=7 v=171 / o=24 v=192 / o=32 v=256:
+// with 64 tiles a strip 56.3 / 100.4 / 384 ms, 512 40.1 / 85.4 / 302, no strips
+// 43.8 / 92.3 / 306.
+std::vector<int> CCSD::adjoint_strips(int a0, int a1, GemmPrec prec) const {
+  return ladder_strips(a0, a1, dm_.naux, prec == GemmPrec::F64 ? 64 : 512);
+}
+
+// Scratch of the bulk products of the forward pass and of transformations in
+// its arithmetic and in the given one.
+ScratchNeed CCSD::lhtr_scratch(GemmPrec transforms) const {
+  ScratchNeed n;
+  lhtr_scratch(n, bulk_);
+  if (transforms != bulk_) lhtr_scratch(n, transforms);
+  return n;
+}
+
+void CCSD::lhtr_scratch(ScratchNeed& n, GemmPrec prec) const {
+  const long v = dm_.v, naux = dm_.naux, nov = dm_.nov, npo = dm_.npo, npv = dm_.npv;
+  const long oo = (long)dm_.o * dm_.o, vv = v * v;
+  auto add = [&](long M, long N, long K, double beta, int batch = 1) { gemm_scratch(n, M, N, K, batch, beta, prec); };
+  add(nov, nov, naux, 1.0);
+  add(nov, nov, nov, 0.0);
+  add(nov, nov, nov, 1.0);
+  add(naux, nov, nov, 0.0);
+  add(naux, nov, nov, 1.0);
+  add(naux, vv, oo, 1.0);
+  add(naux, oo, vv, 1.0);
+  add(oo, oo, vv, 0.0);
+  add(oo, oo, vv, 1.0);
+  add(oo, vv, oo, 0.0);
+  add(oo, vv, oo, 1.0);
+  add(vv, oo, naux, 0.0);
+  for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
+    const int a0 = lad_batches_[bi], a1 = lad_batches_[bi + 1];
+    long rows = 0;
+    for (int a = a0; a < a1; ++a) rows += v - a;
+    const long M = (a1 - a0) * v, Nn = (v - a0) * v;
+    add(npo, npv, rows, 1.0, 2);
+    add(rows, npv, npo, 0.0, 2);
+    if (prec != GemmPrec::BF16X3) {  // whose Y and S products read operands packed for the ladder
+      add(rows, npo, npv, 0.0, 2);
+      const std::vector<int> s = ladder_strips(a0, a1, Nn, 1024);
+      for (size_t q = 0; q + 1 < s.size(); ++q) add((s[q + 1] - s[q]) * v, (v - s[q]) * v, naux, 0.0);
     }
+    const std::vector<int> s = adjoint_strips(a0, a1, prec);
+    for (size_t q = 0; q + 1 < s.size(); ++q) {
+      const long w = (s[q + 1] - s[q]) * v;
+      add(naux, w, Nn - (s[q] - a0) * v / 64 * 64, 1.0);
+      add(naux, w, std::min(M, ((s[q + 1] - a0) * v + 63) / 64 * 64), 1.0);
+    }
+    add(naux, Nn - M, M, 1.0);
   }
+}
+
+// Bytes that the forward pass and the transformations still have to allocate.
+double CCSD::lhtr_need(GemmPrec transforms) const {
+  const double o = dm_.o, v = dm_.v, naux = dm_.naux, N = dm_.N, nov = dm_.nov, oo = o * o;
+  auto more = [](double want, double have) { return std::max(0.0, want - have); };
+  double b = 0.0;
+  if (!Tb_.p)
+    b += 8.0 * (4.0 * dm_.nov2 + naux * (N * N + v * v + oo + 2.0 * nov + 1.0) + oo * nov + N * N + v * v + oo +
+                2.0 * oo * oo + 2.0 * dm_.npo * dm_.npv + 2.0 * nov);
+  if (!lst_.p) b += 8.0 * 4.0 * dm_.ntamp;
+  if (transforms == GemmPrec::BF16X3 || bulk_ == GemmPrec::BF16X3)
+    b += 4.0 * more(ladder_b_size(), lpBh_.n);
+  if (bulk_ == GemmPrec::BF16X3) {
+    const double KpT = bf16x3_kpad(dm_.npv), maxr = ladder_maxrows();
+    b += 4.0 * more(2.0 * bf16x3_rpad(dm_.npo) * KpT, lpTh_.n) + 4.0 * more(2.0 * bf16x3_rpad(maxr) * KpT, lpVh_.n) +
+         8.0 * more(2.0 * maxr * dm_.npo, S2_.n);
+  }
+  return b + (double)scratch_growth(lhtr_scratch(transforms), st_);
+}
+
+// Forward pass at the current amplitudes in the bulk arithmetic: leaves Bt, Bvv,
+// Boo, BvoT, F, h~, Jd, Tx, U, C, D, Gam, E1, E2, Z, W, F_kc and tau+/- on the
+// device.  The DIIS history stays when what the forward pass, transformations in
+// the given arithmetic and the caller (extra bytes) still allocate fits beside
+// it, with 1 GB to spare, for partial sums of small products among others;
+// otherwise it is released, as the converged ground state needs none (a later
+// iterate restarts the DIIS cycle).
+void CCSD::lhtr_prepare(GemmPrec transforms, double extra) {
+  ensure_work();
+  // room made once stays (until the workspace is released)
+  const unsigned room = 1u << (3 * static_cast<int>(bulk_) + static_cast<int>(transforms));
+  if (diisS_.p && (extra > 0.0 || !lst_.p || !(lhtr_room_ & room)) &&
+      (double)device_free() < lhtr_need(transforms) + extra + 1.0e9) {
+    diisS_.release();
+    diisE_.release();
+  }
+  lhtr_room_ |= room;
+  if (lhtr_ready_ && lhtr_prec_ == bulk_) return;
   residual(t1_.p, T_.p, om1_.p, Om_.p);
   ensure_lhtr();
   lhtr_ready_ = true;
@@ -99,7 +171,7 @@ void CCSD::lhtr_ladder(const double* Xb) {
     ladder_gather(S_.p, S_.p + ns, Xb, a0, a1, o, v, st_);
     bulk(npo, npv, rows, 0.5, S_.p, 1, npo, V_.p, npv, 1, 1.0, taub_.p, npv, 1, 2, ns, nv, nt);
     bulk(rows, npv, npo, 0.5, S_.p, npo, 1, tau_.p, npv, 1, 0.0, V_.p, npv, 1, 2, ns, nt, nv);
-    const std::vector<int> sa = ladder_strips(a0, a1, naux, bulk_ == GemmPrec::F64 ? 64 : 512);
+    const std::vector<int> sa = adjoint_strips(a0, a1, bulk_);
     // Entries with b < a: zeros where the sums below read them, the blocks of
     // a strip by itself and of its K padding (v = 192: 1.8 ms of all of Y).
     for (size_t q = 0; q + 1 < sa.size(); ++q) {
@@ -110,11 +182,7 @@ void CCSD::lhtr_ladder(const double* Xb) {
     // Y_bar is zero for b < a: the strip [s0, s1) of a sums over b >= s0, that
     // of b over a < s1.  Both sums start and end at multiples of 64, the K
     // padding of the packed operands, so they add the same terms in the same
-    // groups as the whole sums do.  K is the long side here and only the FP64
-    // GEMM splits it: the others keep one wave of output tiles a strip (512).
-    // FP32, one left transformation at o=7 v=171 / o=24 v=192 / o=32 v=256: with
-    // 64 tiles a strip 56.3 / 100.4 / 384 ms, 512 40.1 / 85.4 / 302, no strips
-    // 43.8 / 92.3 / 306.
+    // groups as the whole sums do.
     double* Bbb = Bvvb_.p + (long)a0 * v;
     for (size_t q = 0; q + 1 < sa.size(); ++q) {
       const long r0 = (long)(sa[q] - a0) * v, nr = (long)(sa[q + 1] - sa[q]) * v, k0 = r0 / 64 * 64;
@@ -257,7 +325,7 @@ void CCSD::lhtr_host(int nvec, const double* l1, const double* l2p, double* rho1
   CCGPU_REQUIRE(iter_ >= 1, "ccgpu_lhtr: no amplitudes (run the CCSD iterations or set amplitudes first)");
   if (nvec == 0) return;
   const long nov = dm_.nov, np2 = dm_.ntamp - nov;
-  lhtr_prepare();
+  lhtr_prepare(bulk_);
   if (!lst_.p) lst_.alloc(4 * (size_t)(np2 + nov));  // [in 0, in 1, out 0, out 1] x (l1/rho1, l2/rho2)
   side_stream();
   const long slot = np2 + nov;

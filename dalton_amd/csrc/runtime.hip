@@ -1,4 +1,5 @@
 // Allocation registry and dry-run support (see common.h).
+#include <cstdlib>
 #include <map>
 #include <mutex>
 
@@ -19,7 +20,25 @@ std::map<uintptr_t, size_t>& allocs() {
   return *m;
 }
 uintptr_t g_next = uintptr_t(1) << 44;  // fake device addresses for dry runs
+size_t g_live = 0;                      // bytes registered
+
+// Device memory of a dry run: CCGPU_DRYRUN_MB, without limit if unset.
+size_t dry_capacity() {
+  const char* e = std::getenv("CCGPU_DRYRUN_MB");
+  return e && std::atof(e) > 0.0 ? (size_t)(std::atof(e) * 1.0e6) : ~size_t(0) / 2;
+}
 }  // namespace
+
+size_t device_free() {
+  size_t fr = 0, tot = 0;
+  if (!dryrun()) {
+    CCGPU_HIP(hipMemGetInfo(&fr, &tot));
+    return fr;
+  }
+  std::lock_guard<std::mutex> lk(g_mu);
+  const size_t cap = dry_capacity();
+  return cap > g_live ? cap - g_live : 0;
+}
 
 bool capturing(hipStream_t s) {
   if (dryrun()) return false;
@@ -54,6 +73,20 @@ void release_scratch(hipStream_t s) {
   delete p;
 }
 
+size_t scratch_growth(const ScratchNeed& n, hipStream_t s) {
+  const StreamScratch& sc = scratch_for(s);
+  auto more = [](size_t want, size_t have, size_t size) { return want > have ? want * size - have * size : 0; };
+  size_t b = more(n.splitk, sc.splitk.n, sizeof(double));
+  for (int q = 0; q < 4; ++q) b += more(n.pack[q], sc.pack[q].n, sizeof(unsigned short));
+  return b;
+}
+
+void reserve_scratch(const ScratchNeed& n, hipStream_t s) {
+  StreamScratch& sc = scratch_for(s);
+  grow_scratch(sc.splitk, n.splitk, s);
+  for (int q = 0; q < 4; ++q) grow_scratch(sc.pack[q], n.pack[q], s);
+}
+
 bool& dryrun() {
   static bool flag = false;
   return flag;
@@ -61,6 +94,7 @@ bool& dryrun() {
 
 void* dry_alloc(size_t bytes) {
   std::lock_guard<std::mutex> lk(g_mu);
+  if (g_live + bytes > dry_capacity()) throw Error(2, "dry run: out of device memory");
   const uintptr_t p = g_next;
   g_next += (bytes + (1u << 20)) & ~uintptr_t((1u << 20) - 1);
   return reinterpret_cast<void*>(p);
@@ -69,11 +103,15 @@ void* dry_alloc(size_t bytes) {
 void register_alloc(const void* p, size_t bytes) {
   std::lock_guard<std::mutex> lk(g_mu);
   allocs()[reinterpret_cast<uintptr_t>(p)] = bytes;
+  g_live += bytes;
 }
 
 void unregister_alloc(const void* p) {
   std::lock_guard<std::mutex> lk(g_mu);
-  allocs().erase(reinterpret_cast<uintptr_t>(p));
+  auto it = allocs().find(reinterpret_cast<uintptr_t>(p));
+  if (it == allocs().end()) return;
+  g_live -= it->second;
+  allocs().erase(it);
 }
 
 namespace {

@@ -192,7 +192,8 @@ int ccgpu_eta(ccgpu_ctx* ctx, double* eta1, double* eta2);
  * equations, at most 2x smaller than that of lambda A + eta) is below thr
  * (Dalton's THRLEQ); at most maxit
  * transformations, maxred trial vectors (capped at 64 and by free device
- * memory; a full space collapses onto the current solution).  precision 1
+ * memory, for which the DIIS history is released if need be; a full space
+ * collapses onto the current solution).  precision 1
  * (BF16x3 bulk) runs an iterative refinement: the FP64 residual of lambda is
  * formed once per step and the correction solved with BF16x3 transformations,
  * so the result meets thr in FP64 arithmetic; niter counts both kinds.
