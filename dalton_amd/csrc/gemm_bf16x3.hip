@@ -650,8 +650,9 @@ void ladder_vpm_pack(unsigned short* hi, unsigned short* lo, const float* Y, lon
   check_span(Y, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(float), "ladder_vpm_pack Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm_pack: ldY too small");
   CCGPU_REQUIRE(v < 32 * 65536, "ladder_vpm_pack: virtual space too large");
-  const dim3 grid(cdiv(v, 128) * cdiv(v, 32) * cdiv(rows, 8) * 8);
-  CCGPU_REQUIRE((double)cdiv(v, 128) * cdiv(v, 32) * rows < 16.0e6, "ladder_vpm_pack: grid too large");
+  const long nblk = (long)cdiv(v, 128) * cdiv(v, 32) * cdiv(rows, 8) * 8;
+  CCGPU_REQUIRE(nblk < (1L << 24), "ladder_vpm_pack: grid too large");
+  const dim3 grid((unsigned)nblk);
   if (v % 4 == 0 && ldY % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0)
     CCGPU_LAUNCH(k_ladder_vpm_pack<true>, grid, dim3(256), 0, st, hi, lo, Y, ldY, a0, v, rows, Rp, Kp);
   else

@@ -547,10 +547,9 @@ void ladder_vpm(double* vp, double* vm, const double* Y, long ldY, int a0, int a
   check_span(Y, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(double), "ladder_vpm Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm: ldY too small");
   CCGPU_REQUIRE(v < 32 * 65536, "ladder_vpm: virtual space too large");
-  const double nblk = (double)cdiv(v, 64) * cdiv(v, 32) * rows;
-  CCGPU_REQUIRE(nblk < 16.0e6, "ladder_vpm: grid too large");
-  CCGPU_LAUNCH(k_ladder_vpm, dim3(cdiv(v, 64) * cdiv(v, 32) * cdiv(rows, 8) * 8), dim3(256), 0, st, vp, vm, Y, ldY, a0,
-               v, rows);
+  const long nblk = (long)cdiv(v, 64) * cdiv(v, 32) * cdiv(rows, 8) * 8;
+  CCGPU_REQUIRE(nblk < (1L << 24), "ladder_vpm: grid too large");
+  CCGPU_LAUNCH(k_ladder_vpm, dim3((unsigned)nblk), dim3(256), 0, st, vp, vm, Y, ldY, a0, v, rows);
   CCGPU_HIPX(hipGetLastError());
 }
 
@@ -856,9 +855,9 @@ void ladder_vpm_adj(double* Yb, long ldY, const double* vpb, const double* vmb, 
   check_span(Yb, 0, ((long)(a1 - a0) * v - 1) * ldY + (long)(v - a0) * v - 1, sizeof(double), "ladder_vpm_adj Y");
   CCGPU_REQUIRE(ldY >= (long)(v - a0) * v, "ladder_vpm_adj: ldY too small");
   const long nt = (v + 31) / 32;
-  CCGPU_REQUIRE(nt * (nt + 1) / 2 * rows < (1L << 26), "ladder_vpm_adj: grid too large");
-  CCGPU_LAUNCH(k_ladder_vpm_adj, dim3((unsigned)(nt * (nt + 1) / 2 * cdiv(rows, 8) * 8)), dim3(32, 8), 0, st, Yb, ldY, vpb,
-               vmb, a0, v, rows);
+  const long nblk = nt * (nt + 1) / 2 * cdiv(rows, 8) * 8;
+  CCGPU_REQUIRE(nblk < (1L << 24), "ladder_vpm_adj: grid too large");
+  CCGPU_LAUNCH(k_ladder_vpm_adj, dim3((unsigned)nblk), dim3(32, 8), 0, st, Yb, ldY, vpb, vmb, a0, v, rows);
   CCGPU_HIPX(hipGetLastError());
 }
 
