@@ -221,7 +221,7 @@ class CCSD {
   DBuf<unsigned short> lpBh_, lpBl_, lpTh_, lpTl_, lpVh_, lpVl_;
   DBuf<double> S2_;
   // DIIS
-  DBuf<double> diisS_, diisE_, dvec_, dots_, coef_, Amat_, diiswork_;
+  DBuf<double> diisS_, diisE_, dots_, coef_, Amat_, diiswork_;
   DBuf<int> ctr_;  // [0] iteration of the DIIS cycle, [1] singular-matrix flag
   DBuf<double> scal_;  // [0] squared residual norm, [1] energy
   double ladder_budget_ = 10.0e9;

@@ -203,8 +203,8 @@ void CCSD::release_work() {
   diis_off_ = iter_ > 0 ? iter_ - 1 : 0;  // the DIIS history is gone: restart the cycle
 }
 
-// Second stream (default priority) with two pairs of events, made once:
-// staging copies of the left transformation, (T) energies beside the W passes.
+// Second stream (default priority) with two pairs of events, made once: the
+// staging copies of the left transformation.
 void CCSD::side_stream() {
   if (cst_ || dryrun()) return;
   CCGPU_HIP(hipStreamCreateWithFlags(&cst_, hipStreamNonBlocking));
@@ -280,8 +280,7 @@ void CCSD::ladder(const double* T, double* Om) {
     ladder_mixed(Om);
     return;
   }
-  const int o = dm_.o, v = dm_.v, naux = dm_.naux;
-  const long vv = (long)v * v;
+  const int o = dm_.o, v = dm_.v;
   const Gemm bulk{bulk_, st_};
   for (size_t bi = 0; bi + 1 < lad_batches_.size(); ++bi) {
     const int a0 = lad_batches_[bi], a1 = lad_batches_[bi + 1];

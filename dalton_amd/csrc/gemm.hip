@@ -1,7 +1,7 @@
 // Strided / batched / split-K GEMM on CDNA4 matrix cores (gfx950).
 //
-// FP64: v_mfma_f64_16x16x4f64.  Block tile 128x128, 64x64 or 32x32 (K step
-// 16, 32 or 64), 256 threads as 2x2 waves.  Operands are staged global ->
+// FP64: v_mfma_f64_16x16x4f64.  Block tile 128x128, 64x64 (K step 16) or 32x32
+// (K step 32), 256 threads as 2x2 waves.  Operands are staged global ->
 // registers -> LDS (padded so a wave's 16x4 fragment reads hit all 64 banks
 // once per half-wave); the next K step's global loads are issued before the
 // MFMAs of the current one.  No load is bounds-checked but those of a last,
@@ -49,7 +49,7 @@ __device__ __forceinline__ void tile_of(long b, long tiles_m, long tiles_n, long
 // (T/32)x(T/32) MFMA 16x16 tiles.  The next step's global loads are in
 // flight while the current step's MFMAs run; one LDS stage, two barriers a
 // step: a second stage saves a barrier but costs the blocks that hide it
-// (128 tile 61 against 68 TFLOP/s; 64 tile, two blocks a CU instead of four,
+// (128 tile 61 against 68 TFLOP/s; 64 tile, two blocks a CU instead of four to six,
 // 1150^3 to 3570^3 products 1.2-1.3x the time).
 template <int AMODE, int BMODE, bool K2, int T>
 __global__ __launch_bounds__(256, T == 128 ? 2 : (T == 64 ? 4 : 5)) void k_dgemm(GemmDesc d, long kchunk, int nz,
@@ -273,7 +273,8 @@ constexpr long kMaxTiles = 1L << 24;
 int step_k(int T) { return T == 32 ? Step<32>::TK : Step<64>::TK; }
 
 // Estimated time (microseconds) of block tile T with K in nz chunks.  kRes
-// blocks of the tile are resident per CU (256 CUs); with c of them a K step
+// blocks of the tile count as resident per CU (256 CUs; by registers 2, 4 to 6
+// and 5 to 8, as the operand orders go); with c of them a K step
 // takes kBase + kPer c cycles, and the blocks beyond whole rounds of 256 kRes
 // take a round of their own.  A two-level K costs kTwoK, a split adds a launch
 // and the pass over the partials, and C bounds the time from below (the

@@ -21,18 +21,10 @@
 
 namespace ccgpu {
 
-
 namespace {
 
-__device__ __forceinline__ unsigned short f2bf(float f) {
-  unsigned int u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);  // round to nearest even
-  return static_cast<unsigned short>(u >> 16);
-}
-__device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float(static_cast<unsigned int>(h) << 16); }
-
 // Two elements split together: packed hi and lo pairs (the conversion
-// instruction rounds to nearest even like f2bf).
+// instruction rounds to nearest even).
 __device__ __forceinline__ unsigned pk_bf16(float a, float b) {
   typedef float f2v __attribute__((ext_vector_type(2)));
   typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
@@ -283,7 +275,8 @@ struct NoTune {
   ~NoTune() { --t_no_tune; }
 };
 
-// Products of fewer 128x128 tiles than this (two per CU) may take the 64x64 one.
+// Products of fewer 128x128 tiles than this (four per CU, two rounds of blocks)
+// may take the 64x64 one.
 constexpr long kSmallTiles = 1024;
 long tiles128(const BMulti& p, int batch) { return (long)cdiv(p.M, TM) * cdiv(p.N, TN) * batch; }
 
