@@ -9,10 +9,10 @@
 // by output orientation (pt_persistent.hip), reading the integrals (yd|zr)
 // in two layouts, G[r][d][y][z] and Gp[r][d][z][y] (packed bf16 hi/lo
 // transposes of both in the mixed path), t2 re-laid as Tvvo[p][x][y][l] =
-// t_pl^{xy} and (zr|lq) as Q[r][q][l][z], all built once from the DF factor
-// and the amplitudes.  The energy evaluates the permutation-symmetrised
-// functional of w_prod (:1547-1640) per orbit {a,b,c}: E4 takes V = W, E5
-// the t1 part of V (v_calc :1345, :1483-1527).
+// t_pl^{xy} and (zr|lq) as Q[r][q][l][z]: the integrals built once from the DF
+// factor, those of t2 again whenever the amplitudes were written.  The energy
+// evaluates the permutation-symmetrised functional of w_prod (:1547-1640) per
+// orbit {a,b,c}: E4 takes V = W, E5 the t1 part of V (v_calc :1345, :1483-1527).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
